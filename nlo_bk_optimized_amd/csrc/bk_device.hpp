@@ -681,11 +681,12 @@ __device__ __forceinline__ NloStable<T> nlo_integrand_stable(T r, T log_r, T lz,
 
 // ------------------------------------------- FP32 path: fast primitives
 //
-// The FP32 integrand works in base-2 logarithms: the VEGAS map hands it
-// t = log2 z (its bin table is scaled by log2 e), so z = 2^t and every
-// logarithm of a distance comes from the hardware log2 with no conversion;
-// the spline coordinate, the kernel's L and the coupling take their constants
-// in the same units.
+// The FP32 integrand works in units of the parent size r and in base-2
+// logarithms: the VEGAS map hands it t = log2(z / r) (its bin table holds the
+// logarithms relative to log2 r, formed in FP64), so every logarithm of a
+// distance comes from the hardware log2 with no conversion, and near z = r,
+// where the largest samples sit, t is small and carries its full relative
+// precision (log2 z of a small distance would round z by up to 1e-6).
 
 constexpr float kLn2f = 0.693147182f;
 constexpr float kLog2ef = 1.44269502f;
@@ -698,19 +699,40 @@ __device__ __forceinline__ float frcp(float x) { return __builtin_amdgcn_rcpf(x)
 
 __device__ __forceinline__ float frsq(float x) { return __builtin_amdgcn_rsqf(x); }
 
-// |sin y| for y in [-pi, pi] (the integrand needs only squares of sines):
-// fold to v = min(|y|, pi - |y|), with pi - |y| computed exactly for
-// |y| >= pi/2 (Sterbenz) plus the low part of pi, then the Taylor polynomial
-// to v^11 (relative error < 6e-8, accurate for small v).
-__device__ __forceinline__ float fsin_abs(float y) {
-    const float ay = fabsf(y);
-    const float v = fminf(ay, (3.14159274f - ay) + -8.74227766e-8f);
-    const float v2 = v * v;
-    float p = fmaf(v2, -2.50521084e-8f, 2.75573192e-6f);
-    p = fmaf(v2, p, -1.98412698e-4f);
-    p = fmaf(v2, p, 8.33333333e-3f);
-    p = fmaf(v2, p, -1.66666667e-1f);
-    return fmaf(v2 * v, p, v);
+// Least and largest values, none of them a signalling NaN: the library forms
+// canonicalise every operand that reaches a loop from outside by a v_max.
+__device__ __forceinline__ float fmin3(float a, float b, float c) {
+    float o;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(o) : "v"(a), "v"(b), "v"(c));
+    return o;
+}
+__device__ __forceinline__ float fmax3(float a, float b, float c) {
+    float o;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(o) : "v"(a), "v"(b), "v"(c));
+    return o;
+}
+__device__ __forceinline__ float fmax2(float a, float b) {
+    float o;
+    asm("v_max_f32 %0, %1, %2" : "=v"(o) : "v"(a), "v"(b));
+    return o;
+}
+// Keeps what follows inside its branch (the compiler would run it always and
+// select, which costs every wave).
+__device__ __forceinline__ void keep_branch(float& v) { asm volatile("" : "+v"(v)); }
+
+// 4 sin^2 y for |y| <= pi.  With w = |y| (pi - |y|), |sin y| = cos((pi^2/4 -
+// w)^1/2) is entire in w, and 2 |sin y| / w is its degree-4 interpolant at
+// Chebyshev nodes of [0, pi^2/4] (relative error 1e-9; all terms positive), so
+// that no fold into [0, pi/2] is needed.  pi - |y| is exact near pi, with the
+// low part of pi added.  pi: 3.14159274f in a vector register.
+__device__ __forceinline__ float f4sin2(float y, float pi) {
+    const float w = fabsf(y) * ((pi - fabsf(y)) + -8.74227766e-8f);
+    float p = fmaf(w, 5.161262147e-07f, 4.312110734e-05f);
+    p = fmaf(w, p, 2.320589108e-03f);
+    p = fmaf(w, p, 6.450305465e-02f);
+    p = fmaf(w, p, 6.366197731e-01f);
+    const float s = w * p;
+    return s * s;
 }
 
 // log2(1 + u) / 2 for |u| < 0.5: atanh(s) log2(e) with s = u / (2 + u),
@@ -725,22 +747,49 @@ __device__ __forceinline__ float fhalf_log2_1p_small(float u) {
     return s * p;
 }
 
-// h(L) = 2L / (e^{2L} - 1) and h(-L) = h(L) e^{2L} for x = 2L given also in
-// base 2 (x2 = 2L log2 e, so e^{2L} = 2^x2 with no rounding of the argument):
-// Bernoulli series 1 - x/2 + x^2/12 - x^4/720 + x^6/30240 for |x| < 0.25,
-// else from e^{2L} (no cancellation there; the second form avoids 1 - e^x
-// for x << 0).  x2 is clamped at 124 (e^86).
-__device__ __forceinline__ void fh_pair(float x, float x2, float& h, float& hm) {
+// 2^t - 1 for |t ln 2| < 1/4: sum_k (ln 2)^k t^k / k!, k = 1..6 (relative error
+// < 2e-8).
+__device__ __forceinline__ float fexp2m1_small(float t) {
+    float p = fmaf(t, 1.54035304e-4f, 1.33335581e-3f);  // (ln 2)^6 / 720, (ln 2)^5 / 120
+    p = fmaf(t, p, 9.61812911e-3f);                     // (ln 2)^4 / 24
+    p = fmaf(t, p, 5.55041087e-2f);                     // (ln 2)^3 / 6
+    p = fmaf(t, p, 2.40226507e-1f);                     // (ln 2)^2 / 2
+    p = fmaf(t, p, 6.93147181e-1f);                     // ln 2
+    return t * p;
+}
+
+// h(L) = 2L / (e^{2L} - 1), h(-L) = h(L) e^{2L} and g(L) = L coth L - 1 =
+// h(|L|) + |L| - 1 for x = 2L given also in base 2 (x2 = 2L log2 e, so e^{2L} =
+// 2^x2 with no rounding of the argument).  |x| < 0.25: the Bernoulli series g =
+// x^2/12 - x^4/720 + x^6/30240, h = g + 1 - x/2; else h from e^{2L} (no
+// cancellation there; the second form avoids 1 - e^x for x << 0; x2 is
+// clamped at 124, e^86), and g by its seven-term series in y = L^2 for |L| < 1
+// (sum_n 2^2n B_2n L^2n / (2n)!, whose terms fall by ~1/pi^2).
+__device__ __forceinline__ void fhg(float x, float x2, float& h, float& hm, float& g) {
     if (fabsf(x) < 0.25f) {
         const float xx = x * x;
         float p = fmaf(xx, 1.0f / 30240.0f, -1.0f / 720.0f);
         p = fmaf(xx, p, 1.0f / 12.0f);
-        h = fmaf(xx, p, fmaf(x, -0.5f, 1.0f));
+        g = xx * p;
+        h = g + fmaf(x, -0.5f, 1.0f);
         hm = h + x;
     } else {
         const float E = fexp2(fminf(x2, 124.0f));
         h = x * frcp(E - 1.0f);
         hm = h * E;
+        const float aL = fabsf(0.5f * x);
+        if (aL < 1.0f) {
+            const float y = aL * aL;
+            float p = fmaf(y, 2.19259479e-7f, -2.16440428e-6f);
+            p = fmaf(y, p, 2.13777992e-5f);
+            p = fmaf(y, p, -2.11640212e-4f);
+            p = fmaf(y, p, 2.11640212e-3f);
+            p = fmaf(y, p, -2.22222222e-2f);
+            p = fmaf(y, p, 3.33333333e-1f);
+            g = y * p;
+        } else {
+            g = aL + (x >= 0.0f ? h : hm) - 1.0f;
+        }
     }
 }
 
@@ -748,21 +797,26 @@ __device__ __forceinline__ void fh_pair(float x, float x2, float& h, float& hm) 
 // t = (ln d - ln r_0) / h - k in [0, 1), coefficients pre-multiplied by
 // log2(e) so that N = 2^(a + t (b + t (c + t d))): one 16-byte LDS read.
 struct FastSpline {
-    // rec[0] and rec[R] are constant records for ln d below ln r_0 (N = 2^-126,
-    // i.e. 0 to FP32 precision, S = 1) and above ln r_{R-1} (N = 1, S = 0);
-    // rec[k], k = 1..R-1, is interval k - 1.  u = log2 d * inv_h2 + off is the
-    // position in records: inv_h2 = ln 2 / h, off = 1 - ln r_0 / h.
+    // The records run from rec[vmin], a constant one for ln d below ln r_0
+    // (N = 2^-126, i.e. 0 to FP32 precision, S = 1), over the R - 1 intervals to
+    // rec[vmax], constant above ln r_{R-1} (N = 1, S = 0); rec[0] starts at the
+    // record boundary nearest to r.  v = log2(d / r) * inv_h2 + off is the
+    // position: inv_h2 = ln 2 / h, off = the distance of r from that boundary
+    // (0 on the evolution's grid, whose node r is).  Counted from r, a position
+    // near r rounds to its own small size; counted from r_0 it would round by
+    // up to 3e-5 of a record, which is 1e-6 of N.
     const float4* rec;
-    float inv_h2, off, umax;  // umax = R
+    float inv_h2, off, vmin, vmax;
 };
 
-// u clamped to [0, umax] by one median-of-three (log2_d is finite: it is the
-// log of a distance); for u >= 0 the fraction u - floor(u) is exact and
-// (int)u = floor(u), so t and the record index need no floor.
+// v clamped to the table by one median-of-three (log2_d is finite: it is the
+// log of a distance); v - floor(v) is exact.
 __device__ __forceinline__ float fspline_log2n(const FastSpline& s, float log2_d) {
-    const float u = __builtin_amdgcn_fmed3f(fmaf(log2_d, s.inv_h2, s.off), 0.0f, s.umax);
-    const float t = __builtin_amdgcn_fractf(u);
-    const float4 c = s.rec[(int)u];
+    const float v = __builtin_amdgcn_fmed3f(fmaf(log2_d, s.inv_h2, s.off), s.vmin, s.vmax);
+    const float t = __builtin_amdgcn_fractf(v);
+    int k;
+    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(k) : "v"(v));
+    const float4 c = s.rec[k];
     return fmaf(t, fmaf(t, fmaf(t, c.w, c.z), c.y), c.x);
 }
 
@@ -770,120 +824,151 @@ __device__ __forceinline__ float fspline_n(const FastSpline& s, float log2_d) {
     return fexp2(fspline_log2n(s, log2_d));
 }
 
-// N and S = 1 - N.  Near N = 1 the subtraction would keep only the absolute
-// precision of N, so S = -expm1(p ln 2) comes from the exponent p = log2 N
-// by its series when |p ln 2| < 1/4 (relative error < 2e-8), written in p:
-// expm1(p ln 2) = sum_k (ln 2)^k p^k / k!.
-__device__ __forceinline__ void fspline_ns(const FastSpline& s, float log2_d, float& n, float& sv) {
-    const float p = fspline_log2n(s, log2_d);
-    n = fexp2(p);
-    float e = fmaf(p, 1.54035304e-4f, 1.33335581e-3f);  // (ln 2)^6 / 720, (ln 2)^5 / 120
-    e = fmaf(p, e, 9.61812911e-3f);                     // (ln 2)^4 / 24
-    e = fmaf(p, e, 5.55041087e-2f);                     // (ln 2)^3 / 6
-    e = fmaf(p, e, 2.40226507e-1f);                     // (ln 2)^2 / 2
-    e = fmaf(p, e, 6.93147181e-1f);                     // ln 2
-    sv = fabsf(p) < 0.360673760f ? -(p * e) : 1.0f - n;  // |p ln 2| < 1/4
+// S = 1 - N = -(2^p - 1) from p = log2 N near N = 1, where the subtraction
+// would keep only the absolute precision of N: the series for |p ln 2| < 1/4
+// (relative error < 2e-8).
+constexpr float kNearOne = -0.360673760f;  // p above it: |p ln 2| < 1/4
+
+__device__ __forceinline__ float fs_near_one(float p) {
+    return -fexp2m1_small(p);
 }
 
+// Launch-invariant constants of the FP32 integrand, formed once per lane in
+// vector registers: an FP32 operation with a scalar-register operand issues at
+// half the rate of one with vector or literal operands.
+struct Fp32Consts {
+    float pi;
+    float log2_r;
+    float cut;         // 1e10 r^4
+    float norm;        // Nc^2 / (8 pi^4), halved when symmetrised, times the caller's scale of the weights
+    float mirror;      // 1 when symmetrised (the mirrored sample counts too), else 0
+    float nf_over_nc;
+    float mu;          // ln mu0 log2 e
+    float right0;      // 5 (ln 4 C2 / Lambda^2) log2 e - 10 log2 r
+    float b0;          // b0 0.2 ln 2
+};
+
 // The FP32 K2 + Kf integrand: the cancellation-free formula of
-// nlo_integrand_stable, every transcendental on the fast primitives above,
-// cos(theta) = 1 - 2 sin^2(theta / 2), logs of distances (base 2) from the
-// log1p forms, N from the local-coordinate spline.  t1 = log2 z and
-// t2 = log2 z', log2_r = log2 r.
-template <bool ANYC>
-__device__ __forceinline__ NloStable<float> nlo_integrand_fp32(
-    float r, float log2_r, float t1, float t2, float tz, float tz2, const FastSpline& sp,
-    const NloCoupling<float>& cpl, float nf_over_nc, float nc, float norm, bool symmetrize) {
+// nlo_integrand_stable with every distance in units of r, the transcendentals
+// on the fast primitives above, logs of distances (base 2) from the log1p
+// forms, N from the local-coordinate spline.  t1 = log2(z / r), t2 = log2(z' /
+// r), y1 = theta / 2, y2 = theta' / 2 (modulo pi, in [-pi/2, pi/2] but for the
+// bin across pi/2).
+//
+// Issue-bound: the cost of a sample is its instructions, an FP32 add, mul or fma
+// on vector registers or literals counting 2 cycles, min / max / compare /
+// select / convert 4, a transcendental 8.  Hence the forms below: 4 sin^2 in
+// one polynomial without a fold; the kernels from squared reciprocals (rcp
+// for rsq and its squares); dipoles as n_z S_y' + (n_y' - n_y); and the rare
+// cases (N near 1, the coupling near its freezing scale, the K2 cut, a
+// non-finite value) behind tests that a whole wave takes or skips, which pays
+// because the lanes of a wave hold neighbouring samples (sobol_order.hpp).
+// 2^20 samples of 228 parents: 1.51 -> 1.17 ms (about 770 cycles a sample and
+// wave; the listing counts 345 instructions before), and 2 to 5 times closer
+// to the FP64 evaluation in most parents.
+// SPLIT: the K2 and Kf parts are wanted apart.
+template <bool ANYC, bool SPLIT>
+__device__ __forceinline__ NloStable<float> nlo_integrand_fp32(const Fp32Consts& c, float t1, float t2, float y1,
+                                                               float y2, const FastSpline& sp,
+                                                               const NloCoupling<float>& cpl) {
     NloStable<float> out{0.0f, 0.0f, 0.0f};
     const float z = fexp2(t1), z2 = fexp2(t2);
-    const float s1 = fsin_abs(0.5f * tz), s2 = fsin_abs(0.5f * tz2);
-    const float s3 = fsin_abs(0.5f * (tz - tz2));
-    const float xsq = fmaf(4.0f * r * z, s1 * s1, (r - z) * (r - z));
-    const float x2sq = fmaf(4.0f * r * z2, s2 * s2, (r - z2) * (r - z2));
-    const float zsq = fmaf(4.0f * z * z2, s3 * s3, (z - z2) * (z - z2));
-    if (!(xsq >= 1e-37f) || !(x2sq >= 1e-37f) || !(zsq >= 1e-37f)) return out;
-    // the distances enter only as reciprocals: 1 / X = rsq(X^2)
-    const float iX = frsq(xsq), iX2 = frsq(x2sq), iZ = frsq(zsq);
-    // log2(X / Y): (X^2 - z^2) / z^2 = rho (rho - 2 cos t), cos t = 1 - 2 s^2
-    const float rho1 = r * frcp(z), rho2 = r * frcp(z2);
-    const float u1 = rho1 * (rho1 - 2.0f + 4.0f * s1 * s1);
-    const float u2 = rho2 * (rho2 - 2.0f + 4.0f * s2 * s2);
+    const float s1 = f4sin2(y1, c.pi), s2 = f4sin2(y2, c.pi), s3 = f4sin2(y1 - y2, c.pi);  // 4 sin^2
+    const float zz2 = z * z2;
+    float z1m = z - 1.0f, z2m = z2 - 1.0f;
+    if (__any(fminf(fabsf(t1), fabsf(t2)) < 0.25f)) {  // 2^t - 1 near t = 0 without cancellation
+        keep_branch(t1);
+        z1m = fabsf(t1) < 0.25f ? fexp2m1_small(t1) : z1m;
+        z2m = fabsf(t2) < 0.25f ? fexp2m1_small(t2) : z2m;
+    }
+    const float xsq = fmaf(z, s1, z1m * z1m);
+    const float x2sq = fmaf(z2, s2, z2m * z2m);
+    const float zsq = fmaf(zz2, s3, (z - z2) * (z - z2));
+    if (!(fmin3(xsq, x2sq, zsq) >= 1e-37f)) return out;
+    // log2(X / Y): (X^2 - z^2) / z^2 = rho (rho - 2 cos t), rho = r / z, cos t = 1 - 2 sin^2(t / 2)
+    const float rho1 = frcp(z), rho2 = frcp(z2);
+    const float u1 = rho1 * ((rho1 - 2.0f) + s1);
+    const float u2 = rho2 * ((rho2 - 2.0f) + s2);
     const float lxy = fabsf(u1) < 0.5f ? fhalf_log2_1p_small(u1) : 0.5f * flog2(xsq) - t1;
     const float lx2y2 = fabsf(u2) < 0.5f ? fhalf_log2_1p_small(u2) : 0.5f * flog2(x2sq) - t2;
     const float log_x = t1 + lxy, log_x2 = t2 + lx2y2, log_zz = 0.5f * flog2(zsq);
-    float n_x, s_x, n_y, s_y, n_x2, s_x2, n_y2, s_y2;
-    fspline_ns(sp, log_x, n_x, s_x);
-    fspline_ns(sp, t1, n_y, s_y);
-    fspline_ns(sp, log_x2, n_x2, s_x2);
-    fspline_ns(sp, t2, n_y2, s_y2);
+    const float p_x = fspline_log2n(sp, log_x), p_y = fspline_log2n(sp, t1);
+    const float p_x2 = fspline_log2n(sp, log_x2), p_y2 = fspline_log2n(sp, t2);
+    const float n_x = fexp2(p_x), n_y = fexp2(p_y), n_x2 = fexp2(p_x2), n_y2 = fexp2(p_y2);
     const float n_z = fspline_n(sp, log_zz);
-    float dip = s_x * (n_z + n_y2 - n_y - n_z * n_y2);
-    float dips = s_x2 * (n_z + n_y - n_y2 - n_z * n_y);
+    float s_x = 1.0f - n_x, s_y = 1.0f - n_y, s_x2 = 1.0f - n_x2, s_y2 = 1.0f - n_y2;
+    float dny = n_y2 - n_y, dnx = n_x - n_x2;
+    float p_max = fmax2(fmax3(p_x, p_y, p_x2), p_y2);
+    if (__any(p_max > kNearOne)) {
+        keep_branch(p_max);
+        s_x = p_x > kNearOne ? fs_near_one(p_x) : s_x;
+        s_y = p_y > kNearOne ? fs_near_one(p_y) : s_y;
+        s_x2 = p_x2 > kNearOne ? fs_near_one(p_x2) : s_x2;
+        s_y2 = p_y2 > kNearOne ? fs_near_one(p_y2) : s_y2;
+        // differences of amplitudes near 1 from the more accurate S
+        if (fminf(p_y, p_y2) > kNearOne) dny = s_y - s_y2;
+        if (fminf(p_x, p_x2) > kNearOne) dnx = s_x2 - s_x;
+    }
+    // S_X (S_Y - S_Z S_Y') and its mirror: S_Y - S_Z S_Y' = N_Z S_Y' + N_Y' - N_Y
+    const float dip = s_x * fmaf(n_z, s_y2, dny);
+    const float dips = s_x2 * fmaf(n_z, s_y, -dny);
 
     // L = ln(X Y' / (X' Y)) from its base-2 form
     const float L2 = lxy - lx2y2;
-    const float L = L2 * kLn2f;
-    float h, hm;
-    fh_pair(2.0f * L, 2.0f * L2, h, hm);
-    const float aL = fabsf(L);
-    float g;
-    if (aL < 1.0f) {
-        // L coth L - 1 = sum_n 2^2n B_2n L^2n / (2n)!: seven terms reach the
-        // rounding of y = L^2 on |L| < 1 (the terms fall by ~1/pi^2)
-        const float y = L * L;
-        float p = fmaf(y, 2.19259479e-7f, -2.16440428e-6f);
-        p = fmaf(y, p, 2.13777992e-5f);
-        p = fmaf(y, p, -2.11640212e-4f);
-        p = fmaf(y, p, 2.11640212e-3f);
-        p = fmaf(y, p, -2.22222222e-2f);
-        p = fmaf(y, p, 3.33333333e-1f);
-        g = y * p;
-    } else {
-        g = aL + (L >= 0.0f ? h : hm) - 1.0f;  // |L| + h(|L|) - 1
+    const float x = (2.0f * kLn2f) * L2;  // 2 L
+    float h, hm, g;
+    fhg(x, 2.0f * L2, h, hm, g);
+    const float ix = frcp(xsq), ix2 = frcp(x2sq), iz = frcp(zsq);
+    const float zq = z * z, z2q = z2 * z2;
+    const float B2 = z2q * iz * ix2, C2 = ix * ix2, D2 = zq * iz * ix;
+    const float A = zz2 * iz;
+    const float A2g = (2.0f * A) * (A * g);
+    const float k = fmaf(x, D2, fmaf(h, fmaf(-4.0f, B2, C2), A2g));
+    const float ks = fmaf(-x, B2, fmaf(hm, fmaf(-4.0f, D2, C2), A2g));
+    float k2 = k * dip, k2s = ks * dips;
+    // |K2| > 1e10 with |dipole| < 1e-10 (S/bk/derivatives.py:589), J = z^2 z'^2
+    if (__any(fminf(fabsf(dip), fabsf(dips)) < 1e-10f)) {
+        keep_branch(k2);
+        const float cut = c.cut * (zq * z2q);
+        if (fabsf(k) > cut && fabsf(dip) < 1e-10f) k2 = 0.0f;
+        if (fabsf(ks) > cut && fabsf(dips) < 1e-10f) k2s = 0.0f;
     }
-    const float A = z * z2 * (iZ * iZ);
-    const float rZ = r * iZ;
-    const float B = rZ * z2 * iX2, C = r * r * (iX * iX2), D = rZ * z * iX;
-    const float B2 = B * B, C2 = C * C, D2 = D * D;
-    const float A2g = 2.0f * A * A * g;
-    float k = A2g - 4.0f * h * B2 + h * C2 + 2.0f * L * D2;
-    float ks = A2g - 4.0f * hm * D2 + hm * C2 - 2.0f * L * B2;
-    const float zz2 = z * z2;
-    const float cut = 1e10f * (zz2 * zz2);  // |K2| > 1e10 (S/bk/derivatives.py:589), J = z^2 z'^2
-    if (fabsf(k) > cut && fabsf(dip) < 1e-10f) { k = 0.0f; dip = 0.0f; }
-    if (fabsf(ks) > cut && fabsf(dips) < 1e-10f) { ks = 0.0f; dips = 0.0f; }
-    float k2r = symmetrize ? (k * dip + ks * dips) * 0.5f : k * dip;
-    float kfr = 0.0f;
-    if (nf_over_nc > 0.0f) {
-        const float kf = (h * B2 - A2g) * nf_over_nc;
-        const float kfs = (hm * D2 - A2g) * nf_over_nc;
-        const float df = s_y * (n_x - n_x2);
-        const float dfs = s_y2 * (n_x2 - n_x);
-        kfr = -(symmetrize ? (kf * df + kfs * dfs) * 0.5f : kf * df);
-    }
-    // smallest distance, base 2
-    const float log_min = fminf(fminf(fminf(log2_r, log_x), t1), fminf(fminf(log_x2, t2), log_zz));
+    const float kf = fmaf(h, B2, -A2g) * s_y, kfs = fmaf(hm, D2, -A2g) * s_y2;
+    // smallest distance but r, whose logarithm is 0 here
+    const float log_min = fmin3(fmin3(log_x, t1, log_x2), t2, log_zz);
     float as;
     if (!ANYC || cpl.mode == 0) {  // smooth coupling at the smallest distance (production)
         // in base 2: right = 5 (ln s0 - 2 ln d) log2 e, mu = ln mu0 log2 e,
-        // alpha = 1 / (b0 0.2 ln 2 (max(mu, right) + log2(1 + 2^-|mu - right|)))
-        const float right = fmaf(-10.0f, log_min, cpl.log_scale0 * (5.0f * kLog2ef));
-        const float mu = cpl.log_mu0 * kLog2ef;
-        const float hi = fmaxf(mu, right);
-        // 2^-|d| <= 1 is added to 1: the plain log2 is accurate enough here
-        const float t = fexp2(-fabsf(mu - right));
-        as = frcp((cpl.b0 * (0.2f * kLn2f)) * (hi + flog2(1.0f + t)));
+        // alpha = 1 / (b0 0.2 ln 2 (max(mu, right) + log2(1 + 2^-|mu - right|)));
+        // the last term is below half an ulp of the sum (>= 13) for |mu - right| > 22
+        const float right = fmax2(fmaf(-10.0f, log_min, c.right0), c.right0);
+        float den = fmax2(c.mu, right);
+        float d = c.mu - right;
+        if (__any(fabsf(d) < 22.0f)) {
+            keep_branch(d);
+            den += flog2(1.0f + fexp2(-fabsf(d)));
+        }
+        as = frcp(c.b0 * den);
     } else if (cpl.mode == 1) {
         as = cpl.as_const;
     } else {
-        as = alpha_thresholds_log<float>(log_min * kLn2f, cpl.log_4c2);
+        as = alpha_thresholds_log<float>((fminf(log_min, 0.0f) + c.log2_r) * kLn2f, cpl.log_4c2);
     }
-    const float scale = (as * nc) * (as * nc) * norm;
+    const float scale = (as * as) * c.norm;
+    // Kf's dipole difference is df = n_x - n_x2 and its mirror
+    float k2r = fmaf(c.mirror, k2s, k2), kfr = dnx * fmaf(-c.mirror, kfs, kf);
+    out.total = fmaf(-c.nf_over_nc, kfr, k2r) * scale;
+    const bool finite = isfinite(out.total);
+    if (finite && !SPLIT) return out;
+    if (c.mirror == 0.0f) {  // 0 times an infinite mirror image
+        k2r = k2;
+        kfr = dnx * kf;
+    }
     k2r *= scale;
-    kfr *= scale;
+    kfr = c.nf_over_nc > 0.0f ? -c.nf_over_nc * kfr * scale : 0.0f;
     out.k2 = isfinite(k2r) ? k2r : 0.0f;
     out.kf = isfinite(kfr) ? kfr : 0.0f;
-    out.total = out.k2 + out.kf;
+    if (!finite) out.total = out.k2 + out.kf;
     return out;
 }
 

@@ -64,6 +64,13 @@ namespace {
 
 // ------------------------------------------------------------ LDS staging
 
+// A value the compiler keeps in a vector register (it would put a
+// launch-invariant one into a scalar register).
+__device__ __forceinline__ float vector_reg(float v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 template <typename T>
 __device__ void stage_spline(const T* table, int R, int row, T* x, T* rec, LdsSpline<T>& s) {
     // table: [r_min, r_max, ln r (R), N records 4 (R-1), S records 4 (R-1)]
@@ -750,7 +757,7 @@ __host__ __device__ inline NloLayout nlo_layout(int R, int bins, int spt, bool h
     if (tsize == sizeof(double)) o = align_up(o + (size_t)R * tsize, 16);  // FP32 needs no nodes
     L.rec = o;  // FP64: R - 1 records; FP32: R + 1 (with the two range records)
     o = align_up(o + (size_t)4 * (tsize == sizeof(double) ? R - 1 : R + 1) * tsize, 16);
-    L.edges = o;  // FP64: 4 x (bins + 1) edges; FP32: 4 x bins (left, width) pairs
+    L.edges = o;  // FP64: 4 x (bins + 1) edges; FP32: bins x 4 (left, width) pairs
     o = align_up(o + (size_t)4 * (bins + 1) * sizeof(double), 16);
     if (hist) {
         L.absw = o;
@@ -778,12 +785,13 @@ struct NloArgs {
     double* part_hist;  // (R - 1) x bpp x 4 x bins
     double* part_cnt;
     BkConsts c;
-    // direction numbers: [0] as the sequence has them, [1] reordered for the
-    // first `ordered` 64-point groups (sobol_order.hpp)
+    // the Sobol state times 4 (32 bits of the unit interval); direction
+    // numbers: [0] as the sequence has them, [1] reordered for the first
+    // `ordered` 64-point groups (sobol_order.hpp)
     uint32_t dir[2][4][NLO_SOBOL_BITS];
     int64_t ordered;
     uint32_t shift[4];
-    uint32_t first_q[4];
+    uint32_t first_q[4];  // the first point's state itself (2^30 may occur)
 };
 
 // The Sobol side of the arguments.  Reordering whole blocks of spt groups per
@@ -794,14 +802,16 @@ struct NloArgs {
 // branches, 6.30 -> 6.27 ms at 2^18 points.
 void set_sobol(NloArgs& a, const nlo_sobol_table& t, bool hist) {
     for (int d = 0; d < 4; ++d) {
-        for (int b = 0; b < NLO_SOBOL_BITS; ++b) a.dir[0][d][b] = a.dir[1][d][b] = t.direction[d][b];
-        a.shift[d] = t.shift[d];
+        for (int b = 0; b < NLO_SOBOL_BITS; ++b) a.dir[0][d][b] = a.dir[1][d][b] = t.direction[d][b] << 2;
+        a.shift[d] = t.shift[d] << 2;
         a.first_q[d] = t.first[d];
     }
     a.ordered = 0;
     const int bits = hist ? 0 : coherent_bits(a.first, a.n, kLaneBits + __builtin_ctz(a.spt));
     if (bits) {
         coherent_order(t, 4, bits, a.dir[1]);
+        for (auto& row : a.dir[1])
+            for (uint32_t& v : row) v <<= 2;
         a.ordered = (a.n >> bits) << (bits - kLaneBits);
     }
 }
@@ -869,10 +879,13 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
         }
         const double x0 = v.t64[2], xl = v.t64[2 + v.R - 1];
         const double inv_h = (double)(v.R - 1) / (xl - x0);
-        fsp.rec = rec4;
+        const double pos = 1.0 + (v.t64[2 + p] - x0) * inv_h;  // of r_p, in records
+        const double at = rint(pos);
+        fsp.rec = rec4 + (int)at;
         fsp.inv_h2 = (float)(inv_h * kLn2);  // the integrand's logarithms are base 2
-        fsp.off = (float)(1.0 - x0 * inv_h);
-        fsp.umax = (float)v.R;
+        fsp.off = (float)(pos - at);
+        fsp.vmin = (float)-at;
+        fsp.vmax = (float)(v.R - at);
     } else {
         // FP64 reference formula reads the S spline (row 1); the stable form reads N (row 0).
         stage_spline<double>(v.t64, v.R, MODE == NLO_PREC_FP64 ? 1 : 0, reinterpret_cast<double*>(sx),
@@ -885,24 +898,26 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
     const int ne = 4 * (a.bins + 1);
     const double* ep = v.edges + (size_t)p * ne;
     if constexpr (MODE == NLO_PREC_FP32) {
-        // Per bin, the absolute left end lo + w left and width w (right - left)
-        // of the mapped interval, formed in FP64 and rounded once: the sample
-        // is then x = X_b + W_b frac with one more rounding, where forming
-        // lo + w (left + width frac) in FP32 cancels (lo = ln(r_0 / 2) against
-        // the scaled edge) and leaves several ulp in ln z.  The two log-r
-        // dimensions are tabulated in base 2 (times log2 e), so the sample is
-        // t = log2 z and z = 2^t exactly up to the hardware exp2; the Jacobian
-        // then carries (log2 e)^2, which the volume factor takes back.  Wave 0
-        // alone builds the table, so that only one wave of the block evaluates
-        // the two FP64 logarithms of the bounds.
+        // Per bin, the left end lo + w left and width w (right - left) of the
+        // mapped interval, formed in FP64 and rounded once: the sample is then
+        // x = X_b + W_b frac with one more rounding.  The two log-r dimensions
+        // are tabulated in base 2 and relative to log2 r_p, the two angles as
+        // half-angles modulo pi in [-pi/2, pi/2] (both ends of the angle near 0,
+        // where small values keep their precision), and every width times
+        // 2^-32, the unit of the fraction (a 32-bit word); the volume factor
+        // takes these units back.  The four dimensions of a bin are adjacent,
+        // so that the LDS address is the bin number shifted.  Wave 0 alone
+        // builds the table, so that only one wave of the block evaluates the
+        // two FP64 logarithms of the bounds.
         float2* E2 = reinterpret_cast<float2*>(smem + lay.edges);
         if (threadIdx.x < kWave) {
+            const double log_rp = v.t64[2 + p];
             for (int i = threadIdx.x; i < 4 * a.bins; i += kWave) {
-                const int d = i / a.bins, b = i - d * a.bins;
-                const double lo_d = d < 2 ? lo_r : 0.0, w_d = d < 2 ? w_r : 2.0 * kPi;
-                const double unit = d < 2 ? kLog2e : 1.0;
+                const int b = i >> 2, d = i & 3;
                 const double left = ep[d * (a.bins + 1) + b], right = ep[d * (a.bins + 1) + b + 1];
-                E2[i] = make_float2((float)((lo_d + w_d * left) * unit), (float)(w_d * (right - left) * unit));
+                const double x = d < 2 ? ((lo_r - log_rp) + w_r * left) * kLog2e : kPi * (left < 0.5 ? left : left - 1.0);
+                const double w = d < 2 ? w_r * kLog2e : kPi;
+                E2[i] = make_float2((float)x, (float)(w * (right - left)) * 0x1p-32f);
             }
         }
     } else {
@@ -929,18 +944,16 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
     const T wd[4] = {(T)w_r, (T)w_r, (T)(2.0 * kPi), (T)(2.0 * kPi)};
     T vol = T(1);
     if constexpr (MODE == NLO_PREC_FP32) {
-        // the widths W_b already carry the volume; (ln 2)^2 undoes the base-2
-        // units of the two log-r widths (one rounding of B^4 (ln 2)^2)
+        // B^4 and the table's units: (ln 2)^2 of the log-r widths, 2^2 of the
+        // half-angles, 2^96 of the four widths' 2^-128 (the other 2^32 sits in
+        // Fp32Consts::norm: the product of widths stays in the normal range)
         const double bb = (double)a.bins;
-        vol = (T)((bb * bb) * (bb * bb) * (kLn2 * kLn2));
+        vol = (T)((bb * bb) * (bb * bb) * (4.0 * kLn2 * kLn2) * 0x1p96);
     } else {
         for (int d = 0; d < 4; ++d) vol = vol * wd[d];
     }
-    const T r_t = (T)rp;
     // ln r_p as the spline table holds it (the same FP64 log of r_p)
     const double log_rp = v.t64[2 + p];
-    // the FP32 integrand takes log2 r
-    const T log_r_t = MODE == NLO_PREC_FP32 ? (T)(log_rp * kLog2e) : (T)log_rp;
     NloCoupling<float> cpl32;
     NloCoupling<double> cpl64;
     if constexpr (ANYC) {
@@ -949,6 +962,23 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
     } else {
         cpl32 = NloCoupling<float>{0, (float)a.c.b0, (float)a.c.log_mu0, (float)a.c.log_scale0, 0.0f, 0.0f};
         cpl64 = NloCoupling<double>{0, a.c.b0, a.c.log_mu0, a.c.log_scale0, 0.0, 0.0};
+    }
+    Fp32Consts c32{};
+    if constexpr (MODE == NLO_PREC_FP32) {
+        c32.pi = vector_reg(3.14159274f);
+        c32.log2_r = (float)(log_rp * kLog2e);
+        c32.cut = (float)(1e10 * ((rp * rp) * (rp * rp)));
+        c32.norm = vector_reg((float)(a.c.nc * a.c.nc * a.c.norm * (a.c.symmetrize ? 0.5 : 1.0) * 0x1p32));
+        c32.mirror = vector_reg(a.c.symmetrize ? 1.0f : 0.0f);
+        c32.nf_over_nc = vector_reg((float)(a.c.nf / a.c.nc));
+        c32.mu = vector_reg((float)a.c.log_mu0 * kLog2ef);
+        c32.right0 = vector_reg((float)((5.0 * a.c.log_scale0 - 10.0 * log_rp) * kLog2e));
+        c32.b0 = vector_reg((float)a.c.b0 * (0.2f * kLn2f));
+        vol = vector_reg((float)vol);
+        fsp.inv_h2 = vector_reg(fsp.inv_h2);
+        fsp.off = vector_reg(fsp.off);
+        fsp.vmin = vector_reg(fsp.vmin);
+        fsp.vmax = vector_reg(fsp.vmax);
     }
     const double r_min64 = v.t64[0], r_max64 = v.t64[1];
 
@@ -991,41 +1021,43 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
             if (b < NLO_SOBOL_BITS)
                 for (int d = 0; d < 4; ++d) vhi[d] ^= dir[d][b];
         }
-        const int64_t sample = (hi << 6) + lane - a.first;
-        const bool valid = sample < a.n;
+        // samples left from this group on (only the last group is ragged)
+        const int rest = (int)(a.n - ((hi << 6) - a.first));
+        const bool valid = lane < min(rest, kWave);
         const bool odd = (hi & 1) != 0;
-        uint32_t q[4];
-        for (int d = 0; d < 4; ++d) q[d] = vlo[d] ^ (odd ? (vhi[d] ^ dir[d][5]) : vhi[d]);
-        if (FIRST && lane == 0)
-            for (int d = 0; d < 4; ++d) q[d] = a.first_q[d];
         T x[4];
-        T jac = T(1);
+        T jac = vol;
         uint32_t packed = 0u;
         for (int d = 0; d < 4; ++d) {
             // bin = min(floor(u B), B - 1), frac = u B - bin with u = q 2^-30:
             // for q < 2^30, 4 q B = bin 2^32 + frac 2^32 (high and low words of
             // one 32 x 32 product); q = 2^30 (only a rounded first point) is
             // the clamped case bin = B - 1, frac = 1.
-            const uint32_t q4 = q[d] << 2;
-            uint32_t b = __umulhi(q4, (uint32_t)a.bins);
-            T frac = (T)(q4 * (uint32_t)a.bins) * (T)0x1p-32;
-            if (FIRST && q[d] >= (1u << 30)) {
+            uint32_t q4 = vlo[d] ^ (odd ? (vhi[d] ^ dir[d][5]) : vhi[d]);
+            bool top = false;
+            if (FIRST && lane == 0) {
+                q4 = a.first_q[d] << 2;
+                top = a.first_q[d] >= (1u << 30);
+            }
+            const uint64_t prod = (uint64_t)q4 * (uint32_t)a.bins;
+            uint32_t b = (uint32_t)(prod >> 32);
+            T frac = (T)(uint32_t)prod;  // times 2^32
+            if (FIRST && top) {
                 b = (uint32_t)(a.bins - 1);
-                frac = T(1);
+                frac = T(0x1p32);
             }
             if constexpr (MODE == NLO_PREC_FP32) {
-                const float2 e = reinterpret_cast<const float2*>(E)[d * a.bins + b];
+                const float2 e = reinterpret_cast<const float2(*)[4]>(E)[b][d];
                 x[d] = fmaf(e.y, frac, e.x);
                 jac = jac * e.y;
             } else {
                 const T left = E[d * (a.bins + 1) + b], right = E[d * (a.bins + 1) + b + 1];
                 const T w = right - left;
-                x[d] = lo[d] + wd[d] * (left + w * frac);
+                x[d] = lo[d] + wd[d] * (left + w * (frac * T(0x1p-32)));
                 jac = jac * ((T)a.bins * w);
             }
-            packed |= b << (8 * d);
+            if (HIST) packed |= b << (8 * d);
         }
-        jac = vol * jac;
         double wv = 0.0, k2 = 0.0, kf = 0.0;
         if (valid) {
             if constexpr (MODE == NLO_PREC_FP64) {
@@ -1035,9 +1067,8 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
                 k2 = f.k2 * (double)jac;
                 kf = f.kf * (double)jac;
             } else if constexpr (MODE == NLO_PREC_FP32) {
-                const NloStable<float> f = nlo_integrand_fp32<ANYC>(
-                    r_t, log_r_t, x[0], x[1], x[2], x[3], fsp, cpl32, (float)(a.c.nf / a.c.nc),
-                    (float)a.c.nc, (float)a.c.norm, a.c.symmetrize != 0);
+                const NloStable<float> f =
+                    nlo_integrand_fp32<ANYC, FULL>(c32, x[0], x[1], x[2], x[3], fsp, cpl32);
                 wv = (double)(f.total * jac);
                 k2 = (double)(f.k2 * jac);
                 kf = (double)(f.kf * jac);
@@ -1105,10 +1136,12 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
     }
 }
 
-// The evolver's FP32 instance (sum of w only) fits 72 VGPRs without spills:
-// 7 waves per SIMD instead of the 6 that its natural 76 would allow.
+// Waves per SIMD of the FP32 instance that sums w only (the evolver's): 8 (64
+// VGPRs, no spills); in the batch kernel, which carries its work item too, 6.
 template <int MODE, bool FULL, bool ANYC>
-constexpr int kNloWaves = (MODE == NLO_PREC_FP32 && !FULL && !ANYC) ? 7 : 1;
+constexpr int kNloWaves = (MODE == NLO_PREC_FP32 && !FULL && !ANYC) ? 8 : 1;
+template <int MODE, bool ANYC>
+constexpr int kNloBatchWaves = (MODE == NLO_PREC_FP32 && !ANYC) ? 6 : 1;
 
 template <int MODE, bool HIST, bool FULL, bool ANYC>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kNloWaves<MODE, FULL, ANYC>))) nlo_kernel(NloArgs a) {
@@ -1298,7 +1331,7 @@ struct BatchNlo {
 // run's slices; each item writes its own partial sums, so the result does not
 // depend on which block took it.
 template <int MODE, bool ANYC>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kNloWaves<MODE, false, ANYC>))) nlo_batch_kernel(NloArgs a, BatchNlo w) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kNloBatchWaves<MODE, ANYC>))) nlo_batch_kernel(NloArgs a, BatchNlo w) {
     __shared__ int64_t item_s;
     for (;;) {
         if (threadIdx.x == 0) item_s = (int64_t)atomicAdd(w.counter, 1ull);
