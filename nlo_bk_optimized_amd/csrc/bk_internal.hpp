@@ -12,7 +12,7 @@ constexpr int kMaxGaussT = 64;    // K1 angular GL order
 constexpr int kMaxGkIntervals = 100;  // adaptive K1: intervals per list (RINTPOINTS, THETAINTPOINTS)
 
 struct NloPlan {
-    int spt;              // samples per lane
+    int spt;              // samples per lane, at most
     int bpp;              // blocks per parent
     size_t part_bytes;    // per-block sums
     size_t hist_bytes;    // per-block histograms (0 without histogram)
@@ -25,7 +25,9 @@ int validate_physics(const nlo_bk_physics* p);
 // (once per process; must run before any stream capture).
 int init_kernel_attributes();
 
-NloPlan nlo_plan(int R, int bins, int64_t n, bool hist);
+// The workspace of the FP64 plan, which has the shorter runs, holds the FP32
+// plan's too.
+NloPlan nlo_plan(int R, int bins, int64_t n, bool hist, bool fp32 = false);
 
 int launch_spline_build(int R, const double* r, const double* N, int force_positive, double* t64,
                         float* t32, hipStream_t stream);

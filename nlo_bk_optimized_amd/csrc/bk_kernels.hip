@@ -2,6 +2,7 @@
 // sums with in-kernel Sobol points, deterministic reductions, RHS finalize and
 // RK stage updates.  Reference prefixes: S/ = torch_nlo_clean/src/nlo_torch/,
 // K/ = S/custom_kernels/.
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 #include <type_traits>
@@ -774,7 +775,10 @@ __host__ __device__ inline NloLayout nlo_layout(int R, int bins, int spt, bool h
 }
 
 struct NloArgs {
-    int R, bins, spt, bpp;
+    int R, bins;
+    int spt;     // 64-point groups per wave, at most (the LDS stages so many of a histogram pass)
+    int bpp;     // blocks per parent
+    int groups;  // 64-point groups of the launch
     int64_t n, first;
     const double* r;
     const double* N;
@@ -787,33 +791,43 @@ struct NloArgs {
     BkConsts c;
     // the Sobol state times 4 (32 bits of the unit interval); direction
     // numbers: [0] as the sequence has them, [1] reordered for the first
-    // `ordered` 64-point groups (sobol_order.hpp)
+    // `ordered` 64-point groups, which the parent's first `ordered_waves`
+    // waves take (sobol_order.hpp)
     uint32_t dir[2][4][NLO_SOBOL_BITS];
-    int64_t ordered;
+    int ordered, ordered_waves;
     uint32_t shift[4];
     uint32_t first_q[4];  // the first point's state itself (2^30 may occur)
 };
 
-// The Sobol side of the arguments.  Reordering whole blocks of spt groups per
-// wave or more, so that a wave's groups lie on one side of the border; not
-// for histogram passes, whose LDS atomics want the lanes of a wave in
-// different bins.  A 256-node FP32 RK2 step of 2^20 points: 3.424 -> 3.336 ms
-// (the branches on r/z and L no longer diverge); FP64, which has few such
-// branches, 6.30 -> 6.27 ms at 2^18 points.
+// The Sobol side of the arguments (after n, first).  Not reordered for
+// histogram passes, whose LDS atomics want the lanes of a wave in different
+// bins.  A 256-node FP32 RK2 step of 2^20 points: 3.424 -> 3.336 ms (the
+// branches on r/z and L no longer diverge); FP64, which has few such branches,
+// 6.30 -> 6.27 ms at 2^18 points.
 void set_sobol(NloArgs& a, const nlo_sobol_table& t, bool hist) {
     for (int d = 0; d < 4; ++d) {
         for (int b = 0; b < NLO_SOBOL_BITS; ++b) a.dir[0][d][b] = a.dir[1][d][b] = t.direction[d][b] << 2;
         a.shift[d] = t.shift[d] << 2;
         a.first_q[d] = t.first[d];
     }
-    a.ordered = 0;
-    const int bits = hist ? 0 : coherent_bits(a.first, a.n, kLaneBits + __builtin_ctz(a.spt));
-    if (bits) {
-        coherent_order(t, 4, bits, a.dir[1]);
-        for (auto& row : a.dir[1])
-            for (uint32_t& v : row) v <<= 2;
-        a.ordered = (a.n >> bits) << (bits - kLaneBits);
-    }
+    a.ordered = a.ordered_waves = 0;
+    a.groups = (int)((a.n + kWave - 1) / kWave);
+    const int bits = hist ? 0 : coherent_bits(a.first, a.n);
+    if (!bits) return;
+    // The rest behind the ordered blocks has waves of its own, as many as its
+    // share asks for; where the longest run of groups would grow by more than
+    // a sixteenth for it, the order is left alone.
+    const int waves = 4 * a.bpp, ordered = (int)((a.n >> bits) << (bits - kLaneBits)), rest = a.groups - ordered;
+    const int rest_waves = (int)(((int64_t)rest * waves + a.groups - 1) / a.groups);
+    if (rest_waves >= waves) return;
+    auto longest = [](int groups, int w) { return w ? (groups + w - 1) / w : 0; };
+    const int run = longest(a.groups, waves);
+    if (std::max(longest(ordered, waves - rest_waves), longest(rest, rest_waves)) > run + run / 16) return;
+    coherent_order(t, 4, bits, a.dir[1]);
+    for (auto& row : a.dir[1])
+        for (uint32_t& v : row) v <<= 2;
+    a.ordered = ordered;
+    a.ordered_waves = waves - rest_waves;
 }
 
 // One evolution's arrays as an NLO block reads them (a single run: NloArgs'
@@ -828,10 +842,10 @@ struct RunView {
     double* part;
 };
 
-// Per (parent, block): spt samples per lane.  Sample ordinal
-// s = (blk * spt * 4 + j * 4 + wave) * 64 + lane, Sobol index first + s, so
-// lanes of a wave hold 64 consecutive indices and the gray-code state splits
-// into a wave-uniform high part and a per-lane low part.
+// Per (parent, block): the launch's 64-point groups are dealt to the parent's
+// 4 bpp waves in consecutive runs of equal length (one more for the first
+// ones; ordered groups and the rest each by themselves).  Group hi holds the Sobol indices 64 hi + lane, so that the gray-code
+// state splits into a wave-uniform high part and a per-lane low part.
 // FULL = false (the evolver): only sum w is accumulated; the sum of w^2 and
 // the K2 / Kf split read as 0.
 // ANYC: any coupling choice (NloCoupling modes); false = the production
@@ -984,14 +998,20 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
 
     const int lane = threadIdx.x & 63;
     const int wave = uniform(threadIdx.x >> 6);
-    // Each wave walks spt consecutive 64-point groups hi0 + j; the state splits
-    // into a per-lane part (direction bits 0..5 of the lane's gray code) and a
-    // wave-uniform part (bits 6..29 of gray(hi), and bit 5 for odd hi), read
-    // from the kernel arguments so that it stays scalar, built once and then
-    // updated by one XOR per group: gray(h) ^ gray(h - 1) = lowest set bit of h.
-    const int64_t g0 = ((int64_t)blk * 4 + wave) * a.spt;
-    const int64_t hi0 = (a.first >> 6) + g0;
-    const uint32_t(*dir)[NLO_SOBOL_BITS] = a.dir[g0 < a.ordered ? 1 : 0];
+    // this wave's groups g0 .. g0 + mine of the launch, hi0 .. of the sequence
+    const int wv = blk * 4 + wave;
+    const bool ordered = wv < a.ordered_waves;
+    const int waves = ordered ? a.ordered_waves : 4 * a.bpp - a.ordered_waves;
+    const int total = ordered ? a.ordered : a.groups - a.ordered, w0 = ordered ? wv : wv - a.ordered_waves;
+    const int share = total / waves, extra = total - share * waves;
+    const int mine = share + (w0 < extra ? 1 : 0);
+    const int64_t hi0 = (a.first >> 6) + (ordered ? 0 : a.ordered) + (int64_t)w0 * share + min(w0, extra);
+    // The state of group hi: a per-lane part (direction bits 0..5 of the lane's
+    // gray code) and a wave-uniform part (bits 6..29 of gray(hi), and bit 5 for
+    // odd hi), read from the kernel arguments so that it stays scalar, built
+    // once and then updated by one XOR per group: gray(h) ^ gray(h - 1) =
+    // lowest set bit of h.
+    const uint32_t(*dir)[NLO_SOBOL_BITS] = a.dir[ordered ? 1 : 0];
     const uint32_t glo = (uint32_t)(lane ^ (lane >> 1));
     uint32_t vlo[4], vhi[4];
     for (int d = 0; d < 4; ++d) {
@@ -1017,7 +1037,7 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
         constexpr bool FIRST = decltype(first_tag)::value;
         const int64_t hi = hi0 + j;
         if (j > 0) {
-            const int b = 6 + __builtin_ctzll((unsigned long long)hi);
+            const int b = kLaneBits + __builtin_ctzll((unsigned long long)hi);
             if (b < NLO_SOBOL_BITS)
                 for (int d = 0; d < 4; ++d) vhi[d] ^= dir[d][b];
         }
@@ -1093,11 +1113,11 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
         }
     };
     int j0 = 0;
-    if (hi0 == 0) {
+    if (hi0 == 0 && mine > 0) {
         group(0, std::true_type{});
         j0 = 1;
     }
-    for (int j = j0; j < a.spt; ++j) group(j, std::false_type{});
+    for (int j = j0; j < mine; ++j) group(j, std::false_type{});
     // the block's partials, each one rounding of its compensated pair
     if constexpr (FULL) {
         double t[4] = {s1, s2, sk2, skf}, e[4] = {c1, c2, ck2, ckf};
@@ -1110,14 +1130,14 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
     if (HIST) {
         // block max of |w| -> fixed-point scale; integer LDS sums are exact
         double m = 0.0;
-        for (int j = 0; j < a.spt; ++j) m = fmax(m, st_w[threadIdx.x + j * 256]);
+        for (int j = 0; j < mine; ++j) m = fmax(m, st_w[threadIdx.x + j * 256]);
         m = wave_max(m);
         if (lane == 0) wmax[wave] = m;
         __syncthreads();
         m = fmax(fmax(wmax[0], wmax[1]), fmax(wmax[2], wmax[3]));
         const int e = m > 0.0 ? ilogb(m) : 0;
         const int sc = 50 - e;  // m 2^sc < 2^51, <= 2^12 terms stay below 2^63
-        for (int j = 0; j < a.spt; ++j) {
+        for (int j = 0; j < mine; ++j) {
             const uint32_t pk = st_b[threadIdx.x + j * 256];
             if (pk == 0xffffffffu) continue;
             const unsigned long long v =
@@ -1520,16 +1540,26 @@ int launch_k1_adaptive(int R, const double* r, const double* N, const double* t6
     return NLO_OK;
 }
 
-NloPlan nlo_plan(int R, int bins, int64_t n, bool hist) {
+// How many 64-point groups a wave runs through.  A block pays for its tables
+// and for the reads that lead to them once, which long runs amortise; runs are
+// as long as still leaves about 2 500 blocks (256 CUs hold 2 048 of the FP32
+// evolver's), at least 4 and, for the tail of the launch, at most 16 groups;
+// 64 in FP32 beyond 2^18 points (up to there a single run keeps the batch
+// kernel's 16 and both sum alike bit for bit; FP64 samples take ten times as
+// long and gain nothing).  A launch with runs of 4, 8 or 16 by 8 192 blocks
+// against this rule: 100 000 points of 100 parents 91 -> 80 us, 2^14 of 255
+// 80 -> 44 us, 2^20 of 255 1 222 -> 1 160 us.  A histogram pass stages its
+// samples in the LDS, at most 8 per lane.
+NloPlan nlo_plan(int R, int bins, int64_t n, bool hist, bool fp32) {
     NloPlan pl{};
-    // Enough blocks to fill 256 CUs several times over; each lane evaluates
-    // spt samples (at most 8 when the histogram stages them in LDS).
-    const int64_t parents = R - 1;
-    int spt = 16;
-    while (spt > 1 && parents * ((n + 256 * spt - 1) / (256 * spt)) < 8192) spt /= 2;
-    if (hist && spt > 8) spt = 8;
-    pl.spt = spt;
-    pl.bpp = (int)((n + 256 * spt - 1) / (256 * spt));
+    const int64_t parents = R - 1, groups = (n + kWave - 1) / kWave;
+    int64_t run = std::min<int64_t>(std::max<int64_t>(parents * groups / 10000, 4), fp32 && n > (1 << 18) ? 64 : 16);
+    if (hist) {
+        run = 8;
+        while (run > 1 && parents * ((groups + 4 * run - 1) / (4 * run)) < 8192) run /= 2;
+    }
+    pl.spt = (int)run;
+    pl.bpp = (int)((groups + 4 * run - 1) / (4 * run));
     pl.part_bytes = (size_t)parents * pl.bpp * 4 * sizeof(double);
     pl.hist_bytes = hist ? (size_t)parents * pl.bpp * 4 * bins * sizeof(double) : 0;
     pl.workspace = align_up(pl.part_bytes, 256) + 2 * align_up(pl.hist_bytes, 256);
@@ -1541,7 +1571,7 @@ int launch_nlo(int R, const double* r, const double* N, const double* t64, const
                int precision, const BkConsts& c, double* sums, double* hist, double* count,
                void* ws, size_t ws_bytes, hipStream_t stream, bool components) {
     const bool want_hist = hist != nullptr;
-    const NloPlan pl = nlo_plan(R, bins, n, want_hist);
+    const NloPlan pl = nlo_plan(R, bins, n, want_hist, precision == NLO_PREC_FP32);
     if (ws_bytes < pl.workspace || (!ws && pl.workspace)) {
         set_error("nlo_bk_nlo: workspace %zu bytes < %zu", ws_bytes, pl.workspace);
         return NLO_ERR_WORKSPACE;

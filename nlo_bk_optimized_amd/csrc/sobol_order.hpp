@@ -23,10 +23,10 @@ namespace nlo {
 constexpr int kLaneBits = 6;  // 64 lanes
 
 // The largest block worth reordering for points [first, first + n): aligned
-// to first, at least `min_bits`, and whole blocks holding 15/16 of the points
-// (the rest keeps the natural order).  0: no such block.
-inline int coherent_bits(int64_t first, int64_t n, int min_bits) {
-    for (int bits = 24; bits >= min_bits && bits > kLaneBits; --bits) {
+// to first, and whole blocks holding 15/16 of the points (the rest keeps the
+// natural order).  0: no such block.
+inline int coherent_bits(int64_t first, int64_t n) {
+    for (int bits = 24; bits > kLaneBits; --bits) {
         const int64_t size = (int64_t)1 << bits;
         if (first % size == 0 && (n >> bits << bits) >= n - n / 16) return bits;
     }
