@@ -344,12 +344,21 @@ __global__ void __launch_bounds__(kK1Threads) k1_kernel(int R, const double* __r
 // Gauss-Kronrod 21 (adaptive_gauss_kronrod_1d, S/numerics/integration.py:
 // 43-92; the rule and its error of :624-746) in ln z over [ln r_0, ln r_{R-1}]
 // of 2 z^2 times the adaptive rule in theta over [0, pi].  One block per
-// parent: thread 0 keeps the outer interval list; every outer node is an
-// inner integral, taken by the next free wave, whose 64 lanes evaluate the
-// 21 (first interval) or 42 (two halves) theta nodes of each bisection step
-// while every lane runs the same list bookkeeping on LDS.  Interval lists
-// stay in order and sums run in list order, as in the reference.
-constexpr int kK1aWaves = 8;
+// parent; every outer node is an inner integral, taken by the next free wave.
+//
+// Bound by latency: a bisection is one step of a serial chain, so the design
+// shortens the step.  A wave keeps an interval list in registers, one or two
+// intervals per lane; the two halves of a bisection are evaluated by its two
+// half-waves, one node per lane, and every sum over nodes or intervals is a
+// lane reduction by data-parallel moves with no trip through the LDS.  The
+// rule's weights are then one register per lane.  With the list, the rule and
+// the sums in one lane's code and the list in the LDS the same work took 4.83
+// ms on 256 nodes (epsrel 1e-3) and 7.09 ms on 101; now 3.35 and 4.81 ms.
+// Three waves per SIMD (168 registers, 12 spilled) are the best: 8 waves a
+// block take 3.60 and 5.21 ms, 16 waves (30 spilled) 3.98 and 5.62.
+// The second coupling keeps its 8.
+template <bool ANY>
+constexpr int kK1aWaves = ANY ? 8 : 12;
 
 // QUADPACK's 21-point Kronrod extension of the 10-point Gauss rule: nodes
 // kGkX[0..9] (kGkX[1, 3, .., 9] are the Gauss nodes), centre node last.
@@ -371,33 +380,85 @@ __device__ constexpr double kGW[5] = {
     0.219086362515982043995534934228163, 0.269266719309996355091226921569469,
     0.295524224714752870173892994651338};
 
-// Node k (0..20) of [a, b]: centre - h x_k, k < 10; centre, k = 10; centre + h x_{k-11}.
-__device__ __forceinline__ double gk_node(double a, double b, int k) {
-    const double center = (a + b) / 2.0, half = (b - a) / 2.0;
-    if (k < 10) return center - half * kGkX[k];
-    if (k == 10) return center;
-    return center + half * kGkX[k - 11];
+// A lane's node of the rule on the interval its half-wave looks at: lanes 0-20
+// and 32-52 hold centre - half x_k (k < 10), the centre, centre + half x_k;
+// the others sit out with weight 0.
+struct GkLane {
+    double x, wk, wg;  // node on [-1, 1], Kronrod weight, Gauss weight (0 off the Gauss nodes)
+    bool active;
+};
+
+__device__ __forceinline__ GkLane gk_lane(int lane) {
+    const int k = lane & 31;
+    GkLane g;
+    g.active = k < 21;
+    const int i = k < 10 ? k : (k > 10 && k < 21 ? k - 11 : 0);
+    g.x = k < 10 ? -kGkX[i] : (k > 10 && k < 21 ? kGkX[i] : 0.0);
+    g.wk = k == 10 ? kGkWCenter : (g.active ? kGkW[i] : 0.0);
+    g.wg = g.active && k != 10 && (i & 1) ? kGW[i >> 1] : 0.0;
+    return g;
 }
 
-// The estimate and error of _gauss_kronrod_intervals from the 21 values v
-// (node order of gk_node): min(1, (200 |K - G| / resasc)^1.5) resasc, at
-// least 50 eps resabs.
-__device__ __forceinline__ void gk_from_values(double a, double b, const double* v, double& est,
-                                               double& err) {
-    const double half = (b - a) / 2.0;
-    const double fc = v[10];
-    double kron = 0.0, gauss = 0.0;
-    for (int i = 0; i < 10; ++i) kron += (v[i] + v[11 + i]) * kGkW[i];
-    kron += kGkWCenter * fc;
-    for (int i = 0; i < 5; ++i) gauss += (v[2 * i + 1] + v[12 + 2 * i]) * kGW[i];
+// Sums over lanes, the same bits in every lane that shares a sum: within a row
+// of 16 lanes by rotations, then over the rows of a half-wave and the two
+// half-waves by the row exchanges.
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ void row_pair(double v, double& a, double& b) {
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
+    a = __hiloint2double(hi[0], lo[0]);
+    b = __hiloint2double(hi[1], lo[1]);
+}
+__device__ __forceinline__ void half_pair(double v, double& a, double& b) {
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
+    a = __hiloint2double(hi[0], lo[0]);
+    b = __hiloint2double(hi[1], lo[1]);
+}
+__device__ __forceinline__ double half_wave_sum(double v) {
+    v += dpp_move<0x128>(v);  // row rotations by 8, 4, 2, 1
+    v += dpp_move<0x124>(v);
+    v += dpp_move<0x122>(v);
+    v += dpp_move<0x121>(v);
+    double a, b;
+    row_pair(v, a, b);
+    return a + b;
+}
+__device__ __forceinline__ double whole_wave_sum(double v) {
+    double a, b;
+    half_pair(half_wave_sum(v), a, b);
+    return a + b;
+}
+__device__ __forceinline__ double whole_wave_max(double v) {
+    v = fmax(v, dpp_move<0x128>(v));
+    v = fmax(v, dpp_move<0x124>(v));
+    v = fmax(v, dpp_move<0x122>(v));
+    v = fmax(v, dpp_move<0x121>(v));
+    double a, b;
+    row_pair(v, a, b);
+    half_pair(fmax(a, b), a, b);
+    return fmax(a, b);
+}
+__device__ __forceinline__ double read_lane(double v, int lane) {
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
+    return __hiloint2double(hi, lo);
+}
+
+// The estimate and error of _gauss_kronrod_intervals on an interval of half
+// width `half` from the nodes' values v, one interval per half-wave: min(1,
+// (200 |K - G| / resasc)^1.5) resasc, at least 50 eps resabs.
+__device__ __forceinline__ void gk_rule(const GkLane& g, double half, double v, double& est, double& err) {
+    const double f = g.active ? v : 0.0;
+    const double kron = half_wave_sum(g.wk * f), gauss = half_wave_sum(g.wg * f);
     const double mean = kron / 2.0;
-    double sabs = 0.0, sasc = 0.0;
-    for (int i = 0; i < 10; ++i) {
-        sabs += (fabs(v[i]) + fabs(v[11 + i])) * kGkW[i];
-        sasc += (fabs(v[i] - mean) + fabs(v[11 + i] - mean)) * kGkW[i];
-    }
-    const double resabs = half * (sabs + kGkWCenter * fabs(fc));
-    const double resasc = half * (sasc + kGkWCenter * fabs(fc - mean));
+    const double resabs = half * half_wave_sum(g.wk * fabs(f));
+    const double resasc = half * half_wave_sum(g.wk * fabs(f - mean));
     double e = half * fabs(kron - gauss);
     // (200 |K - G| / resasc)^1.5 as q sqrt(q): within an ulp of pow(q, 1.5)
     // at the cost of one square root
@@ -408,95 +469,71 @@ __device__ __forceinline__ void gk_from_values(double a, double b, const double*
     err = fmax(e, 50.0 * 2.220446049250313e-16 * resabs);
 }
 
-// Ordered interval list in LDS: lower, upper, estimate, error (cap entries each).
+// An interval list of at most 128 entries over the lanes of a wave: entry i in
+// slot i / 64 of lane i % 64.  An empty slot holds estimate and error 0.
 struct GkList {
-    double* lo;
-    double* hi;
-    double* est;
-    double* err;
+    double lo[2], hi[2], est[2], err[2];
 };
 
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+__device__ __forceinline__ void gk_set(GkList& L, int entry, int lane, double lo, double hi, double est,
+                                       double err) {
+    if (lane == (entry & 63)) {
+        const bool second = entry >= 64;
+        L.lo[0] = second ? L.lo[0] : lo;
+        L.hi[0] = second ? L.hi[0] : hi;
+        L.est[0] = second ? L.est[0] : est;
+        L.err[0] = second ? L.err[0] : err;
+        L.lo[1] = second ? lo : L.lo[1];
+        L.hi[1] = second ? hi : L.hi[1];
+        L.est[1] = second ? est : L.est[1];
+        L.err[1] = second ? err : L.err[1];
+    }
 }
 
-// The summed estimate and error of a list in list order, and its first
-// interval of largest error, by a whole wave: lanes 0-31 sum the estimates,
-// lanes 32-63 the errors and find the first largest one; lanes 0 and 32 hand
-// the results to the wave.
-__device__ __forceinline__ void gk_scan_wave(const GkList& L, int count, double& value, double& error,
-                                             int& split, int lane) {
-    const bool upper = lane >= 32;
-    const double* x = upper ? L.err : L.est;
-    double acc = 0.0, best = L.err[0];
-    int arg = 0;
-    for (int i = 0; i < count; ++i) {
-        const double xi = x[i];
-        acc += xi;
-        if (xi > best) {  // err[i] > err[arg] on the upper half
-            best = xi;
-            arg = i;
-        }
-    }
-    value = __shfl(acc, 0, 64);
-    error = __shfl(acc, 32, 64);
-    split = __shfl(arg, 32, 64);
+__device__ __forceinline__ void gk_start(GkList& L, int lane, double lo, double hi, double est, double err) {
+    for (int s = 0; s < 2; ++s) L.lo[s] = L.hi[s] = L.est[s] = L.err[s] = 0.0;
+    gk_set(L, 0, lane, lo, hi, est, err);
 }
 
-// The rule on [a, mid] (values v[0..20]) and on [mid, b] (v[21..41]) by a
-// whole wave: lanes 0-31 sum the first, lanes 32-63 the second; lanes 0 and
-// 32 hand the results to the wave.
-__device__ __forceinline__ void gk_halves_wave(double a, double mid, double b, const double* v, double& e0,
-                                               double& r0, double& e1, double& r1, int lane) {
-    const bool upper = lane >= 32;
-    double eh, rh;
-    gk_from_values(upper ? mid : a, upper ? b : mid, upper ? v + 21 : v, eh, rh);
-    e0 = __shfl(eh, 0, 64);
-    r0 = __shfl(rh, 0, 64);
-    e1 = __shfl(eh, 32, 64);
-    r1 = __shfl(rh, 32, 64);
+__device__ __forceinline__ void gk_totals(const GkList& L, int count, double& value, double& error) {
+    double v = L.est[0], e = L.err[0];
+    if (count > 64) {
+        v += L.est[1];
+        e += L.err[1];
+    }
+    value = whole_wave_sum(v);
+    error = whole_wave_sum(e);
 }
 
-// Replace entry `split` of a list of `count` (< cap <= 128) entries by its
-// halves [lo, mid] and [mid, hi] (estimates e0, e1; errors r0, r1), moving the
-// entries after it one place up.  Every lane of one wave calls it: each lane
-// reads up to two of the entries to move, the fence orders all reads before
-// the writes, then lane 0 writes the two halves.
-__device__ __forceinline__ void gk_insert_wave(const GkList& L, int count, int split, double mid,
-                                               double e0, double r0, double e1, double r1, int lane) {
-    const double l = L.lo[split], u = L.hi[split];
-    double m[2][4];
-    int idx[2];
-    for (int k = 0; k < 2; ++k) {
-        idx[k] = split + 1 + lane + 64 * k;
-        if (idx[k] < count) {
-            m[k][0] = L.lo[idx[k]];
-            m[k][1] = L.hi[idx[k]];
-            m[k][2] = L.est[idx[k]];
-            m[k][3] = L.err[idx[k]];
-        }
+// The entry of largest error (the first one) and its interval.
+__device__ __forceinline__ int gk_worst(const GkList& L, int count, double& lo, double& hi) {
+    const double top = whole_wave_max(count > 64 ? fmax(L.err[0], L.err[1]) : L.err[0]);
+    unsigned long long m = __ballot(L.err[0] == top);
+    int slot = 0;
+    if (m == 0 && count > 64) {
+        m = __ballot(L.err[1] == top);
+        slot = 1;
     }
-    wave_sync();
-    for (int k = 0; k < 2; ++k) {
-        if (idx[k] < count) {
-            L.lo[idx[k] + 1] = m[k][0];
-            L.hi[idx[k] + 1] = m[k][1];
-            L.est[idx[k] + 1] = m[k][2];
-            L.err[idx[k] + 1] = m[k][3];
-        }
-    }
-    if (lane == 0) {
-        L.lo[split] = l;
-        L.hi[split] = mid;
-        L.est[split] = e0;
-        L.err[split] = r0;
-        L.lo[split + 1] = mid;
-        L.hi[split + 1] = u;
-        L.est[split + 1] = e1;
-        L.err[split + 1] = r1;
-    }
+    const int at = m ? __builtin_ctzll(m) : 0;  // no match: errors that are no numbers
+    lo = read_lane(slot ? L.lo[1] : L.lo[0], at);
+    hi = read_lane(slot ? L.hi[1] : L.hi[0], at);
+    return 64 * slot + at;
+}
+
+// Both halves of [a, b] as the half-waves see them, and the lane's node there.
+__device__ __forceinline__ double gk_half_node(const GkLane& g, double a, double mid, double b, int lane,
+                                               double& half) {
+    const double l = lane < 32 ? a : mid, u = lane < 32 ? mid : b;
+    half = (u - l) / 2.0;
+    return (l + u) / 2.0 + half * g.x;
+}
+
+// Entry `worst` of a list of `count` becomes [a, mid], a new entry [mid, b],
+// from the half-waves' estimates and errors.
+__device__ __forceinline__ void gk_split(GkList& L, int worst, int count, int lane, double a, double mid, double b,
+                                         double est, double err) {
+    gk_set(L, worst, lane, a, mid, read_lane(est, 0), read_lane(err, 0));
+    gk_set(L, count, lane, mid, b, read_lane(est, 32), read_lane(err, 32));
 }
 
 // The per-daughter terms of the K1 integrand at z = e^{log_z} (K1Z).
@@ -516,68 +553,68 @@ __device__ __forceinline__ K1Z k1_daughter(const K1Parent& P, double log_z, cons
     return Z;
 }
 
-// _lo_integrand (S/bk/derivatives.py:434-468) at angle theta.
+// sin^2 y for y in [0, pi/2]: with w = y (pi - y), sin y = cos((pi^2/4 -
+// w)^1/2) is entire in w, and sin y / w is its degree-8 interpolant at
+// Chebyshev nodes of [0, pi^2/4] (relative error 3e-20; all terms positive).
+__device__ __forceinline__ double sin2_quadrant(double y) {
+    const double w = y * (kPi - y);
+    double p = fma(w, 1.5070686439285400088e-16, 4.4416425756421120182e-14);
+    p = fma(w, p, 1.0560867829056239888e-11);
+    p = fma(w, p, 1.8975085675213420456e-9);
+    p = fma(w, p, 2.4609343506619309446e-7);
+    p = fma(w, p, 0.000021586579361110788302);
+    p = fma(w, p, 0.0011602715472401966982);
+    p = fma(w, p, 0.03225153443319948851);
+    p = fma(w, p, 0.31830988618379067155);
+    const double s = w * p;
+    return s * s;
+}
+
+// _lo_integrand (S/bk/derivatives.py:434-468) at angle theta, s2 = sin^2(theta / 2).
 template <bool ANY>
-__device__ __forceinline__ double k1_theta_value(const K1Parent& P, const K1Z& Z, double theta,
+__device__ __forceinline__ double k1_theta_value(const K1Parent& P, const K1Z& Z, double s2,
                                                  const LdsSpline<double>& s, const BkConsts& c,
                                                  const K1History& H, int rows, double rapidity) {
-    const double sn = sin(0.5 * theta);
     if constexpr (ANY)
-        return k1_theta_term_any(P, Z, sn * sn, s, c, H, rows, rapidity);
+        return k1_theta_term_any(P, Z, s2, s, c, H, rows, rapidity);
     else
-        return k1_theta_term(P, Z, sn * sn, s, c);
+        return k1_theta_term(P, Z, s2, s, c);
 }
 
 // The theta integral at one daughter size z (terms Z) for parent P, by one
-// wave, from the rule on [0, pi] of the block's first pass (estimate e,
-// error r); each bisection
-// of [a, b] evaluates the 21 nodes of [a, mid] (lanes 0-20) and of [mid, b]
-// (lanes 21-41).
+// wave, from the rule on [0, pi] of the block's first pass (estimate e, error
+// r).
 template <bool ANY>
-__device__ double k1_theta_adaptive(const K1Parent& P, const K1Z& Z, double e, double r,
-                                    const LdsSpline<double>& s, const BkConsts& c, const K1History& H,
-                                    int rows, double rapidity, int tint, double epsrel, const GkList& L,
-                                    double* v, int lane, long long& evals) {
-    if (lane == 0) {
-        L.lo[0] = 0.0;
-        L.hi[0] = kPi;
-        L.est[0] = e;
-        L.err[0] = r;
-    }
+__device__ __forceinline__ double k1_theta_adaptive(const K1Parent& P, const K1Z& Z, double e, double r,
+                                                    const LdsSpline<double>& s, const BkConsts& c,
+                                                    const K1History& H, int rows, double rapidity, int tint,
+                                                    double epsrel, const GkLane& g, int lane, int& evals) {
+    GkList L;
+    gk_start(L, lane, 0.0, kPi, e, r);
     evals += 21;
-    int count = 1, split = 0;
-    double value = e;
-    for (;;) {
-        wave_sync();
-        double error;
-        gk_scan_wave(L, count, value, error, split, lane);
-        if (count >= tint || error <= epsrel * fabs(value)) break;
-        const double a = L.lo[split], b = L.hi[split], mid = (a + b) / 2.0;
-        if (lane < 42) {
-            const double x = lane < 21 ? gk_node(a, mid, lane) : gk_node(mid, b, lane - 21);
-            v[lane] = k1_theta_value<ANY>(P, Z, x, s, c, H, rows, rapidity);
-        }
-        wave_sync();
-        double e0, r0, e1, r1;
-        gk_halves_wave(a, mid, b, v, e0, r0, e1, r1, lane);
-        gk_insert_wave(L, count, split, mid, e0, r0, e1, r1, lane);
-        ++count;
+    for (int count = 1;; ++count) {
+        double value, error;
+        gk_totals(L, count, value, error);
+        if (count >= tint || error <= epsrel * fabs(value)) return value;
+        double a, b, half, est, err;
+        const int worst = gk_worst(L, count, a, b);
+        const double mid = (a + b) / 2.0;
+        const double theta = gk_half_node(g, a, mid, b, lane, half);
+        const double v = g.active ? k1_theta_value<ANY>(P, Z, sin2_quadrant(0.5 * theta), s, c, H, rows, rapidity) : 0.0;
+        gk_rule(g, half, v, est, err);
+        gk_split(L, worst, count, lane, a, mid, b, est, err);
         evals += 42;
     }
-    wave_sync();
-    return value;
 }
 
 // LDS of the adaptive K1 kernel (doubles): spline (R nodes + 4 (R - 1)
-// coefficients), J1 table, outer list (4 cap), outer nodes and values (2 x
-// 42), the first-pass values of the pending inner integrals (42 x 21), their
-// daughter terms (42 K1Z) and first-pass estimates and errors (2 x 42), then
-// per wave a list (4 cap) and 42 node values.
+// coefficients), J1 table, outer list (4 x 128), outer nodes and values (2 x
+// 42), the daughter terms of the pending inner integrals (42 K1Z), their
+// first-pass estimates and errors (2 x 42).
 constexpr int kK1ZWords = sizeof(K1Z) / sizeof(double);
 static_assert(sizeof(K1Z) == kK1ZWords * sizeof(double), "K1Z is a record of doubles");
-__host__ __device__ inline size_t k1a_lds_doubles(int R, int cap) {
-    return (size_t)R + 4 * (size_t)(R - 1) + kJ1Pieces * (kJ1Deg + 1) + 4 * (size_t)cap + 84 + 42 * 21 +
-           42 * kK1ZWords + 84 + (size_t)kK1aWaves * (4 * (size_t)cap + 42);
+__host__ __device__ inline size_t k1a_lds_doubles(int R) {
+    return (size_t)R + 4 * (size_t)(R - 1) + kJ1Pieces * (kJ1Deg + 1) + 4 * 128 + 84 + 42 * kK1ZWords + 84;
 }
 
 // Parent p of one evolution (arrays of that evolution).
@@ -585,9 +622,8 @@ template <bool ANY>
 __device__ __forceinline__ void k1_adaptive_body(int R, const double* __restrict__ r,
                                                  const double* __restrict__ N,
                                                  const double* __restrict__ t64, const BkConsts& c,
-                                                 const K1History& H, int rint, int tint, int cap,
-                                                 double epsrel, int p, double* __restrict__ k1,
-                                                 double* __restrict__ k1_err,
+                                                 const K1History& H, int rint, int tint, double epsrel, int p,
+                                                 double* __restrict__ k1, double* __restrict__ k1_err,
                                                  long long* __restrict__ k1_evals) {
     extern __shared__ double sh[];
     __shared__ int task_next, n_tasks, o_done, n_open;
@@ -602,27 +638,22 @@ __device__ __forceinline__ void k1_adaptive_body(int R, const double* __restrict
         return;
     }
     double* j1tab = sh + R + 4 * (R - 1);
-    double* o_base = j1tab + kJ1Pieces * (kJ1Deg + 1);
-    const GkList O{o_base, o_base + cap, o_base + 2 * cap, o_base + 3 * cap};
-    double* o_node = o_base + 4 * cap;  // 42 ln z nodes
-    double* o_val = o_node + 42;        // 42 outer integrand values
-    double* f_val = o_val + 42;         // 42 x 21 first-pass theta values
-    K1Z* z_tab = reinterpret_cast<K1Z*>(f_val + 42 * 21);  // daughter terms of the 42 nodes
-    double* f_est = f_val + 42 * 21 + 42 * kK1ZWords;       // first-pass estimates
-    double* f_err = f_est + 42;                              // and errors
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    double* w_base = f_err + 42 + (size_t)wave * (4 * cap + 42);
-    const GkList W{w_base, w_base + cap, w_base + 2 * cap, w_base + 3 * cap};
-    double* w_val = w_base + 4 * cap;
+    double* o_list = j1tab + kJ1Pieces * (kJ1Deg + 1);  // lower, upper, estimate, error: 128 each
+    double* o_node = o_list + 4 * 128;                  // 42 ln z nodes
+    double* o_val = o_node + 42;                        // 42 outer integrand values
+    K1Z* z_tab = reinterpret_cast<K1Z*>(o_val + 42);    // daughter terms of the 42 nodes
+    double* f_est = o_val + 42 + 42 * kK1ZWords;        // first-pass estimates
+    double* f_err = f_est + 42;                         // and errors
+    const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
+    const GkLane g = gk_lane(lane);
 
     for (int i = threadIdx.x; i < kJ1Pieces * (kJ1Deg + 1); i += blockDim.x) j1tab[i] = kJ1Cheb[i];
     LdsSpline<double> s;
     stage_spline<double>(t64, R, 0, sh, sh + R, s);
     const double a0 = t64[2], b0 = t64[2 + R - 1];  // ln r_0, ln r_{R-1}
+    if (threadIdx.x < 21) o_node[threadIdx.x] = (a0 + b0) / 2.0 + (b0 - a0) / 2.0 * g.x;
     if (threadIdx.x == 0) {
-        for (int k = 0; k < 21; ++k) o_node[k] = gk_node(a0, b0, k);
         n_tasks = 21;
-        task_next = 0;
         o_done = 0;
         ev_total = 0ull;
     }
@@ -639,39 +670,34 @@ __device__ __forceinline__ void k1_adaptive_body(int R, const double* __restrict
     P.j1tab = j1tab;
     const int rows = (ANY && H.rows) ? min(max(*H.rows, 1), H.capacity) : 0;
     const double rapidity = rows > 0 ? H.y[rows - 1] : 0.0;
+    // sin^2(theta / 2) at the lane's node of the rule on [0, pi]
+    const double s2_pi = sin2_quadrant(kPi / 4.0 + kPi / 4.0 * g.x);
 
-    int count = 0;  // outer intervals (wave 0 keeps the outer list; its lanes hold equal copies)
-    int split = 0;
-    double value = 0.0, error = 0.0;
-    long long evals = 0;
-    for (int step = 0; step < rint; ++step) {
+    double value = 0.0, error = 0.0;  // wave 0
+    int evals = 0;
+    for (int count = 0; count < rint; ++count) {  // outer intervals so far
         // the daughter terms of every pending inner integral, once
-        for (int t = threadIdx.x; t < n_tasks; t += blockDim.x) z_tab[t] = k1_daughter<ANY>(P, o_node[t], s, c);
-        if (threadIdx.x == 0) n_open = 0;
+        if (threadIdx.x < n_tasks) z_tab[threadIdx.x] = k1_daughter<ANY>(P, o_node[threadIdx.x], s, c);
+        if (threadIdx.x == 0) task_next = n_open = 0;
         __syncthreads();
-        // first pass on [0, pi] of every pending inner integral, over the
-        // whole block (n_tasks x 21 theta nodes)
-        for (int i = threadIdx.x; i < n_tasks * 21; i += blockDim.x) {
-            const int t = i / 21, k = i - 21 * t;
-            const K1Z Z = z_tab[t];
-            f_val[i] = k1_theta_value<ANY>(P, Z, gk_node(0.0, kPi, k), s, c, H, rows, rapidity);
-        }
-        __syncthreads();
-        // the rule on [0, pi] of every pending inner integral, one thread each;
-        // an integral that meets its tolerance there (the first test of
-        // k1_theta_adaptive, on the list's sums 0 + e and 0 + r) is done, the
-        // others go to the bisections
-        for (int t = threadIdx.x; t < n_tasks; t += blockDim.x) {
-            double e, r;
-            gk_from_values(0.0, kPi, f_val + 21 * t, e, r);
-            const double value = 0.0 + e, err = 0.0 + r;
-            if (1 >= tint || err <= epsrel * fabs(value)) {
-                o_val[t] = value * exp(2.0 * o_node[t]) * 2.0;
-                atomicAdd(&ev_total, 21ull);
-            } else {
-                f_est[t] = e;
-                f_err[t] = r;
-                open_task[atomicAdd(&n_open, 1)] = t;
+        // the rule on [0, pi] of every pending inner integral, one per
+        // half-wave; an integral that meets its tolerance there (the first test
+        // of k1_theta_adaptive) is done, the others go to the bisections
+        for (int pair = wave; 2 * pair < n_tasks; pair += kK1aWaves<ANY>) {
+            const int t = 2 * pair + (lane >> 5);
+            const bool on = t < n_tasks;
+            double v = 0.0, e, r;
+            if (on && g.active) v = k1_theta_value<ANY>(P, z_tab[t], s2_pi, s, c, H, rows, rapidity);
+            gk_rule(g, kPi / 2.0, v, e, r);
+            if (on && (lane & 31) == 0) {
+                if (1 >= tint || r <= epsrel * fabs(e)) {
+                    o_val[t] = e * exp(2.0 * o_node[t]) * 2.0;
+                    atomicAdd(&ev_total, 21ull);
+                } else {
+                    f_est[t] = e;
+                    f_err[t] = r;
+                    open_task[atomicAdd(&n_open, 1)] = t;
+                }
             }
         }
         __syncthreads();
@@ -679,48 +705,52 @@ __device__ __forceinline__ void k1_adaptive_body(int R, const double* __restrict
         for (;;) {
             int t = 0;
             if (lane == 0) t = atomicAdd(&task_next, 1);
-            t = __shfl(t, 0, 64);
+            t = uniform(t);
             if (t >= n_open) break;
-            t = open_task[t];
-            const double lz = o_node[t];
+            t = uniform(open_task[t]);
             const K1Z Z = z_tab[t];
-            const double inner = k1_theta_adaptive<ANY>(P, Z, f_est[t], f_err[t], s, c, H, rows, rapidity,
-                                                        tint, epsrel, W, w_val, lane, evals);
-            if (lane == 0) o_val[t] = inner * exp(2.0 * lz) * 2.0;
+            const double inner = k1_theta_adaptive<ANY>(P, Z, f_est[t], f_err[t], s, c, H, rows, rapidity, tint,
+                                                        epsrel, g, lane, evals);
+            if (lane == 0) o_val[t] = inner * exp(2.0 * o_node[t]) * 2.0;
         }
         __syncthreads();
         if (wave == 0) {
+            // the outer list's step: the rule from the nodes' values, the
+            // split, the totals, the next interval
+            GkList O;
+            double a = a0, b = b0, mid = 0.0, half, est, err;
+            const int k = lane < 21 ? lane : (lane >= 32 && lane < 53 ? lane - 32 + 21 : 0);
             if (count == 0) {
-                double e, rr;
-                gk_from_values(a0, b0, o_val, e, rr);
-                if (lane == 0) {
-                    O.lo[0] = a0;
-                    O.hi[0] = b0;
-                    O.est[0] = e;
-                    O.err[0] = rr;
-                }
-                count = 1;
+                gk_rule(g, (b0 - a0) / 2.0, lane < 32 && g.active ? o_val[k] : 0.0, est, err);
+                gk_start(O, lane, a0, b0, read_lane(est, 0), read_lane(err, 0));
             } else {
-                const double a = O.lo[split], b = O.hi[split], mid = (a + b) / 2.0;
-                double e0, r0, e1, r1;
-                gk_halves_wave(a, mid, b, o_val, e0, r0, e1, r1, lane);
-                gk_insert_wave(O, count, split, mid, e0, r0, e1, r1, lane);
-                ++count;
+                for (int q = 0; q < 2; ++q) {
+                    O.lo[q] = o_list[lane + 64 * q];
+                    O.hi[q] = o_list[128 + lane + 64 * q];
+                    O.est[q] = o_list[256 + lane + 64 * q];
+                    O.err[q] = o_list[384 + lane + 64 * q];
+                }
+                const int worst = gk_worst(O, count, a, b);
+                mid = (a + b) / 2.0;
+                (void)gk_half_node(g, a, mid, b, lane, half);
+                gk_rule(g, half, g.active ? o_val[k] : 0.0, est, err);
+                gk_split(O, worst, count, lane, a, mid, b, est, err);
             }
-            wave_sync();
-            gk_scan_wave(O, count, value, error, split, lane);
-            if (count >= rint || error <= epsrel * fabs(value)) {
+            gk_totals(O, count + 1, value, error);
+            if (count + 1 >= rint || error <= epsrel * fabs(value)) {
                 if (lane == 0) o_done = 1;
             } else {
-                const double a = O.lo[split], b = O.hi[split], mid = (a + b) / 2.0;
-                if (lane < 21) {
-                    o_node[lane] = gk_node(a, mid, lane);
-                    o_node[21 + lane] = gk_node(mid, b, lane);
+                gk_worst(O, count + 1, a, b);
+                mid = (a + b) / 2.0;
+                const double node = gk_half_node(g, a, mid, b, lane, half);
+                if (g.active) o_node[k] = node;
+                for (int q = 0; q < 2; ++q) {
+                    o_list[lane + 64 * q] = O.lo[q];
+                    o_list[128 + lane + 64 * q] = O.hi[q];
+                    o_list[256 + lane + 64 * q] = O.est[q];
+                    o_list[384 + lane + 64 * q] = O.err[q];
                 }
-                if (lane == 0) {
-                    n_tasks = 42;
-                    task_next = 0;
-                }
+                if (lane == 0) n_tasks = 42;
             }
         }
         __syncthreads();
@@ -736,12 +766,12 @@ __device__ __forceinline__ void k1_adaptive_body(int R, const double* __restrict
 }
 
 template <bool ANY>
-__global__ void __launch_bounds__(kK1aWaves * 64)
+__global__ void __launch_bounds__(kK1aWaves<ANY> * 64)
     k1_adaptive_kernel(int R, const double* __restrict__ r, const double* __restrict__ N,
                        const double* __restrict__ t64, BkConsts c, K1History H, int rint, int tint,
-                       int cap, double epsrel, double* __restrict__ k1, double* __restrict__ k1_err,
+                       double epsrel, double* __restrict__ k1, double* __restrict__ k1_err,
                        long long* __restrict__ k1_evals) {
-    k1_adaptive_body<ANY>(R, r, N, t64, c, H, rint, tint, cap, epsrel, blockIdx.x, k1, k1_err, k1_evals);
+    k1_adaptive_body<ANY>(R, r, N, t64, c, H, rint, tint, epsrel, blockIdx.x, k1, k1_err, k1_evals);
 }
 
 // ------------------------------------------------------------- K2 + Kf
@@ -1320,15 +1350,15 @@ __global__ void __launch_bounds__(kK1Threads) k1_batch_kernel(const BatchRun* __
 
 // The adaptive rule, one block per node of every run.
 template <bool ANY>
-__global__ void __launch_bounds__(kK1aWaves * 64)
+__global__ void __launch_bounds__(kK1aWaves<ANY> * 64)
     k1_adaptive_batch_kernel(const BatchRun* __restrict__ runs, const int32_t* __restrict__ node_run,
                              const double* __restrict__ r, const double* __restrict__ N,
-                             const double* __restrict__ t64, BkConsts c, int rint, int tint, int cap,
+                             const double* __restrict__ t64, BkConsts c, int rint, int tint,
                              double epsrel, double* __restrict__ k1) {
     const BatchRun run = runs[node_run[blockIdx.x]];
     const K1History H{};
     k1_adaptive_body<ANY>(run.R, r + run.node_off, N + run.node_off, t64 + run.spline_off, c, H, rint,
-                          tint, cap, epsrel, blockIdx.x - run.node_off, k1 + run.node_off, nullptr,
+                          tint, epsrel, blockIdx.x - run.node_off, k1 + run.node_off, nullptr,
                           nullptr);
 }
 
@@ -1518,24 +1548,22 @@ int launch_k1(int R, const double* r, const double* N, const double* t64, const 
 int launch_k1_adaptive(int R, const double* r, const double* N, const double* t64, const BkConsts& c,
                        int rint, int tint, double epsrel, double* k1, double* k1_err,
                        long long* k1_evals, hipStream_t stream, const K1History* hist) {
-    const int cap = rint > tint ? rint : tint;
-    const size_t smem = k1a_lds_doubles(R, cap) * sizeof(double);
+    const size_t smem = k1a_lds_doubles(R) * sizeof(double);
     int rc = init_kernel_attributes();
     if (rc != NLO_OK) return rc;
     int dev = 0, max_lds = 0;
     NLO_HIP_CHECK(hipGetDevice(&dev));
     NLO_HIP_CHECK(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
     NLO_REQUIRE(smem + 64 <= (size_t)max_lds,
-                "adaptive K1: R=%d with %d intervals needs %zu bytes of LDS (device: %d)", R, cap, smem,
-                max_lds);
+                "adaptive K1: R=%d needs %zu bytes of LDS (device: %d)", R, smem, max_lds);
     K1History H{};
     if (hist) H = *hist;
     if (c.production && !hist)
-        hipLaunchKernelGGL(k1_adaptive_kernel<false>, dim3(R), dim3(kK1aWaves * 64), smem, stream, R, r,
-                           N, t64, c, H, rint, tint, cap, epsrel, k1, k1_err, k1_evals);
+        hipLaunchKernelGGL(k1_adaptive_kernel<false>, dim3(R), dim3(kK1aWaves<false> * 64), smem, stream, R, r,
+                           N, t64, c, H, rint, tint, epsrel, k1, k1_err, k1_evals);
     else
-        hipLaunchKernelGGL(k1_adaptive_kernel<true>, dim3(R), dim3(kK1aWaves * 64), smem, stream, R, r,
-                           N, t64, c, H, rint, tint, cap, epsrel, k1, k1_err, k1_evals);
+        hipLaunchKernelGGL(k1_adaptive_kernel<true>, dim3(R), dim3(kK1aWaves<true> * 64), smem, stream, R, r,
+                           N, t64, c, H, rint, tint, epsrel, k1, k1_err, k1_evals);
     NLO_LAUNCH_CHECK();
     return NLO_OK;
 }
@@ -1691,22 +1719,20 @@ int launch_k1_batch(const BatchView& b, const double* r, const double* N, const 
 int launch_k1_adaptive_batch(const BatchView& b, const double* r, const double* N, const double* t64,
                              const BkConsts& c, int rint, int tint, double epsrel, double* k1,
                              hipStream_t stream) {
-    const int cap = rint > tint ? rint : tint;
-    const size_t smem = k1a_lds_doubles(b.Rmax, cap) * sizeof(double);
+    const size_t smem = k1a_lds_doubles(b.Rmax) * sizeof(double);
     int rc = init_kernel_attributes();
     if (rc != NLO_OK) return rc;
     int dev = 0, max_lds = 0;
     NLO_HIP_CHECK(hipGetDevice(&dev));
     NLO_HIP_CHECK(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
     NLO_REQUIRE(smem + 64 <= (size_t)max_lds,
-                "adaptive K1: R=%d with %d intervals needs %zu bytes of LDS (device: %d)", b.Rmax, cap,
-                smem, max_lds);
+                "adaptive K1: R=%d needs %zu bytes of LDS (device: %d)", b.Rmax, smem, max_lds);
     if (c.production)
-        hipLaunchKernelGGL(k1_adaptive_batch_kernel<false>, dim3(b.nodes), dim3(kK1aWaves * 64), smem,
-                           stream, b.runs_d, b.node_run, r, N, t64, c, rint, tint, cap, epsrel, k1);
+        hipLaunchKernelGGL(k1_adaptive_batch_kernel<false>, dim3(b.nodes), dim3(kK1aWaves<false> * 64), smem,
+                           stream, b.runs_d, b.node_run, r, N, t64, c, rint, tint, epsrel, k1);
     else
-        hipLaunchKernelGGL(k1_adaptive_batch_kernel<true>, dim3(b.nodes), dim3(kK1aWaves * 64), smem,
-                           stream, b.runs_d, b.node_run, r, N, t64, c, rint, tint, cap, epsrel, k1);
+        hipLaunchKernelGGL(k1_adaptive_batch_kernel<true>, dim3(b.nodes), dim3(kK1aWaves<true> * 64), smem,
+                           stream, b.runs_d, b.node_run, r, N, t64, c, rint, tint, epsrel, k1);
     NLO_LAUNCH_CHECK();
     return NLO_OK;
 }

@@ -99,6 +99,27 @@ def test_k1_adaptive_interval_limits_and_tolerance(dev):
         _compare(dev, BKConfig(MINR=1e-6, **kw), O.params(minr=1e-6), r, N)
 
 
+@pytest.mark.parametrize("rint,tint", [(1, 1), (1, 65), (2, 100), (64, 2), (100, 1)])
+def test_k1_adaptive_runs_to_the_interval_limits(dev, rint, tint):
+    """A tolerance that no integral meets: every list grows to its limit, over
+    one and two entries per lane, and the evaluations are exactly those of the
+    limits (21 nodes at first, 42 for each bisection, at both levels).  K1
+    within the bounds of _compare (equal evaluations, so the 1e-10 one)."""
+
+    from nlo_bk_optimized_amd.bk.config import BKConfig
+
+    print(f"adaptive K1 to the limits {rint} {tint}", flush=True)
+    r, N = workload(R=8)
+    cfg = BKConfig(MINR=1e-6, RINTPOINTS=rint, THETAINTPOINTS=tint, INTACCURACY=1e-30)
+    _compare(dev, cfg, O.params(minr=1e-6), r, N)
+    t64, _ = dev.spline_build(cuda(r), cuda(N))
+    stats = {}
+    dev.bk_k1(cuda(r), cuda(N), t64, cfg, rule="adaptive", stats=stats)
+    active = (np.arange(r.size) >= 1) & (N <= 0.99999)
+    count = (21 + 42 * (rint - 1)) * (21 + 42 * (tint - 1))
+    assert np.array_equal(stats["evaluations"].cpu().numpy()[active], np.full(active.sum(), count))
+
+
 @pytest.mark.parametrize("name", ["parent_dls", "beuf_dls", "nf5_dls", "nf0_lo"])
 def test_k1_adaptive_other_physics_matches_oracle(dev, name):
     print(f"adaptive K1 {name}", flush=True)
