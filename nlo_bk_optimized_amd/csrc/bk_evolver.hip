@@ -23,6 +23,7 @@ struct nlo_bk_evolver {
     double* T;      // adaptive: two half steps
     double* ctl;    // adaptive: [0] step, [1] error ratio
     double* k1;
+    void* k1_ws;  // the adaptive rule's queue
     double* k2kf;
     double* sums;
     double* t64;
@@ -49,7 +50,7 @@ namespace nlo {
 namespace {
 
 struct EvolverLayout {
-    size_t N, Nst, K, F, Hs, T, ctl, k1, k2kf, sums, t64, t32, flag, rows, active, nlo_ws,
+    size_t N, Nst, K, F, Hs, T, ctl, k1, k2kf, sums, t64, t32, flag, rows, active, k1_ws, nlo_ws,
         nlo_ws_bytes, total;
 };
 
@@ -77,6 +78,7 @@ EvolverLayout evolver_layout(const nlo_bk_evolver_desc& d) {
     L.flag = take(sizeof(int32_t));
     L.rows = take(sizeof(int32_t));
     L.active = take(sizeof(unsigned long long));
+    L.k1_ws = take(d.k1_rule == NLO_K1_ADAPTIVE ? k1_queue_workspace(d.R) : 1);
     L.nlo_ws_bytes = d.nlo ? nlo_plan(d.R, d.bins, d.n_samples, false).workspace : 0;
     L.nlo_ws = take(L.nlo_ws_bytes > 0 ? L.nlo_ws_bytes : 1);
     L.total = o;
@@ -206,8 +208,8 @@ int enqueue_rhs(nlo_bk_evolver* ev, const double* in, double* out, hipStream_t s
     if (rc != NLO_OK) return rc;
     K1History H{d.d_history_y, d.d_history_N, ev->r, ev->rows, R, d.history_capacity};
     if (d.k1_rule == NLO_K1_ADAPTIVE)
-        rc = launch_k1_adaptive(R, ev->r, in, ev->t64, ev->c, d.k1_rint, d.k1_tint, d.k1_epsrel, ev->k1,
-                                nullptr, nullptr, s, d.kinematical ? &H : nullptr);
+        rc = launch_k1_queue(R, ev->r, in, ev->t64, ev->c, d.k1_rint, d.k1_tint, d.k1_epsrel, ev->k1, ev->k1_ws,
+                             ev->flag, s, d.kinematical ? &H : nullptr);
     else
         rc = launch_k1(R, ev->r, in, ev->t64, ev->c, d.nr, d.nt, ev->k1, s, d.kinematical ? &H : nullptr);
     if (rc != NLO_OK) return rc;
@@ -443,6 +445,7 @@ int nlo_bk_evolver_create(const nlo_bk_evolver_desc* desc, const double* d_r, co
     ev->flag = reinterpret_cast<int32_t*>(w + L.flag);
     ev->rows = reinterpret_cast<int32_t*>(w + L.rows);
     ev->active = reinterpret_cast<unsigned long long*>(w + L.active);
+    ev->k1_ws = w + L.k1_ws;
     ev->nlo_ws = w + L.nlo_ws;
     ev->nlo_ws_bytes = L.nlo_ws_bytes;
     ev->y = 0.0;

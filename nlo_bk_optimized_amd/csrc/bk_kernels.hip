@@ -243,6 +243,23 @@ struct GaussRule {
 // whose sin^2(theta/2) and weights sit in LDS.
 constexpr int kK1Threads = 1024;
 
+// The terms of K1 that a parent's integrals share.
+template <bool ANY>
+__device__ __forceinline__ K1Parent k1_parent(double r, const LdsSpline<double>& s, double r_min, double r_max,
+                                              const BkConsts& c, const double* j1tab) {
+    K1Parent P;
+    P.r = r;
+    P.log_r = log(P.r);
+    P.n_r = fmin(loglog64(s, r_min, r_max, P.r, 0.0, 1.0), 1.0);
+    P.a_r = ANY ? 0.0 : alpha_s64(P.r, c);
+    P.lo_coef = c.nc / (2.0 * kPi * kPi) * P.a_r;
+    P.fin_coef = P.a_r * c.nc / (4.0 * kPi) * (67.0 / 9.0 - kPi * kPi / 3.0 - 10.0 / 9.0 * c.nf / c.nc);
+    P.log_ksub = log(c.ksub);
+    P.resum_on = P.r > 1.01 * c.minr ? 1.0 : 0.0;
+    P.j1tab = j1tab;
+    return P;
+}
+
 // ANY = false: the production physics with the hoisted per-z-node terms;
 // ANY = true: every coupling / order choice and the kinematical constraint
 // (H.rows set), the full Kernel_lo per theta node.
@@ -274,16 +291,7 @@ __device__ __forceinline__ void k1_body(int R, const double* __restrict__ r, con
     }
     __syncthreads();
     const double r_min = t64[0], r_max = t64[1];
-    K1Parent P;
-    P.r = r[p];
-    P.log_r = log(P.r);
-    P.n_r = fmin(loglog64(s, r_min, r_max, P.r, 0.0, 1.0), 1.0);
-    P.a_r = ANY ? 0.0 : alpha_s64(P.r, c);
-    P.lo_coef = c.nc / (2.0 * kPi * kPi) * P.a_r;
-    P.fin_coef = P.a_r * c.nc / (4.0 * kPi) * (67.0 / 9.0 - kPi * kPi / 3.0 - 10.0 / 9.0 * c.nf / c.nc);
-    P.log_ksub = log(c.ksub);
-    P.resum_on = P.r > 1.01 * c.minr ? 1.0 : 0.0;
-    P.j1tab = j1tab;
+    const K1Parent P = k1_parent<ANY>(r[p], s, r_min, r_max, c, j1tab);
     const int znodes = (R - 1) * g.nr;
     // kinematical constraint: history rows and the current rapidity (last row)
     const int rows = (ANY && H.rows) ? min(max(*H.rows, 1), H.capacity) : 0;
@@ -607,6 +615,29 @@ __device__ __forceinline__ double k1_theta_adaptive(const K1Parent& P, const K1Z
     }
 }
 
+// The outer list's step: from the values v of the nodes (lane's entry
+// gk_outer_index) the rule on [lo, hi] (count 0) or on the halves of the worst
+// of `count` intervals, its split, and the totals.
+__device__ __forceinline__ int gk_outer_index(int lane) {
+    return lane < 21 ? lane : (lane >= 32 && lane < 53 ? lane - 32 + 21 : 0);
+}
+__device__ __forceinline__ void gk_outer_step(GkList& O, const GkLane& g, int count, int lane, double lo, double hi,
+                                              double v, double& value, double& error) {
+    double est, err;
+    if (count == 0) {
+        gk_rule(g, (hi - lo) / 2.0, lane < 32 ? v : 0.0, est, err);
+        gk_start(O, lane, lo, hi, read_lane(est, 0), read_lane(err, 0));
+    } else {
+        double a, b, half;
+        const int worst = gk_worst(O, count, a, b);
+        const double mid = (a + b) / 2.0;
+        (void)gk_half_node(g, a, mid, b, lane, half);
+        gk_rule(g, half, v, est, err);
+        gk_split(O, worst, count, lane, a, mid, b, est, err);
+    }
+    gk_totals(O, count + 1, value, error);
+}
+
 // LDS of the adaptive K1 kernel (doubles): spline (R nodes + 4 (R - 1)
 // coefficients), J1 table, outer list (4 x 128), outer nodes and values (2 x
 // 42), the daughter terms of the pending inner integrals (42 K1Z), their
@@ -658,16 +689,7 @@ __device__ __forceinline__ void k1_adaptive_body(int R, const double* __restrict
         ev_total = 0ull;
     }
     __syncthreads();
-    K1Parent P;
-    P.r = r[p];
-    P.log_r = log(P.r);
-    P.n_r = fmin(loglog64(s, t64[0], t64[1], P.r, 0.0, 1.0), 1.0);
-    P.a_r = ANY ? 0.0 : alpha_s64(P.r, c);
-    P.lo_coef = c.nc / (2.0 * kPi * kPi) * P.a_r;
-    P.fin_coef = P.a_r * c.nc / (4.0 * kPi) * (67.0 / 9.0 - kPi * kPi / 3.0 - 10.0 / 9.0 * c.nf / c.nc);
-    P.log_ksub = log(c.ksub);
-    P.resum_on = P.r > 1.01 * c.minr ? 1.0 : 0.0;
-    P.j1tab = j1tab;
+    const K1Parent P = k1_parent<ANY>(r[p], s, t64[0], t64[1], c, j1tab);
     const int rows = (ANY && H.rows) ? min(max(*H.rows, 1), H.capacity) : 0;
     const double rapidity = rows > 0 ? H.y[rows - 1] : 0.0;
     // sin^2(theta / 2) at the lane's node of the rule on [0, pi]
@@ -715,34 +737,22 @@ __device__ __forceinline__ void k1_adaptive_body(int R, const double* __restrict
         }
         __syncthreads();
         if (wave == 0) {
-            // the outer list's step: the rule from the nodes' values, the
-            // split, the totals, the next interval
             GkList O;
-            double a = a0, b = b0, mid = 0.0, half, est, err;
-            const int k = lane < 21 ? lane : (lane >= 32 && lane < 53 ? lane - 32 + 21 : 0);
-            if (count == 0) {
-                gk_rule(g, (b0 - a0) / 2.0, lane < 32 && g.active ? o_val[k] : 0.0, est, err);
-                gk_start(O, lane, a0, b0, read_lane(est, 0), read_lane(err, 0));
-            } else {
+            double a, b, half;
+            const int k = gk_outer_index(lane);
+            if (count > 0)
                 for (int q = 0; q < 2; ++q) {
                     O.lo[q] = o_list[lane + 64 * q];
                     O.hi[q] = o_list[128 + lane + 64 * q];
                     O.est[q] = o_list[256 + lane + 64 * q];
                     O.err[q] = o_list[384 + lane + 64 * q];
                 }
-                const int worst = gk_worst(O, count, a, b);
-                mid = (a + b) / 2.0;
-                (void)gk_half_node(g, a, mid, b, lane, half);
-                gk_rule(g, half, g.active ? o_val[k] : 0.0, est, err);
-                gk_split(O, worst, count, lane, a, mid, b, est, err);
-            }
-            gk_totals(O, count + 1, value, error);
+            gk_outer_step(O, g, count, lane, a0, b0, o_val[k], value, error);
             if (count + 1 >= rint || error <= epsrel * fabs(value)) {
                 if (lane == 0) o_done = 1;
             } else {
                 gk_worst(O, count + 1, a, b);
-                mid = (a + b) / 2.0;
-                const double node = gk_half_node(g, a, mid, b, lane, half);
+                const double node = gk_half_node(g, a, (a + b) / 2.0, b, lane, half);
                 if (g.active) o_node[k] = node;
                 for (int q = 0; q < 2; ++q) {
                     o_list[lane + 64 * q] = O.lo[q];
@@ -772,6 +782,259 @@ __global__ void __launch_bounds__(kK1aWaves<ANY> * 64)
                        double epsrel, double* __restrict__ k1, double* __restrict__ k1_err,
                        long long* __restrict__ k1_evals) {
     k1_adaptive_body<ANY>(R, r, N, t64, c, H, rint, tint, epsrel, blockIdx.x, k1, k1_err, k1_evals);
+}
+
+// ---- the same rule with the inner integrals of all parents in one queue
+//
+// The evaluations of a parent spread over a factor of 6 about their mean, and
+// a block per parent leaves the rest of the chip idle while the heaviest one
+// ends (256 nodes: 16963 bisections in the heaviest parent, 2340 on average,
+// and at most 657 of them in sequence).  Here every wave of the chip takes
+// inner integrals, of any parent, from one queue in global memory.  The wave
+// that ends the last pending integral of a parent does the parent's outer
+// step and queues the 42 integrals of the next one.  Every sum has the order
+// of the kernel above, whichever wave took what.
+//
+// The queue is a ring of tasks: a wave draws a ticket from `head` and waits
+// for the entry of its ticket, which carries the ticket's lap of the ring; a
+// step draws 42 entries from `tail`.  A reader leaves its entry empty for the
+// next lap, and a writer waits for that.  At most 42 tasks per parent are
+// pending and the ring holds at least as many, so the ticket one lap before a
+// writer's has been drawn, by a wave that runs, and its writer runs too.  The wave that ends the last parent queues one
+// end mark per wave of the launch; every wave has drawn one ticket more than
+// it had tasks, so each finds one mark and leaves.  No wave waits for one that
+// has not started: blocks that the chip has no room for start late, find their
+// end marks and leave.  What waves share goes through atomics at the scope of
+// the device.
+//
+// There are kK1Rings such rings, parent p in ring p % kK1Rings: tickets of one
+// ring are atomics on one address.  A wave starts at the ring of its block,
+// goes on to the next ring with each end mark that it finds, and leaves after
+// the last.
+//
+// Bound by the sequence of the heaviest parent and by what a step costs
+// besides: one RHS on 64 / 256 / 400 nodes (epsrel 1e-3) takes 1.57 / 1.96 /
+// 2.36 ms, a block per parent 2.72 / 3.35 / 4.54 ms.  One ring takes 1.77 /
+// 2.60 / 3.39 ms, eight 1.61 / 1.92 / 2.45 ms.  Release and acquire fences,
+// which write back and drop the caches, in place of q_settle made it 2.09 /
+// 4.28 / 6.09 ms (one ring).
+constexpr int kK1Rings = 4;
+struct K1Queue {
+    unsigned* ctl;      // ring by ring: head, tail, open parents, kK1QueueCtl words apart
+    unsigned* ring;     // kK1Rings x 2^bits: lap << 18 | (64 parent + integral + 1; 0: empty)
+    int bits;
+    K1Parent* parents;  // R
+    double* state;      // R x kK1QueueState: outer list (4 x 128), 42 ln z nodes, 42 values
+    int* pending;       // R: inner integrals that have not ended
+    int* count;         // R: outer intervals
+    int* flag;          // set when a wait ran out of its limit
+};
+constexpr int kK1QueueCtl = 32;
+constexpr int kK1QueueState = 4 * 128 + 84;
+constexpr int kK1QueueWaves = 4096;     // most waves of a launch
+constexpr unsigned kK1QueueEnd = (1u << 18) - 1u;
+static_assert(64 * kMaxR < (int)kK1QueueEnd, "a task fits below the lap");
+// laps: at most kMaxGkIntervals rings of tasks and one of end marks
+static_assert(kMaxGkIntervals + 2 < 1 << 14, "a lap fits above the task");
+// Bound of one wait in ticks of the 100 MHz clock (20 s).  A wait ends when a
+// running task does (at most kMaxGkIntervals bisections), so it is never met.
+constexpr long long kK1QueueTicks = 2000000000ll;
+
+template <typename T>
+__device__ __forceinline__ T q_load(const T* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void q_store(T* p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ T q_add(T* p, T v) {
+    return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ unsigned* k1_queue_entry(const K1Queue& q, int ring, unsigned ticket, unsigned& lap) {
+    lap = (ticket >> q.bits) << 18;
+    return q.ring + ((unsigned)ring << q.bits) + (ticket & ((1u << q.bits) - 1u));
+}
+
+// Orders what a wave shares: every access before it has reached the memory
+// that all XCDs see (stores at device scope are written through and
+// acknowledged there) before any after it is issued; loads at device scope
+// pass by the caches, so no cache is written back or dropped.
+__device__ __forceinline__ void q_settle() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
+
+// Writes an entry of the ring when the reader of the lap before has emptied it.
+__device__ __forceinline__ void k1_queue_put(const K1Queue& q, int ring, unsigned ticket, unsigned task) {
+    unsigned lap;
+    unsigned* e = k1_queue_entry(q, ring, ticket, lap);
+    const long long t0 = wall_clock64();
+    while (q_load(e) != lap) {
+        if (wall_clock64() - t0 > kK1QueueTicks) {
+            q_store(q.flag, 1);
+            return;
+        }
+        __builtin_amdgcn_s_sleep(1);
+    }
+    q_store(e, lap | task);
+}
+
+// The first integrals of every active parent; one block.
+template <bool ANY>
+__global__ void __launch_bounds__(1024)
+    k1_queue_init_kernel(int R, const double* __restrict__ r, const double* __restrict__ N,
+                         const double* __restrict__ t64, BkConsts c, K1Queue q, int waves,
+                         double* __restrict__ k1) {
+    extern __shared__ double sh[];
+    __shared__ int open[kK1Rings];
+    LdsSpline<double> s;
+    stage_spline<double>(t64, R, 0, sh, sh + R, s);
+    if (threadIdx.x < kK1Rings) open[threadIdx.x] = 0;
+    for (unsigned i = threadIdx.x; i < (unsigned)kK1Rings << q.bits; i += blockDim.x) q.ring[i] = 0u;
+    __syncthreads();
+    const double a0 = t64[2], b0 = t64[2 + R - 1];
+    for (int p = threadIdx.x; p < R; p += blockDim.x) {
+        k1[p] = 0.0;
+        if (p == 0 || !(N[p] <= 0.99999)) continue;  // reference active set: index >= 1, N <= 0.99999
+        q.parents[p] = k1_parent<ANY>(r[p], s, t64[0], t64[1], c, nullptr);
+        q.pending[p] = 21;
+        q.count[p] = 0;
+        unsigned* at = q.ring + ((unsigned)(p % kK1Rings) << q.bits) + 21 * atomicAdd(&open[p % kK1Rings], 1);
+        double* node = q.state + (size_t)p * kK1QueueState + 4 * 128;
+        for (int k = 0; k < 21; ++k) {
+            node[k] = (a0 + b0) / 2.0 + (b0 - a0) / 2.0 * gk_lane(k).x;
+            at[k] = 64u * p + k + 1u;
+        }
+    }
+    __syncthreads();
+    for (int k = 0; k < kK1Rings; ++k)
+        if (open[k] == 0)  // no parent: the end marks
+            for (int i = threadIdx.x; i < waves; i += blockDim.x) q.ring[((unsigned)k << q.bits) + i] = kK1QueueEnd;
+    if (threadIdx.x < kK1Rings) {
+        unsigned* ctl = q.ctl + threadIdx.x * 3 * kK1QueueCtl;
+        ctl[0] = 0u;
+        ctl[kK1QueueCtl] = 21u * open[threadIdx.x];
+        ctl[2 * kK1QueueCtl] = open[threadIdx.x];
+    }
+}
+
+// LDS (doubles): spline (R nodes + 4 (R - 1) coefficients), J1 table.
+__host__ __device__ inline size_t k1_queue_lds_doubles(int R) {
+    return (size_t)R + 4 * (size_t)(R - 1) + kJ1Pieces * (kJ1Deg + 1);
+}
+
+template <bool ANY>
+__global__ void __launch_bounds__(kK1aWaves<ANY> * 64)
+    k1_queue_kernel(int R, const double* __restrict__ t64, BkConsts c, K1History H, int rint, int tint,
+                    double epsrel, K1Queue q, double* __restrict__ k1) {
+    extern __shared__ double sh[];
+    double* j1tab = sh + R + 4 * (R - 1);
+    const int lane = threadIdx.x & 63;
+    const GkLane g = gk_lane(lane);
+    for (int i = threadIdx.x; i < kJ1Pieces * (kJ1Deg + 1); i += blockDim.x) j1tab[i] = kJ1Cheb[i];
+    LdsSpline<double> s;
+    stage_spline<double>(t64, R, 0, sh, sh + R, s);
+    __syncthreads();
+    const double a0 = t64[2], b0 = t64[2 + R - 1];  // ln r_0, ln r_{R-1}
+    const int rows = (ANY && H.rows) ? min(max(*H.rows, 1), H.capacity) : 0;
+    const double rapidity = rows > 0 ? H.y[rows - 1] : 0.0;
+    // sin^2(theta / 2) at the lane's node of the rule on [0, pi]
+    const double s2_pi = sin2_quadrant(kPi / 4.0 + kPi / 4.0 * g.x);
+    for (int ring = blockIdx.x % kK1Rings, ended = 0; ended < kK1Rings;) {
+        unsigned* ctl = q.ctl + ring * 3 * kK1QueueCtl;
+        unsigned ticket = 0u;
+        if (lane == 0) ticket = q_add(ctl, 1u);
+        ticket = (unsigned)uniform((int)ticket);
+        unsigned lap, task;
+        unsigned* entry = k1_queue_entry(q, ring, ticket, lap);
+        const long long t0 = wall_clock64();
+        for (;;) {
+            task = (unsigned)uniform((int)q_load(entry)) - lap;
+            if (task - 1u < kK1QueueEnd) break;
+            if (wall_clock64() - t0 > kK1QueueTicks) {
+                q_store(q.flag, 1);
+                return;
+            }
+            __builtin_amdgcn_s_sleep(4);
+        }
+        q_settle();
+        if (lane == 0) q_store(entry, lap + (1u << 18));
+        if (task == kK1QueueEnd) {
+            ring = (ring + 1) % kK1Rings;
+            ++ended;
+            continue;
+        }
+        const int p = (int)((task - 1u) >> 6), t = (int)((task - 1u) & 63u);
+        K1Parent P = q.parents[p];
+        P.j1tab = j1tab;
+        double* list = q.state + (size_t)p * kK1QueueState;
+        double* node = list + 4 * 128;
+        double* val = node + 42;
+        {
+            const double log_z = q_load(node + t);
+            const K1Z Z = k1_daughter<ANY>(P, log_z, s, c);
+            double v = 0.0, e, err;
+            if (lane < 21) v = k1_theta_value<ANY>(P, Z, s2_pi, s, c, H, rows, rapidity);
+            gk_rule(g, kPi / 2.0, v, e, err);
+            e = read_lane(e, 0);
+            err = read_lane(err, 0);
+            int evals = 0;
+            if (!(1 >= tint || err <= epsrel * fabs(e)))
+                e = k1_theta_adaptive<ANY>(P, Z, e, err, s, c, H, rows, rapidity, tint, epsrel, g, lane, evals);
+            if (lane == 0) q_store(val + t, e * exp(2.0 * log_z) * 2.0);
+            q_settle();
+        }
+        int left = 0;
+        if (lane == 0) left = q_add(q.pending + p, -1);
+        q_settle();
+        if (uniform(left) != 1) continue;
+
+        // the parent's outer step
+        const int count = uniform(q_load(q.count + p)), k = gk_outer_index(lane);
+        GkList O;
+        double value, error, a, b, half;
+        if (count > 0)
+            for (int w = 0; w < 2; ++w) {
+                const bool on = lane + 64 * w < count;
+                O.lo[w] = on ? q_load(list + lane + 64 * w) : 0.0;
+                O.hi[w] = on ? q_load(list + 128 + lane + 64 * w) : 0.0;
+                O.est[w] = on ? q_load(list + 256 + lane + 64 * w) : 0.0;
+                O.err[w] = on ? q_load(list + 384 + lane + 64 * w) : 0.0;
+            }
+        gk_outer_step(O, g, count, lane, a0, b0, count > 0 || lane < 21 ? q_load(val + k) : 0.0, value, error);
+        unsigned at = 0u;
+        if (count + 1 >= rint || error <= epsrel * fabs(value)) {
+            unsigned open = 0u;
+            if (lane == 0) {
+                k1[p] = value;
+                open = q_add(ctl + 2 * kK1QueueCtl, ~0u);
+                if (open == 1u) at = q_load(ctl + kK1QueueCtl);
+            }
+            if (uniform((int)open) != 1) continue;
+            at = (unsigned)uniform((int)at);
+            const unsigned waves = gridDim.x * kK1aWaves<ANY>;
+            for (unsigned i = lane; i < waves; i += 64u) k1_queue_put(q, ring, at + i, kK1QueueEnd);
+        } else {
+            gk_worst(O, count + 1, a, b);
+            const double x = gk_half_node(g, a, (a + b) / 2.0, b, lane, half);
+            if (g.active) q_store(node + k, x);
+            for (int w = 0; w < 2; ++w)
+                if (lane + 64 * w < count + 1) {
+                    q_store(list + lane + 64 * w, O.lo[w]);
+                    q_store(list + 128 + lane + 64 * w, O.hi[w]);
+                    q_store(list + 256 + lane + 64 * w, O.est[w]);
+                    q_store(list + 384 + lane + 64 * w, O.err[w]);
+                }
+            if (lane == 0) {
+                q_store(q.pending + p, 42);
+                q_store(q.count + p, count + 1);
+                at = q_add(ctl + kK1QueueCtl, 42u);
+            }
+            at = (unsigned)uniform((int)at);
+            q_settle();
+            if (lane < 42) k1_queue_put(q, ring, at + lane, 64u * p + lane + 1u);
+        }
+    }
 }
 
 // ------------------------------------------------------------- K2 + Kf
@@ -1479,6 +1742,10 @@ int init_kernel_attributes() {
             (const void*)k1_kernel<true>,
             (const void*)k1_adaptive_kernel<false>,
             (const void*)k1_adaptive_kernel<true>,
+            (const void*)k1_queue_init_kernel<false>,
+            (const void*)k1_queue_init_kernel<true>,
+            (const void*)k1_queue_kernel<false>,
+            (const void*)k1_queue_kernel<true>,
             (const void*)spline_build_batch_kernel,
             (const void*)k1_batch_kernel<false>,
             (const void*)k1_batch_kernel<true>,
@@ -1541,6 +1808,68 @@ int launch_k1(int R, const double* r, const double* N, const double* t64, const 
     else
         hipLaunchKernelGGL(k1_kernel<true>, dim3(R), dim3(kK1Threads), smem, stream, R, r, N, t64, c, g,
                            H, k1);
+    NLO_LAUNCH_CHECK();
+    return NLO_OK;
+}
+
+// The queue of the adaptive rule: ring, parents, outer lists.  A power of two
+// of entries that holds every pending integral and every end mark.
+int k1_queue_bits(int R) {
+    int bits = 12;
+    static_assert(1 << 12 >= kK1QueueWaves, "an end mark per wave");
+    while (1 << bits < 42 * ((R + kK1Rings - 1) / kK1Rings)) ++bits;
+    return bits;
+}
+
+size_t k1_queue_workspace(int R) {
+    return align_up(kK1Rings * 3 * kK1QueueCtl * sizeof(unsigned), 256) + align_up((size_t)kK1Rings * 4 << k1_queue_bits(R), 256) +
+           align_up(R * sizeof(K1Parent), 256) + align_up((size_t)R * kK1QueueState * sizeof(double), 256) +
+           2 * align_up(R * sizeof(int), 256);
+}
+
+int launch_k1_queue(int R, const double* r, const double* N, const double* t64, const BkConsts& c, int rint,
+                    int tint, double epsrel, double* k1, void* workspace, int32_t* flag, hipStream_t stream,
+                    const K1History* hist) {
+    const size_t smem = k1_queue_lds_doubles(R) * sizeof(double);
+    int rc = init_kernel_attributes();
+    if (rc != NLO_OK) return rc;
+    int dev = 0, max_lds = 0, cus = 0;
+    NLO_HIP_CHECK(hipGetDevice(&dev));
+    NLO_HIP_CHECK(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+    NLO_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    NLO_REQUIRE(k1a_lds_doubles(R) * sizeof(double) + 64 <= (size_t)max_lds,
+                "adaptive K1: R=%d needs %zu bytes of LDS (device: %d)", R, smem, max_lds);
+    K1Queue q{};
+    char* w = static_cast<char*>(workspace);
+    auto take = [&w](size_t bytes) {
+        char* at = w;
+        w += align_up(bytes, 256);
+        return at;
+    };
+    q.ctl = reinterpret_cast<unsigned*>(take(kK1Rings * 3 * kK1QueueCtl * sizeof(unsigned)));
+    q.bits = k1_queue_bits(R);
+    q.ring = reinterpret_cast<unsigned*>(take((size_t)kK1Rings * 4 << q.bits));
+    q.parents = reinterpret_cast<K1Parent*>(take(R * sizeof(K1Parent)));
+    q.state = reinterpret_cast<double*>(take((size_t)R * kK1QueueState * sizeof(double)));
+    q.pending = reinterpret_cast<int*>(take(R * sizeof(int)));
+    q.count = reinterpret_cast<int*>(take(R * sizeof(int)));
+    q.flag = flag;
+    K1History H{};
+    if (hist) H = *hist;
+    auto launch = [&](auto any) {
+        constexpr bool kAny = decltype(any)::value;
+        constexpr int kWaves = kK1aWaves<kAny>;
+        // one block per CU, no more than the tasks that can be pending
+        const int grid = std::max(1, std::min({cus, (42 * (R - 1) + kWaves - 1) / kWaves, kK1QueueWaves / kWaves}));
+        hipLaunchKernelGGL(k1_queue_init_kernel<kAny>, dim3(1), dim3(1024), smem, stream, R, r, N, t64, c, q,
+                           grid * kWaves, k1);
+        hipLaunchKernelGGL(k1_queue_kernel<kAny>, dim3(grid), dim3(kWaves * 64), smem, stream, R, t64, c, H, rint,
+                           tint, epsrel, q, k1);
+    };
+    if (c.production && !hist)
+        launch(std::false_type{});
+    else
+        launch(std::true_type{});
     NLO_LAUNCH_CHECK();
     return NLO_OK;
 }

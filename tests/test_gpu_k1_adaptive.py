@@ -163,6 +163,59 @@ def test_evolver_adaptive_k1_step(dev):
     assert torch.allclose(got, want, rtol=1e-14, atol=1e-300)
 
 
+@pytest.mark.parametrize("R,active,limits,variant", [
+    (3, None, {}, None),
+    (3, 0, {}, None),  # no active parent: only the end marks
+    (24, 2, {"RINTPOINTS": 1, "THETAINTPOINTS": 1}, None),
+    (40, None, {"INTACCURACY": 1e-5}, None),
+    (30, None, {"RINTPOINTS": 100, "THETAINTPOINTS": 1, "INTACCURACY": 1e-30}, None),  # most laps of the ring
+    (150, None, {}, None),  # more first tasks than waves, a longer ring
+    (24, None, {"INTACCURACY": 1e-2}, "parent_dls"),
+])
+def test_evolver_queue_matches_the_block_kernel(dev, R, active, limits, variant):
+    """The evolver takes the inner integrals of all parents from one queue,
+    nlo_bk_k1_adaptive one block per parent: the same sums in the same order,
+    so K1 agrees to rounding (1e-10 as in _compare; 1e-12 of the largest K1
+    where a parent's cancels), and within the error estimate where a decision
+    at the tolerance went the other way.  Each of several steps (replays of one
+    graph) is compared; the queue's own results are the same bits every time,
+    whichever wave took what."""
+
+    from nlo_bk_optimized_amd.bk.config import BKConfig
+    from nlo_bk_optimized_amd.bk.evolution import prepare
+
+    print(f"queue R={R} active={active} {limits} {variant}", flush=True)
+    kw = dict(RPOINTS=R, MAXR=1e2, MCINTPOINTS=1 << 10, RK_METHOD="euler", DE_SOLVER_STEP=0.1,
+              K1_RULE="adaptive", **limits)
+    cfg = configs(variant, **kw)[0] if variant else BKConfig(MINR=1e-6, **kw)
+    setup = prepare(_mv(), cfg, device=torch.device("cuda"), seed=0)
+    N0 = setup.N0.clone()
+    if active is not None:
+        N0[1 + active:] = 1.0
+    ev = dev.Evolver(setup.r, setup.edges, setup.table, cfg, n_samples=setup.n_samples, precision="fp64",
+                     rk_method="euler", step=0.1, nlo=False, k1_rule="adaptive")
+    try:
+        ev.state.copy_(N0)
+        for _ in range(3):
+            state = ev.state.clone()
+            t64, _ = dev.spline_build(setup.r, state)
+            stats = {}
+            want = dev.bk_k1(setup.r, state, t64, cfg, rule="adaptive", stats=stats)
+            ev.step()
+            got = ev.k1.clone()
+            diff, floor = (got - want).abs(), 1e-12 * want.abs().max()
+            near = diff <= 1e-10 * want.abs() + floor
+            print(f"near for {int(near.sum())} of {near.numel()} parents", flush=True)
+            assert near.double().mean() >= 0.9
+            assert torch.all(near | (diff <= 2.0 * stats["error"] + floor))
+            after = ev.state.clone()
+            ev.state.copy_(state)
+            ev.step()
+            assert torch.equal(ev.k1, got) and torch.equal(ev.state, after)
+    finally:
+        ev.close()
+
+
 def _order(name):
     from nlo_bk_optimized_amd.bk.config import BKOrder
 
