@@ -15,6 +15,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "fp64_math.hpp"
+
 namespace nlo {
 
 #include "bessel_j1_i1_tables.inc"
@@ -35,10 +37,10 @@ __device__ constexpr double kI1Series[21] = {
 // Horner's rule.  For |s| <= 16 (2a <= 8) the tail is below 4e-18 of the
 // I1 sum; on the J1 side the alternating terms (at most ~23) leave an
 // absolute rounding error below 1e-14.
-__host__ __device__ inline __attribute__((noinline)) double j1_i1_series(double s) {
-    double sum = kI1Series[20];
+__host__ __device__ inline double j1_i1_series(double s) {
+    double sum = coef64(kI1Series[20]);
 #pragma unroll
-    for (int k = 19; k >= 0; --k) sum = fma(sum, s, kI1Series[k]);
+    for (int k = 19; k >= 0; --k) sum = fma(sum, s, coef64(kI1Series[k]));
     return sum;
 }
 

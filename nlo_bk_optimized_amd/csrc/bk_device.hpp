@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include "bessel_j1_i1.hpp"
+#include "fp64_math.hpp"
 #include "common.hpp"
 
 namespace nlo {
@@ -33,6 +34,7 @@ struct BkConsts {
     int production;     // Balitsky LO, smallest resummation, DLOG_SLOG, smooth coupling
     double fixed_as;
     double log_4c2;     // ln(4 C2)
+    double freeze;      // 2.5^2 Lambda^2 / (4 C2): the coupling freezes at d^2 = 1 / freeze
 };
 
 // -------------------------------------------------------------- coupling
@@ -194,7 +196,11 @@ template <typename T>
 __device__ __forceinline__ T loglog_from_log(const LdsSpline<T>& s, T log_d, T underflow,
                                             T overflow) {
     const T lv = fmin(fmax(log_d, s.log_min), s.log_max);
-    T out = exp(spline_poly(s, lv));
+    T out;
+    if constexpr (sizeof(T) == 8)
+        out = exp64(spline_poly(s, lv));
+    else
+        out = exp(spline_poly(s, lv));
     out = isfinite(out) ? out : T(0);
     out = log_d < s.log_min ? underflow : out;
     return log_d > s.log_max ? overflow : out;
@@ -214,16 +220,17 @@ __device__ __forceinline__ T loglog_from_log(const LdsSpline<T>& s, T log_d, T u
 // alpha(d) from ln d (S/coupling.py:81-97): ln(4 C2 / (d^2 Lambda^2)) =
 // log_scale0 - 2 ln d.  The denominator is returned too, so that ratios of
 // couplings need no division: alpha_a / alpha_b = alpha_a * den_b.
-// Far from the freezing scale (|mu0 - right| > 40) the smooth-max term
-// log1p(e^-|d|) < 4.3e-18 is below half an ulp of hi >= mu0 = 10 ln 2.5, so
-// hi + term rounds to hi: skipping the exp and log1p there changes no bit,
+// Far from the freezing scale (a factor above 1e18) the smooth-max term
+// log1p(e^-|mu0 - right|) < 1e-18 is below half an ulp of hi >= mu0 = 10 ln 2.5, so
+// hi + term rounds to hi: skipping it there changes no bit,
 // and whole waves (small distances) skip them.
-__device__ __forceinline__ double alpha_s64_den(double log_d, const BkConsts& c) {
+// e^(mu0 - right) is the fifth power of d^2 / (d^2 at the freezing), so the
+// smooth-max term needs no exponential.
+__device__ __forceinline__ double alpha_s64_den(double dsq, double log_d, const BkConsts& c) {
     const double right = (c.log_scale0 - 2.0 * log_d) * 5.0;  // / 0.2 within one rounding
-    const double hi = fmax(c.log_mu0, right);
-    const double d = fabs(c.log_mu0 - right);
-    double sum = hi;
-    if (!(d > 40.0)) sum = hi + log1p(exp(-d));  // NaN keeps the full formula
+    const double v = dsq * c.freeze, v2 = v * v, u = v2 * v2 * v;
+    double sum = fmax(c.log_mu0, right);
+    if (u > 1e-18 && u < 1e18) sum += log1p_fold64(u);
     return c.b0 * (0.2 * sum);
 }
 
@@ -245,17 +252,16 @@ __device__ __forceinline__ double k1_theta_term(const K1Parent& P, const K1Z& Z,
     const double r = P.r, z = Z.z;
     const double xsq = (r - z) * (r - z) + 4.0 * r * z * s2;
     if (xsq < 1e-40 || z < 1e-20 || r < 1e-20) return 0.0;
-    const double X = sqrt(xsq);
-    const double lnX = log(X);
+    // X itself is never needed: ln X = ln(X^2) / 2, and squares compare alike
+    const double lnX = 0.5 * log64(xsq), zsq = z * z;
     const double n_x = fmin(loglog_from_log(sN, lnX, 0.0, 1.0), 1.0);
     const double dipole = n_x + Z.n_y - P.n_r - n_x * Z.n_y;
-    const double den_x = alpha_s64_den(lnX, c);
+    const double den_x = alpha_s64_den(xsq, lnX, c);
     // one division for both reciprocals: q = 1 / (den_x X^2)
-    const double q = 1.0 / (den_x * xsq);
+    const double q = rcp64(den_x * xsq);
     const double a_x = q * xsq;
     const double inv_x2 = q * den_x;
-    const double Y = z;
-    const double a_min = fmin(X, Y) <= r ? (X <= Y ? a_x : Z.a_y) : P.a_r;
+    const double a_min = fmin(xsq, zsq) <= r * r ? (xsq <= zsq ? a_x : Z.a_y) : P.a_r;
     const double rxy2 = r * r * inv_x2 * Z.inv_y2;  // r^2 / (X^2 Y^2)
     // Kernel_lo: alpha_r (r^2/(X^2 Y^2) + (alpha_Y/alpha_X - 1)/Y^2 + (alpha_X/alpha_Y - 1)/X^2)
     double lo = P.lo_coef * (rxy2 + (Z.a_y * den_x - 1.0) * Z.inv_y2 + (a_x * Z.den_y - 1.0) * inv_x2);
@@ -277,9 +283,9 @@ __device__ __forceinline__ double k1_theta_term(const K1Parent& P, const K1Z& Z,
     }
     if (!isfinite(dlog)) return 0.0;
     // ln(KSUB r^2 / min(X, Y)^2): the single-log exponent of both slog terms
-    const double lmin = X <= Y ? lnX : Z.log_z;
+    const double lmin = xsq <= zsq ? lnX : Z.log_z;
     const double slog_exp = -abar * (11.0 / 12.0) * fabs(P.log_ksub + 2.0 * (P.log_r - lmin));
-    const double slog = exp(slog_exp);
+    const double slog = exp64(slog_exp);
     const double lo_single = P.lo_coef * rxy2;
     const double k1fin = lo * P.fin_coef;
     return (dlog * slog * lo - lo_single * slog_exp + k1fin) * dipole;

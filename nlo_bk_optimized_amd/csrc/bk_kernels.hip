@@ -35,6 +35,7 @@ BkConsts make_consts(const nlo_bk_physics& p) {
     c.thresholds = p.nf > 3.0;
     c.fixed_as = p.fixed_as;
     c.log_4c2 = std::log(4.0 * p.c2);
+    c.freeze = 2.5 * 2.5 * (p.lambda_qcd * p.lambda_qcd) / (4.0 * p.c2);
     c.production = p.rc_lo == NLO_RC_LO_BALITSKY && p.resum_rc == NLO_RESUM_RC_SMALLEST &&
                    (p.order == NLO_ORDER_NLO_RESUM_DLOG_SLOG || p.order == NLO_ORDER_LO_RESUM_DLOG_SLOG) &&
                    !c.fixed && !c.thresholds;
@@ -316,7 +317,7 @@ __device__ __forceinline__ void k1_body(int R, const double* __restrict__ r, con
             for (int j = j0; j < j1; ++j)
                 acc += k1_theta_term_any(P, Z, s2t[j], s, c, H, rows, rapidity) * wtt[j];
         } else {
-            Z.den_y = alpha_s64_den(Z.log_z, c);
+            Z.den_y = alpha_s64_den(Z.z * Z.z, Z.log_z, c);
             Z.a_y = 1.0 / Z.den_y;
             Z.ly = Z.log_z - P.log_r;
             Z.inv_y2 = 1.0 / (Z.z * Z.z);
@@ -553,29 +554,12 @@ __device__ __forceinline__ K1Z k1_daughter(const K1Parent& P, double log_z, cons
     Z.z = exp(log_z);
     Z.n_y = fmin(loglog_from_log(s, Z.log_z, 0.0, 1.0), 1.0);
     if constexpr (!ANY) {
-        Z.den_y = alpha_s64_den(Z.log_z, c);
+        Z.den_y = alpha_s64_den(Z.z * Z.z, Z.log_z, c);
         Z.a_y = 1.0 / Z.den_y;
         Z.ly = Z.log_z - P.log_r;
         Z.inv_y2 = 1.0 / (Z.z * Z.z);
     }
     return Z;
-}
-
-// sin^2 y for y in [0, pi/2]: with w = y (pi - y), sin y = cos((pi^2/4 -
-// w)^1/2) is entire in w, and sin y / w is its degree-8 interpolant at
-// Chebyshev nodes of [0, pi^2/4] (relative error 3e-20; all terms positive).
-__device__ __forceinline__ double sin2_quadrant(double y) {
-    const double w = y * (kPi - y);
-    double p = fma(w, 1.5070686439285400088e-16, 4.4416425756421120182e-14);
-    p = fma(w, p, 1.0560867829056239888e-11);
-    p = fma(w, p, 1.8975085675213420456e-9);
-    p = fma(w, p, 2.4609343506619309446e-7);
-    p = fma(w, p, 0.000021586579361110788302);
-    p = fma(w, p, 0.0011602715472401966982);
-    p = fma(w, p, 0.03225153443319948851);
-    p = fma(w, p, 0.31830988618379067155);
-    const double s = w * p;
-    return s * s;
 }
 
 // _lo_integrand (S/bk/derivatives.py:434-468) at angle theta, s2 = sin^2(theta / 2).
@@ -608,7 +592,7 @@ __device__ __forceinline__ double k1_theta_adaptive(const K1Parent& P, const K1Z
         const int worst = gk_worst(L, count, a, b);
         const double mid = (a + b) / 2.0;
         const double theta = gk_half_node(g, a, mid, b, lane, half);
-        const double v = g.active ? k1_theta_value<ANY>(P, Z, sin2_quadrant(0.5 * theta), s, c, H, rows, rapidity) : 0.0;
+        const double v = g.active ? k1_theta_value<ANY>(P, Z, sin2_64(0.5 * theta), s, c, H, rows, rapidity) : 0.0;
         gk_rule(g, half, v, est, err);
         gk_split(L, worst, count, lane, a, mid, b, est, err);
         evals += 42;
@@ -693,7 +677,7 @@ __device__ __forceinline__ void k1_adaptive_body(int R, const double* __restrict
     const int rows = (ANY && H.rows) ? min(max(*H.rows, 1), H.capacity) : 0;
     const double rapidity = rows > 0 ? H.y[rows - 1] : 0.0;
     // sin^2(theta / 2) at the lane's node of the rule on [0, pi]
-    const double s2_pi = sin2_quadrant(kPi / 4.0 + kPi / 4.0 * g.x);
+    const double s2_pi = sin2_64(kPi / 4.0 + kPi / 4.0 * g.x);
 
     double value = 0.0, error = 0.0;  // wave 0
     int evals = 0;
@@ -939,7 +923,7 @@ __global__ void __launch_bounds__(kK1aWaves<ANY> * 64)
     const int rows = (ANY && H.rows) ? min(max(*H.rows, 1), H.capacity) : 0;
     const double rapidity = rows > 0 ? H.y[rows - 1] : 0.0;
     // sin^2(theta / 2) at the lane's node of the rule on [0, pi]
-    const double s2_pi = sin2_quadrant(kPi / 4.0 + kPi / 4.0 * g.x);
+    const double s2_pi = sin2_64(kPi / 4.0 + kPi / 4.0 * g.x);
     for (int ring = blockIdx.x % kK1Rings, ended = 0; ended < kK1Rings;) {
         unsigned* ctl = q.ctl + ring * 3 * kK1QueueCtl;
         unsigned ticket = 0u;
