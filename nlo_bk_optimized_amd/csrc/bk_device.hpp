@@ -466,61 +466,55 @@ struct NloValue64 {
     double total, k2, kf;
 };
 
-__device__ __forceinline__ double kernel_nlo64(double r, double X, double Y, double X2, double Y2,
-                                               double Z, double z4) {
-    // S/bk_kernels/k2.py:24-36
-    const double a2 = (X * Y2) * (X * Y2), b2 = (X2 * Y) * (X2 * Y);
-    const double diff = a2 - b2;
-    const double rz = r * Z;
-    const double k = -2.0 / z4 + ((a2 + b2 - 4.0 * rz * rz) / (z4 * diff) + (r * r) * (r * r) / (a2 * diff) +
-                                  r * r / ((X * Y2 * Z) * (X * Y2 * Z))) *
-                                     2.0 * log(X * Y2 / (X2 * Y));
-    return isfinite(k) ? k : 0.0;
-}
-
-__device__ __forceinline__ double kernel_nlo_fermion64(double r, double X, double Y, double X2,
-                                                       double Y2, double Z, double z4, double nf,
-                                                       double nc) {
-    // S/bk_kernels/kf.py:28-38
-    const double a2 = (X * Y2) * (X * Y2), b2 = (X2 * Y) * (X2 * Y);
-    const double rz = r * Z;
-    double k = 2.0 / z4 - (a2 + b2 - rz * rz) / (z4 * (a2 - b2)) * 2.0 * log(X * Y2 / (X2 * Y));
-    k = k * nf / nc;
-    return isfinite(k) ? k : 0.0;
-}
-
 // _nlo_integrand (S/bk/derivatives.py:521-612) times exp(2 ln z + 2 ln z')
-// (S/bk/derivatives.py:335), with the reference's kernels and S dipoles.
+// (S/bk/derivatives.py:335), with the reference's kernels and S dipoles
+// (S/bk_kernels/k2.py:24-36, kf.py:28-38).
+//
+// Bound by FP64 issue.  Only squares of distances and their logarithms are
+// formed, each once: the splines, the coupling and the comparisons take them
+// (X itself never appears).  With a2 = X^2 z'^2, b2 = X'^2 z^2, d = a2 - b2
+// and L = ln(a2 / b2) the kernels are
+//   K2  = c / Z^4 + (r^4 L/d + r^2 L / Z^2) / a2,  c = (a2 + b2 - 4 r^2 Z^2) L/d - 2,
+//   K2s = c / Z^4 + (r^4 L/d - r^2 L / Z^2) / b2,
+//   Kf  = Kfs = (2 - (a2 + b2 - r^2 Z^2) L/d) / Z^4 Nf / Nc,
+// so that one logarithm and four reciprocals serve all four.  d and L come
+// from the same a2 and b2: where they cancel their quotient keeps its value.
 template <bool ANYC>
-__device__ NloValue64 nlo_integrand64(double r, double lz, double lz2, double tz, double tz2,
-                                      const LdsSpline<double>& sS, double r_min, double r_max,
-                                      const BkConsts& c) {
+__device__ NloValue64 nlo_integrand64(double r, double log_r, double lz, double lz2, double tz, double tz2,
+                                      const LdsSpline<double>& sS, const BkConsts& c) {
     NloValue64 out{0.0, 0.0, 0.0};
-    const double z = exp(lz), z2 = exp(lz2);
-    const double s1 = sin(tz / 2.0), s2 = sin(tz2 / 2.0), s3 = sin((tz - tz2) / 2.0);
-    const double xsq = (r - z) * (r - z) + 4.0 * r * z * s1 * s1;
-    const double x2sq = (r - z2) * (r - z2) + 4.0 * r * z2 * s2 * s2;
-    const double zsq = (z - z2) * (z - z2) + 4.0 * z * z2 * s3 * s3;
-    const double X = sqrt(xsq), X2 = sqrt(x2sq), Z = sqrt(zsq);
-    if (X < 1e-20 || z < 1e-20 || X2 < 1e-20 || z2 < 1e-20 || Z < 1e-20) return out;
-    const double Y = z, Y2 = z2;
-    const double S_X = loglog64(sS, r_min, r_max, X, 1.0, 0.0);
-    const double S_Y = loglog64(sS, r_min, r_max, Y, 1.0, 0.0);
-    const double S_X2 = loglog64(sS, r_min, r_max, X2, 1.0, 0.0);
-    const double S_Y2 = loglog64(sS, r_min, r_max, Y2, 1.0, 0.0);
-    const double S_Z = loglog64(sS, r_min, r_max, Z, 1.0, 0.0);
-    const double dmin = fmin(fmin(fmin(r, X), Y), fmin(fmin(X2, Y2), Z));
+    const double z = exp64(lz), z2 = exp64(lz2);
+    const double rsq = r * r, ysq = z * z, y2sq = z2 * z2;
+    const double xsq = (r - z) * (r - z) + 4.0 * r * z * sin2_64(0.5 * tz);
+    const double x2sq = (r - z2) * (r - z2) + 4.0 * r * z2 * sin2_64(0.5 * tz2);
+    const double zsq = (z - z2) * (z - z2) + 4.0 * z * z2 * sin2_64(0.5 * fabs(tz - tz2));
+    if (xsq < 1e-40 || z < 1e-20 || x2sq < 1e-40 || z2 < 1e-20 || zsq < 1e-40) return out;
+    const double lx = 0.5 * log64(xsq), lx2 = 0.5 * log64(x2sq), lZ = 0.5 * log64(zsq);
+    const double S_X = loglog_from_log(sS, lx, 1.0, 0.0);
+    const double S_Y = loglog_from_log(sS, lz, 1.0, 0.0);
+    const double S_X2 = loglog_from_log(sS, lx2, 1.0, 0.0);
+    const double S_Y2 = loglog_from_log(sS, lz2, 1.0, 0.0);
+    const double S_Z = loglog_from_log(sS, lZ, 1.0, 0.0);
+    const double dminsq = fmin(fmin(fmin(rsq, xsq), ysq), fmin(fmin(x2sq, y2sq), zsq));
+    const double lmin = fmin(fmin(fmin(log_r, lx), lz), fmin(fmin(lx2, lz2), lZ));
     // _nlo_alpha_s (S/bk/derivatives.py:615-632)
     double as;
     if constexpr (ANYC)
         as = (c.fixed || c.rc_nlo == NLO_RC_NLO_FIXED) ? c.fixed_as
              : c.rc_nlo == NLO_RC_NLO_PARENT           ? alpha_any64(r, c)
-                                                       : alpha_any64(dmin, c);
+                                                       : alpha_any64(sqrt(dminsq), c);
     else
-        as = alpha_s64(dmin, c);
-    const double z4 = Z * Z * Z * Z;
-    double k = kernel_nlo64(r, X, Y, X2, Y2, Z, z4);
-    double ks = kernel_nlo64(r, X2, Y2, X, Y, Z, z4);
+        as = rcp64(alpha_s64_den(dminsq, lmin, c));
+    const double a2 = xsq * y2sq, b2 = x2sq * ysq, sum = a2 + b2;
+    const double L = log64(div64(a2, b2));
+    // d = 0: no kernel is finite, and each counts as 0
+    const double t = L * rcp64(a2 - b2), iz = rcp64(zsq), iab = rcp64(a2 * b2);
+    const double iz4 = iz * iz, rz = rsq * zsq;
+    const double c2 = ((sum - 4.0 * rz) * t - 2.0) * iz4, u1 = rsq * rsq * t, u2 = rsq * iz * L;
+    double k = c2 + (iab * b2) * (u1 + u2);
+    double ks = c2 + (iab * a2) * (u1 - u2);
+    k = isfinite(k) ? k : 0.0;
+    ks = isfinite(ks) ? ks : 0.0;
     double dip = -(S_X * S_Z * S_Y2 - S_X * S_Y);
     double dips = -(S_X2 * S_Z * S_Y - S_X2 * S_Y2);
     if (fabs(k) > 1e10 && fabs(dip) < 1e-10) { k = 0.0; dip = 0.0; }
@@ -528,13 +522,14 @@ __device__ NloValue64 nlo_integrand64(double r, double lz, double lz2, double tz
     double k2r = c.symmetrize ? (k * dip + ks * dips) / 2.0 : k * dip;
     double kfr = 0.0;
     if (c.nf > 0.0) {
-        const double kf = kernel_nlo_fermion64(r, X, Y, X2, Y2, Z, z4, c.nf, c.nc);
-        const double kfs = kernel_nlo_fermion64(r, X2, Y2, X, Y, Z, z4, c.nf, c.nc);
+        double kf = (2.0 - (sum - rz) * t) * iz4 * (c.nf / c.nc);
+        kf = isfinite(kf) ? kf : 0.0;
         const double df = S_Y * (S_X2 - S_X);
         const double dfs = S_Y2 * (S_X - S_X2);
-        kfr = -(c.symmetrize ? (kf * df + kfs * dfs) / 2.0 : kf * df);
+        kfr = -(c.symmetrize ? kf * (df + dfs) / 2.0 : kf * df);
     }
-    const double scale = (as * c.nc) * (as * c.nc) * c.norm * exp(2.0 * lz + 2.0 * lz2);
+    const double zz = z * z2;
+    const double scale = (as * c.nc) * (as * c.nc) * c.norm * (zz * zz);
     k2r *= scale;
     kfr *= scale;
     out.k2 = isfinite(k2r) ? k2r : 0.0;

@@ -1271,7 +1271,6 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
         fsp.vmin = vector_reg(fsp.vmin);
         fsp.vmax = vector_reg(fsp.vmax);
     }
-    const double r_min64 = v.t64[0], r_max64 = v.t64[1];
 
     const int lane = threadIdx.x & 63;
     const int wave = uniform(threadIdx.x >> 6);
@@ -1358,8 +1357,7 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
         double wv = 0.0, k2 = 0.0, kf = 0.0;
         if (valid) {
             if constexpr (MODE == NLO_PREC_FP64) {
-                const NloValue64 f = nlo_integrand64<ANYC>(rp, x[0], x[1], x[2], x[3], spl, r_min64,
-                                                           r_max64, a.c);
+                const NloValue64 f = nlo_integrand64<ANYC>(rp, log_rp, x[0], x[1], x[2], x[3], spl, a.c);
                 wv = f.total * (double)jac;
                 k2 = f.k2 * (double)jac;
                 kf = f.kf * (double)jac;
