@@ -42,6 +42,21 @@ __device__ __forceinline__ double div64(double a, double b) {
     return fma(fma(-b, q, a), r, q);
 }
 
+// 1 / sqrt(x) for ordinary x > 0: the hardware estimate (2^-24) and one step
+// of third order.
+__device__ __forceinline__ double rsqrt64(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x * y, y, 1.0);
+    return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+// sqrt(x) for x = 0 and ordinary x > 0 (NaN below 0).
+__device__ __forceinline__ double sqrt64(double x) {
+    const double y = rsqrt64(x), g = x * y;
+    const double r = fma(fma(-g, g, x), 0.5 * y, g);
+    return x == 0.0 ? 0.0 : r;
+}
+
 // ln x for finite x > 0 (NaN for NaN).  x = 2^e (1 + f), 1 + f in [1/sqrt 2,
 // sqrt 2); with s = f / (2 + f), ln(1 + f) = 2 atanh s = f - f^2/2 +
 // s (f^2/2 + R(s^2)), where R(z) = 2 (z/3 + z^2/5 + ..) (degree 7,
