@@ -72,6 +72,16 @@ __device__ inline RuleView stage_nested_rule(int n, double* y, double* w) {
     return {n, y, w};
 }
 
+// The same from nodes and weights that were prepared once (n of each).
+__device__ inline RuleView load_nested_rule(int n, const double* rule, double* y, double* w) {
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+        y[i] = rule[i];
+        w[i] = rule[kMaxNested + i];
+    }
+    __syncthreads();
+    return {n, y, w};
+}
+
 // Everything an integrand reads, by value in the kernel arguments.
 struct DisArgs {
     double Q2, xbj;

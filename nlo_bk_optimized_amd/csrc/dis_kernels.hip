@@ -213,6 +213,7 @@ struct VegasView {
     double* part;         // blocks x 2
     double* part_hist;    // blocks x D x bins
     double* part_cnt;
+    const double* rule;   // the nested rule (2 x kMaxNested), or null: made here
 };
 
 struct ArgsSobol {  // a single pass: the table in the kernel arguments
@@ -241,7 +242,8 @@ __device__ __forceinline__ void vegas_pass(const DisArgs& a, const VegasView& v,
     __shared__ double wmax[4];
     __shared__ double ry[kMaxNested], rw[kMaxNested];
     RuleView rule{0, ry, rw};
-    if constexpr (K == NLO_DIS_QG_I2_NESTED || K == NLO_DIS_QG_I3_NESTED) rule = stage_nested_rule(a.nested_points, ry, rw);
+    if constexpr (K == NLO_DIS_QG_I2_NESTED || K == NLO_DIS_QG_I3_NESTED)
+        rule = v.rule ? load_nested_rule(a.nested_points, v.rule, ry, rw) : stage_nested_rule(a.nested_points, ry, rw);
     const VegasLayout lay = vegas_layout(D, v.bins, v.spt, HIST);
     double* E = reinterpret_cast<double*>(smem + lay.edges);
     uint32_t* dir = reinterpret_cast<uint32_t*>(smem + lay.dir);
@@ -368,7 +370,7 @@ __device__ __forceinline__ void vegas_pass(const DisArgs& a, const VegasView& v,
 // One VEGAS pass (see nlo_dis_vegas).
 template <typename T, int K, bool HIST>
 __global__ void __launch_bounds__(256) vegas_kernel(DisArgs a, VegasArgs v) {
-    const VegasView view{v.bins, v.spt, v.n, v.first, v.edges, v.part, v.part_hist, v.part_cnt};
+    const VegasView view{v.bins, v.spt, v.n, v.first, v.edges, v.part, v.part_hist, v.part_cnt, nullptr};
     vegas_pass<T, K, HIST>(a, view, ArgsSobol{v}, blockIdx.x);
 }
 
@@ -465,12 +467,29 @@ __global__ void __launch_bounds__(256) gl_kernel(DisArgs a, int points, double* 
 // integrals skip the remaining iterations on the device.
 
 constexpr int kBatchMaxIterations = 16;
-constexpr int kBatchSpt = 8;  // 64-point groups per wave: 2048 samples per block
+
+// 64-point groups per wave (256 samples of a block each): 8, less for integrals
+// whose blocks would not reach kBatchBlocks: an iteration of a point budget of
+// 2^18 evaluations is 2^15 samples or fewer, 16 blocks of 8 groups on 256
+// CUs.  By the integral's own samples alone, so that its result does not
+// depend on what shares its batch.  One point on a table in FP64 / four points
+// in FP32 / F2 of 2 10^6 evaluations: always 8 groups 11.1 / 23.0 / 18.4 ms;
+// 256 blocks 7.8 / 21.8 / 16.9, 512 6.6 / 20.3 / 16.3, 1024 6.8 / 20.6 / 16.2,
+// 2048 7.1 / 22.2 / 16.4 (a block's fixed work, mostly its grid and histogram).
+constexpr int kBatchMaxSpt = 8;
+constexpr int kBatchBlocks = 512;
+
+int batch_spt(int64_t n) {
+    const int64_t g64 = (n + 63) / 64;
+    int spt = kBatchMaxSpt;
+    while (spt > 1 && (g64 + 4 * spt - 1) / (4 * spt) < kBatchBlocks) spt >>= 1;
+    return spt;
+}
 
 // One VEGAS integral of a batch: its item, plan and where its data live.
 struct VItem {
     int item, K, D, table;
-    int blocks, groups, per_group;
+    int spt, blocks, groups, per_group;
     int max_it, min_it;
     int64_t n, stride, first;
     int64_t part;   // doubles into the partial buffer: blocks x 2 sums, then the
@@ -478,6 +497,7 @@ struct VItem {
                     // the group histogram and counts (2 x groups x cells)
     int64_t grid;   // doubles into the grid buffer: edges (2 buffers of
                     // D x (bins + 1)), histogram, counts (cells each), sums (2)
+    int64_t rule;   // doubles into the grid buffer: the nested rule, or -1
 };
 
 // Per-integral iteration state, on the device.
@@ -528,8 +548,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kDisWa
     const double* edges = b.grid + it.grid + (int64_t)(st.iters & 1) * it.D * (b.bins + 1);
     double* part = b.part + it.part;
     double* ph = part + 2 * (int64_t)it.blocks;
-    const VegasView view{b.bins, kBatchSpt, it.n, it.first + (int64_t)st.iters * it.stride, edges, part, ph,
-                         ph + (int64_t)it.blocks * cells};
+    const VegasView view{b.bins, it.spt, it.n, it.first + (int64_t)st.iters * it.stride, edges, part, ph,
+                         ph + (int64_t)it.blocks * cells, it.rule < 0 ? nullptr : b.grid + it.rule};
     vegas_pass<T, K, true>(b.args[it.item], view, TableSobol{b.tables + it.table}, w.y);
 }
 
@@ -675,6 +695,9 @@ __global__ void __launch_bounds__(256) vegas_batch_init_kernel(BatchDev b, const
     }
     double* g = b.grid + it.grid;
     for (int i = threadIdx.x; i < it.D * (b.bins + 1); i += blockDim.x) g[i] = edges0[i % (b.bins + 1)];
+    // the nested rule of the integral, once for all its blocks and iterations
+    if (it.rule >= 0)
+        (void)stage_nested_rule(b.args[it.item].nested_points, b.grid + it.rule, b.grid + it.rule + kMaxNested);
 }
 
 // Gauss-Legendre items of kind K: block (0 | 1, item) the fine or the coarse rule.
@@ -970,7 +993,8 @@ int batch_plan(const nlo_dis_batch_desc* d, BatchPlan& P, bool build_args) {
         v.max_it = item.max_iterations;
         v.min_it = item.min_iterations;
         const int64_t g64 = (item.n + 63) / 64;
-        const int64_t blocks = (g64 + 4 * kBatchSpt - 1) / (4 * kBatchSpt);
+        v.spt = batch_spt(item.n);
+        const int64_t blocks = (g64 + 4 * v.spt - 1) / (4 * v.spt);
         NLO_REQUIRE(blocks <= (1 << 24), "nlo_dis_batch: item %d: too many samples", i);
         v.blocks = (int)blocks;
         v.per_group = (v.blocks + kHistGroups - 1) / kHistGroups;
@@ -980,6 +1004,11 @@ int batch_plan(const nlo_dis_batch_desc* d, BatchPlan& P, bool build_args) {
         P.part_doubles += vpart_doubles(v.blocks, v.groups, cells);
         v.grid = P.grid_doubles;
         P.grid_doubles += vgrid_doubles(D, bins);
+        v.rule = -1;
+        if (K == NLO_DIS_QG_I2_NESTED || K == NLO_DIS_QG_I3_NESTED) {
+            v.rule = P.grid_doubles;
+            P.grid_doubles += 2 * kMaxNested;
+        }
         const int vi = (int)P.vi.size();
         for (int b = 0; b < v.blocks; ++b) work[slot].push_back(make_int2(vi, b));
         for (int dd = 0; dd < D; ++dd) P.rows.push_back(make_int2(vi, dd));
@@ -991,7 +1020,7 @@ int batch_plan(const nlo_dis_batch_desc* d, BatchPlan& P, bool build_args) {
     for (int slot = 0; slot < NLO_DIS_KINDS * 2; ++slot) {
         const int K = slot / 2, prec = (slot & 1) ? NLO_PREC_FP32 : NLO_PREC_FP64;
         if (!work[slot].empty()) {
-            const size_t lds = vegas_layout(kDims[K], bins, kBatchSpt, true).total;
+            const size_t lds = vegas_layout(kDims[K], bins, kBatchMaxSpt, true).total;
             NLO_REQUIRE(lds <= 64 * 1024, "nlo_dis_batch: LDS %zu bytes exceeds 64 KiB (fewer bins)", lds);
             P.launches.push_back({K, prec, (int)P.work.size(), (int)work[slot].size(), lds});
             P.work.insert(P.work.end(), work[slot].begin(), work[slot].end());
