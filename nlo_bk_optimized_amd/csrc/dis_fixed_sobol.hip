@@ -369,11 +369,10 @@ __global__ void __launch_bounds__(256) fs_train_reduce_kernel(FsDev f, int slice
 // (learn_triple_importance_grid, S/dis/fixed_sobol.py:193-208; the per-point
 // scores summed per bin equal the per-bin |w_k| sums so weighted, the sums
 // being linear) and the refined grid: block (estimator, dimension) forms the
-// scores and their smoothed importances (vegas_smoothed) in parallel in LDS,
-// then one lane refines the edge row from the current buffer into the other
-// one with the same operations as vegas_adapt_row.
+// scores in LDS and refines the edge row from the current buffer into the
+// other one.
 __global__ void __launch_bounds__(64) fs_adapt_kernel(FsDev f, int round, double eps, double tiny) {
-    __shared__ double sc[256], cn[256], ed[256], sm[256];
+    __shared__ double sc[256], cn[256], scratch[kAdaptScratch(256)];
     const int item = blockIdx.x / kFsDim, d = blockIdx.x - item * kFsDim;
     const int bins = f.bins, cells = fs_cells(bins);
     double* st = f.stat + (int64_t)item * f.stat_stride;
@@ -393,11 +392,8 @@ __global__ void __launch_bounds__(64) fs_adapt_kernel(FsDev f, int round, double
         cn[b] = cnt[(int64_t)d * bins + b];
         st[fs_train_part(bins) + (int64_t)d * bins + b] = v;
     }
-    for (int b = threadIdx.x; b <= bins; b += blockDim.x) ed[b] = e[b];
     __syncthreads();
-    for (int b = threadIdx.x; b < bins; b += blockDim.x) sm[b] = vegas_smoothed(sc, cn, bins, b, eps);
-    __syncthreads();
-    if (threadIdx.x == 0) vegas_adapt_row_with(ed, [&](int i) { return sm[i]; }, bins, o);
+    vegas_adapt_block(e, sc, cn, bins, eps, o, scratch);
 }
 
 // Replicate estimates: block (estimator, replicate), one wave: the block sums

@@ -615,12 +615,11 @@ __global__ void __launch_bounds__(256) vegas_batch_reduce_kernel(BatchDev b, int
 }
 
 // Grid refinement of every active integral, one (integral, dimension) per
-// thread: the current edge buffer into the other one.
+// block: the current edge buffer into the other one.
 __global__ void __launch_bounds__(64) vegas_batch_adapt_kernel(BatchDev b, const int2* __restrict__ rows,
-                                                               int n_rows, double eps) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n_rows) return;
-    const int2 rw = rows[k];
+                                                               double eps) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int2 rw = rows[blockIdx.x];
     const VItem& it = b.vi[rw.x];
     const VState& st = b.st[rw.x];
     if (!vitem_active(it, st)) return;
@@ -629,7 +628,7 @@ __global__ void __launch_bounds__(64) vegas_batch_adapt_kernel(BatchDev b, const
     const double* e = g + (int64_t)(st.iters & 1) * E + (int64_t)rw.y * (b.bins + 1);
     double* o = g + (int64_t)((st.iters + 1) & 1) * E + (int64_t)rw.y * (b.bins + 1);
     const double* hist = g + 2 * (int64_t)E + (int64_t)rw.y * b.bins;
-    vegas_adapt_row(e, hist, hist + cells, b.bins, eps, o);
+    vegas_adapt_block(e, hist, hist + cells, b.bins, eps, o, reinterpret_cast<double*>(smem));
 }
 
 // s + x into the double-double (s, c) (TwoSum; Knuth).
@@ -1086,7 +1085,8 @@ int enqueue_batch_iteration(const BatchPlan& P, const BatchDev& bd, const int2* 
                        rblocks);
     NLO_LAUNCH_CHECK();
     const int nr = (int)P.rows.size();
-    hipLaunchKernelGGL(vegas_batch_adapt_kernel, dim3((nr + 63) / 64), dim3(64), 0, s, bd, rows, nr, eps);
+    hipLaunchKernelGGL(vegas_batch_adapt_kernel, dim3(nr), dim3(64), kAdaptScratch(bd.bins) * sizeof(double), s, bd,
+                       rows, eps);
     NLO_LAUNCH_CHECK();
     hipLaunchKernelGGL(vegas_batch_stats_kernel, dim3((nv + 63) / 64), dim3(64), 0, s, bd, nv, tiny, epsrel, epsabs);
     NLO_LAUNCH_CHECK();

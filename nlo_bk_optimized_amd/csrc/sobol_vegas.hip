@@ -269,16 +269,16 @@ __global__ void vegas_hist_reduce_kernel(int values, int groups, const double* _
     count[k] = sc;
 }
 
-// _adapt_vegas_edges (S/numerics/integration.py:835-866) for one (row, dim)
-// per thread (vegas_adapt_row, vegas_grid.hpp).
-__global__ void vegas_adapt_kernel(int rows, int dim, int bins, const double* __restrict__ edges,
-                                   const double* __restrict__ hist,
-                                   const double* __restrict__ count, double eps,
-                                   double* __restrict__ out) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= rows * dim) return;
-    vegas_adapt_row(edges + (size_t)k * (bins + 1), hist + (size_t)k * bins, count + (size_t)k * bins, bins,
-                    eps, out + (size_t)k * (bins + 1));
+// _adapt_vegas_edges (S/numerics/integration.py:835-866), one (row, dim) per
+// block (vegas_adapt_block, vegas_grid.hpp).
+__global__ void __launch_bounds__(64) vegas_adapt_kernel(int bins, const double* __restrict__ edges,
+                                                         const double* __restrict__ hist,
+                                                         const double* __restrict__ count, double eps,
+                                                         double* __restrict__ out) {
+    extern __shared__ double scratch[];
+    const size_t k = blockIdx.x;
+    vegas_adapt_block(edges + k * (bins + 1), hist + k * bins, count + k * bins, bins, eps, out + k * (bins + 1),
+                      scratch);
 }
 
 }  // namespace
@@ -305,8 +305,11 @@ const char* last_error() { return g_error.c_str(); }
 int launch_vegas_adapt(int rows, int dim, int bins, const double* edges, const double* hist,
                        const double* count, double eps, double* out, hipStream_t stream) {
     const int items = rows * dim;
-    hipLaunchKernelGGL(vegas_adapt_kernel, dim3((items + 63) / 64), dim3(64), 0, stream, rows, dim,
-                       bins, edges, hist, count, eps, out);
+    const size_t lds = kAdaptScratch(bins) * sizeof(double);
+    if (lds > 65536)  // more than 2730 bins: beyond the default limit of dynamic LDS
+        NLO_HIP_CHECK(hipFuncSetAttribute((const void*)vegas_adapt_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          (int)lds));
+    hipLaunchKernelGGL(vegas_adapt_kernel, dim3(items), dim3(64), lds, stream, bins, edges, hist, count, eps, out);
     NLO_LAUNCH_CHECK();
     return NLO_OK;
 }
