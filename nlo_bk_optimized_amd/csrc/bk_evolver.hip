@@ -23,7 +23,8 @@ struct nlo_bk_evolver {
     double* T;      // adaptive: two half steps
     double* ctl;    // adaptive: [0] step, [1] error ratio
     double* k1;
-    void* k1_ws;  // the adaptive rule's queue
+    void* k1_ws;  // the adaptive rule's queue, or the fixed rule's shares
+    int k1_shares;
     double* k2kf;
     double* sums;
     double* t64;
@@ -78,7 +79,7 @@ EvolverLayout evolver_layout(const nlo_bk_evolver_desc& d) {
     L.flag = take(sizeof(int32_t));
     L.rows = take(sizeof(int32_t));
     L.active = take(sizeof(unsigned long long));
-    L.k1_ws = take(d.k1_rule == NLO_K1_ADAPTIVE ? k1_queue_workspace(d.R) : 1);
+    L.k1_ws = take(d.k1_rule == NLO_K1_ADAPTIVE ? k1_queue_workspace(d.R) : 2 * kK1MaxShares * R * sizeof(double));
     L.nlo_ws_bytes = d.nlo ? nlo_plan(d.R, d.bins, d.n_samples, false).workspace : 0;
     L.nlo_ws = take(L.nlo_ws_bytes > 0 ? L.nlo_ws_bytes : 1);
     L.total = o;
@@ -211,17 +212,19 @@ int enqueue_rhs(nlo_bk_evolver* ev, const double* in, double* out, hipStream_t s
         rc = launch_k1_queue(R, ev->r, in, ev->t64, ev->c, d.k1_rint, d.k1_tint, d.k1_epsrel, ev->k1, ev->k1_ws,
                              ev->flag, s, d.kinematical ? &H : nullptr);
     else
-        rc = launch_k1(R, ev->r, in, ev->t64, ev->c, d.nr, d.nt, ev->k1, s, d.kinematical ? &H : nullptr);
+        rc = launch_k1(R, ev->r, in, ev->t64, ev->c, d.nr, d.nt, ev->k1, s, d.kinematical ? &H : nullptr,
+                       static_cast<double*>(ev->k1_ws), ev->k1_shares);
     if (rc != NLO_OK) return rc;
+    const double* part = ev->k1_shares > 1 ? static_cast<const double*>(ev->k1_ws) : nullptr;
     if (d.nlo) {
         rc = launch_nlo(R, ev->r, in, ev->t64, ev->t32, ev->edges, d.bins, d.sobol, d.first_index,
                         d.n_samples, d.precision, ev->c, ev->sums, nullptr, nullptr, ev->nlo_ws,
                         ev->nlo_ws_bytes, s, /*components=*/false);
         if (rc != NLO_OK) return rc;
-        return launch_rhs_finalize(R, in, ev->k1, ev->sums, d.n_samples, out, ev->k2kf, ev->active, s);
+        return launch_rhs_finalize(R, in, ev->k1, ev->sums, d.n_samples, out, ev->k2kf, ev->active, s, part, ev->k1_shares);
     }
     // LO-only: K2 + Kf sums stay zero
-    return launch_rhs_finalize(R, in, ev->k1, ev->sums, 1, out, ev->k2kf, ev->active, s);
+    return launch_rhs_finalize(R, in, ev->k1, ev->sums, 1, out, ev->k2kf, ev->active, s, part, ev->k1_shares);
 }
 
 // Enqueues one fixed RK step on `s` (captured into the graph).
@@ -446,6 +449,7 @@ int nlo_bk_evolver_create(const nlo_bk_evolver_desc* desc, const double* d_r, co
     ev->rows = reinterpret_cast<int32_t*>(w + L.rows);
     ev->active = reinterpret_cast<unsigned long long*>(w + L.active);
     ev->k1_ws = w + L.k1_ws;
+    ev->k1_shares = d.k1_rule == NLO_K1_ADAPTIVE ? 1 : nlo::k1_shares(d.R);
     ev->nlo_ws = w + L.nlo_ws;
     ev->nlo_ws_bytes = L.nlo_ws_bytes;
     ev->y = 0.0;

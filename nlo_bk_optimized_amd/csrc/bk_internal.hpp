@@ -32,7 +32,12 @@ NloPlan nlo_plan(int R, int bins, int64_t n, bool hist, bool fp32 = false);
 int launch_spline_build(int R, const double* r, const double* N, int force_positive, double* t64,
                         float* t32, hipStream_t stream);
 int launch_k1(int R, const double* r, const double* N, const double* t64, const BkConsts& c, int nr,
-              int nt, double* k1, hipStream_t stream, const K1History* hist = nullptr);
+              int nt, double* k1, hipStream_t stream, const K1History* hist = nullptr, double* part = nullptr,
+              int shares = 1);
+// Blocks per parent of K1 where the caller has room for their sums (`part`:
+// 2 R shares doubles, merged by launch_rhs_finalize).
+constexpr int kK1MaxShares = 8;
+int k1_shares(int R);
 int launch_k1_adaptive(int R, const double* r, const double* N, const double* t64, const BkConsts& c,
                        int rint, int tint, double epsrel, double* k1, double* k1_err,
                        long long* k1_evals, hipStream_t stream, const K1History* hist = nullptr);
@@ -47,8 +52,9 @@ int launch_nlo(int R, const double* r, const double* N, const double* t64, const
                const double* edges, int bins, const nlo_sobol_table& sobol, int64_t first, int64_t n,
                int precision, const BkConsts& c, double* sums, double* hist, double* count, void* ws,
                size_t ws_bytes, hipStream_t stream, bool components = true);
-int launch_rhs_finalize(int R, const double* N, const double* k1, const double* sums, int64_t n,
-                        double* dndy, double* k2kf, unsigned long long* counter, hipStream_t stream);
+int launch_rhs_finalize(int R, const double* N, double* k1, const double* sums, int64_t n,
+                        double* dndy, double* k2kf, unsigned long long* counter, hipStream_t stream,
+                        const double* k1_part = nullptr, int shares = 1);
 int launch_rk_stage(int R, const double* N, const double* K0, const double* K1, const double* K2,
                     double a0, double a1, double a2, double h, double* out, hipStream_t stream);
 int launch_rk_final(int R, double* N, const double* K0, const double* K1, const double* K2,

@@ -261,14 +261,16 @@ __device__ __forceinline__ K1Parent k1_parent(double r, const LdsSpline<double>&
     return P;
 }
 
+// `shares` blocks may split a parent's items: each leaves its compensated sum
+// in part[p][share] and rhs_finalize_kernel merges them (k1_shares).
 // ANY = false: the production physics with the hoisted per-z-node terms;
 // ANY = true: every coupling / order choice and the kinematical constraint
 // (H.rows set), the full Kernel_lo per theta node.
 template <bool ANY>
 __device__ __forceinline__ void k1_body(int R, const double* __restrict__ r, const double* __restrict__ N,
                                         const double* __restrict__ t64, const BkConsts& c,
-                                        const GaussRule& g, const K1History& H, int p,
-                                        double* __restrict__ k1) {
+                                        const GaussRule& g, const K1History& H, int p, int share, int shares,
+                                        double* __restrict__ k1, double2* __restrict__ part) {
     extern __shared__ double sh[];
     __shared__ double red[kK1Threads / 64][2];
     __shared__ double gxr[kMaxGaussR], gwr[kMaxGaussR], s2t[kMaxGaussT], wtt[kMaxGaussT];
@@ -301,7 +303,7 @@ __device__ __forceinline__ void k1_body(int R, const double* __restrict__ r, con
     // waves of one item per z node, so the FP64 latency is better hidden
     const int th = (g.nt + 1) / 2;
     double total = 0.0, total_err = 0.0;  // compensated
-    for (int item = threadIdx.x; item < 2 * znodes; item += blockDim.x) {
+    for (int item = threadIdx.x + share * blockDim.x; item < 2 * znodes; item += shares * blockDim.x) {
         const int zi = item >> 1;
         const int j0 = (item & 1) * th, j1 = min(j0 + th, g.nt);
         const int panel = zi / g.nr;
@@ -334,7 +336,10 @@ __device__ __forceinline__ void k1_body(int R, const double* __restrict__ r, con
     if (threadIdx.x == 0) {
         double t = red[0][0], e = red[0][1];
         for (int w = 1; w < kK1Threads / 64; ++w) comp_merge(t, e, red[w][0], red[w][1]);
-        k1[p] = t + e;
+        if (shares > 1)
+            part[(size_t)p * shares + share] = make_double2(t, e);
+        else
+            k1[p] = t + e;
     }
 }
 
@@ -342,9 +347,9 @@ template <bool ANY>
 __global__ void __launch_bounds__(kK1Threads) k1_kernel(int R, const double* __restrict__ r,
                                                         const double* __restrict__ N,
                                                         const double* __restrict__ t64, BkConsts c,
-                                                        GaussRule g, K1History H,
-                                                        double* __restrict__ k1) {
-    k1_body<ANY>(R, r, N, t64, c, g, H, blockIdx.x, k1);
+                                                        GaussRule g, K1History H, double* __restrict__ k1,
+                                                        double2* __restrict__ part) {
+    k1_body<ANY>(R, r, N, t64, c, g, H, blockIdx.x, blockIdx.y, gridDim.y, k1, part);
 }
 
 // ------------------------------------------------------ K1, adaptive rule
@@ -1514,7 +1519,9 @@ __global__ void __launch_bounds__(256) nlo_reduce_kernel(int R, int bpp, int bin
 
 // counter (optional) accumulates the number of active parents: integer
 // adds, so the total is exact whatever the order.
-__global__ void rhs_finalize_kernel(int R, const double* __restrict__ N, const double* __restrict__ k1,
+// k1_part (k1_shares x R pairs, or null): the shares of K1, merged into k1.
+__global__ void rhs_finalize_kernel(int R, const double* __restrict__ N, double* __restrict__ k1,
+                                    const double2* __restrict__ k1_part, int k1_shares,
                                     const double* __restrict__ sums, double inv_n,
                                     double* __restrict__ dndy, double* __restrict__ k2kf,
                                     unsigned long long* __restrict__ counter) {
@@ -1525,6 +1532,12 @@ __global__ void rhs_finalize_kernel(int R, const double* __restrict__ N, const d
     bool active = false;
     if (p < R) {
         active = p >= 1 && N[p] <= 0.99999;
+        if (active && k1_part) {
+            double t = k1_part[(size_t)p * k1_shares].x, e = k1_part[(size_t)p * k1_shares].y;
+            for (int s = 1; s < k1_shares; ++s)
+                comp_merge(t, e, k1_part[(size_t)p * k1_shares + s].x, k1_part[(size_t)p * k1_shares + s].y);
+            k1[p] = t + e;
+        }
         const double nlo = active ? sums[(size_t)p * 4] * inv_n : 0.0;
         double v = active ? k1[p] + nlo : 0.0;
         dndy[p] = isfinite(v) ? v : 0.0;
@@ -1590,7 +1603,7 @@ __global__ void __launch_bounds__(kK1Threads) k1_batch_kernel(const BatchRun* __
     const BatchRun run = runs[node_run[blockIdx.x]];
     const K1History H{};
     k1_body<ANY>(run.R, r + run.node_off, N + run.node_off, t64 + run.spline_off, c, g, H,
-                 blockIdx.x - run.node_off, k1 + run.node_off);
+                 blockIdx.x - run.node_off, 0, 1, k1 + run.node_off, nullptr);
 }
 
 // The adaptive rule, one block per node of every run.
@@ -1772,8 +1785,32 @@ int launch_spline_build(int R, const double* r, const double* N, int force_posit
     return NLO_OK;
 }
 
+// A block of K1 fills a CU, so R parents leave the last wave of blocks nearly
+// empty, or most of the chip idle (101 nodes: 156 of 256 CUs).  Splitting each
+// parent over s blocks takes ceil(R s / CUs) waves of 1 / s of a parent's work
+// and what a block costs besides (its tables, a tenth); the s of least time.
+// The step on the default 101 nodes went from 424 to 370 us (2 shares).
+int k1_shares(int R) {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) {
+        (void)hipGetLastError();
+        return 1;
+    }
+    int best = 1;
+    double least = 0.0;
+    for (int s = 1; s <= kK1MaxShares; ++s) {
+        const double t = ((R - 1) * s + cus - 1) / cus * (1.0 / s + 0.1);
+        if (s == 1 || t < least) {
+            least = t;
+            best = s;
+        }
+    }
+    return best;
+}
+
 int launch_k1(int R, const double* r, const double* N, const double* t64, const BkConsts& c, int nr,
-              int nt, double* k1, hipStream_t stream, const K1History* hist) {
+              int nt, double* k1, hipStream_t stream, const K1History* hist, double* part, int shares) {
     GaussRule g{};
     g.nr = nr;
     g.nt = nt;
@@ -1785,11 +1822,11 @@ int launch_k1(int R, const double* r, const double* N, const double* t64, const 
     K1History H{};
     if (hist) H = *hist;
     if (c.production && !hist)
-        hipLaunchKernelGGL(k1_kernel<false>, dim3(R), dim3(kK1Threads), smem, stream, R, r, N, t64, c,
-                           g, H, k1);
+        hipLaunchKernelGGL(k1_kernel<false>, dim3(R, shares), dim3(kK1Threads), smem, stream, R, r, N, t64, c,
+                           g, H, k1, reinterpret_cast<double2*>(part));
     else
-        hipLaunchKernelGGL(k1_kernel<true>, dim3(R), dim3(kK1Threads), smem, stream, R, r, N, t64, c, g,
-                           H, k1);
+        hipLaunchKernelGGL(k1_kernel<true>, dim3(R, shares), dim3(kK1Threads), smem, stream, R, r, N, t64, c, g,
+                           H, k1, reinterpret_cast<double2*>(part));
     NLO_LAUNCH_CHECK();
     return NLO_OK;
 }
@@ -1971,10 +2008,11 @@ int launch_nlo(int R, const double* r, const double* N, const double* t64, const
     return NLO_OK;
 }
 
-int launch_rhs_finalize(int R, const double* N, const double* k1, const double* sums, int64_t n,
-                        double* dndy, double* k2kf, unsigned long long* counter, hipStream_t stream) {
+int launch_rhs_finalize(int R, const double* N, double* k1, const double* sums, int64_t n,
+                        double* dndy, double* k2kf, unsigned long long* counter, hipStream_t stream,
+                        const double* k1_part, int shares) {
     hipLaunchKernelGGL(rhs_finalize_kernel, dim3((R + 255) / 256), dim3(256), 0, stream, R, N, k1,
-                       sums, 1.0 / (double)n, dndy, k2kf, counter);
+                       reinterpret_cast<const double2*>(k1_part), shares, sums, 1.0 / (double)n, dndy, k2kf, counter);
     NLO_LAUNCH_CHECK();
     return NLO_OK;
 }
@@ -2352,7 +2390,7 @@ int nlo_bk_rhs_finalize(int32_t R, const double* d_N, const double* d_k1, const 
                         int64_t n, double* d_dndy, double* d_k2kf, hipStream_t stream) {
     NLO_REQUIRE(R >= 1 && n >= 1, "nlo_bk_rhs_finalize: R=%d n=%lld invalid", R, (long long)n);
     NLO_REQUIRE(d_N && d_k1 && d_sums && d_dndy, "nlo_bk_rhs_finalize: null pointer");
-    const int rc = nlo::launch_rhs_finalize(R, d_N, d_k1, d_sums, n, d_dndy, d_k2kf, nullptr, stream);
+    const int rc = nlo::launch_rhs_finalize(R, d_N, const_cast<double*>(d_k1), d_sums, n, d_dndy, d_k2kf, nullptr, stream);
     if (rc == NLO_OK) nlo::clear_error();
     return rc;
 }

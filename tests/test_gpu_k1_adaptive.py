@@ -216,6 +216,37 @@ def test_evolver_queue_matches_the_block_kernel(dev, R, active, limits, variant)
         ev.close()
 
 
+@pytest.mark.parametrize("R", [3, 24, 65, 101, 129, 257, 300])
+def test_evolver_shares_of_a_parent_match_one_block(dev, R):
+    """The fixed rule: the evolver splits a parent over 1 to 8 blocks by the
+    number of nodes, nlo_bk_k1 takes one.  Both sum with compensation: the
+    difference is one rounding of the sum of magnitudes (1e-13 of the largest
+    K1 covers its cancellation)."""
+
+    from nlo_bk_optimized_amd.bk.config import BKConfig
+    from nlo_bk_optimized_amd.bk.evolution import prepare
+
+    print(f"fixed K1 shares R={R}", flush=True)
+    cfg = BKConfig(RPOINTS=R - 1, MINR=1e-6, MAXR=1e2, MCINTPOINTS=1 << 10, RK_METHOD="euler", DE_SOLVER_STEP=0.1)
+    setup = prepare(_mv(), cfg, device=torch.device("cuda"), seed=0)
+    ev = dev.Evolver(setup.r, setup.edges, setup.table, cfg, n_samples=setup.n_samples, precision="fp64",
+                     rk_method="euler", step=0.1, nlo=False)
+    try:
+        state = setup.N0.clone()
+        state[R // 2] = 1.0  # an inactive parent between active ones
+        ev.state.copy_(state)
+        t64, _ = dev.spline_build(setup.r, state)
+        want = dev.bk_k1(setup.r, state, t64, cfg)
+        for _ in range(2):
+            ev.state.copy_(state)
+            ev.step()
+            active = state <= 0.99999
+            active[0] = False
+            assert torch.all((ev.k1 - want).abs()[active] <= 1e-12 * want.abs()[active] + 1e-13 * want.abs().max())
+    finally:
+        ev.close()
+
+
 def _order(name):
     from nlo_bk_optimized_amd.bk.config import BKOrder
 
