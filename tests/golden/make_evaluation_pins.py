@@ -1,0 +1,59 @@
+"""Values of the plain evaluation of the integrands, recorded on an MI355X.
+
+    python tests/golden/make_evaluation_pins.py OUTPUT_DIRECTORY
+
+The FP64 integrands have samples whose terms cancel by many digits, where
+another order of the same operations gives other digits.  The recorded numbers
+are those of the formulas written out with the math library's functions and
+IEEE operations (the library as built from commit de78377); later kernels keep
+them.  Each section is one .npz next to this file.
+"""
+
+from __future__ import annotations
+
+import sys
+
+import numpy as np
+import torch
+
+from nlo_bk_optimized_amd import device as dev
+from nlo_bk_optimized_amd.bk import MV, BKConfig
+from nlo_bk_optimized_amd.bk.config import RunningCouplingNLO
+from nlo_bk_optimized_amd.bk.evolution import uniform_edges
+
+NODES = 24
+SOBOL_SEEDS = (109, 110, 215, 339)  # each with a sample next to a2 = b2 in some parent
+
+
+def bk_sums() -> dict[str, np.ndarray]:
+    """Per-parent K2 + Kf sums of the FP64 formula, by kernel instance."""
+
+    r = (1e-6 * torch.pow(torch.tensor((100.0 / 1e-6) ** (1 / (NODES - 1)), dtype=torch.float64),
+                          torch.arange(NODES, dtype=torch.float64))).cuda()
+    N = MV(qs0sqr=0.2).dipole_amplitude(r)
+    t64, t32 = dev.spline_build(r, N)
+    edges = uniform_edges(NODES, 50, r.device)
+    config = BKConfig(RPOINTS=NODES - 1, MAXR=100.0)
+    parent = BKConfig(RPOINTS=NODES - 1, MAXR=100.0, RC_NLO=RunningCouplingNLO.PARENT_NLO)
+    out = {}
+    for seed in SOBOL_SEEDS:
+        table = dev.sobol_table(4, seed)
+        for name, kwargs, cfg in (("full", {}, config), ("sum", {"sum_only": True}, config),
+                                  ("histogram", {"histogram": True}, config), ("parent", {}, parent)):
+            sums = dev.bk_nlo(r, N, t64, t32, edges, table, 1 << 17, cfg, precision="fp64", **kwargs)[0]
+            out[f"{name}_{seed}"] = sums[:, 0].cpu().numpy()
+    ev = dev.BatchEvolver(torch.cat([r, r]), torch.cat([edges, edges]), [NODES, NODES], dev.sobol_table(4, 109), config,
+                          n_samples=1 << 17, precision="fp64", rk_method="euler", step=0.1, k1_rule="fixed")
+    state = torch.cat([N, N])
+    ev.state.copy_(state)
+    ev.step()
+    out["batch_109"] = (ev.state - state).cpu().numpy()
+    return out
+
+
+SECTIONS = {"bk_fp64_sums": bk_sums}
+
+if __name__ == "__main__":
+    for section, values in SECTIONS.items():
+        np.savez_compressed(f"{sys.argv[1]}/{section}.npz", **values())
+        print(section, flush=True)
