@@ -1241,10 +1241,11 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
     T vol = T(1);
     if constexpr (MODE == NLO_PREC_FP32) {
         // B^4 and the table's units: (ln 2)^2 of the log-r widths, 2^2 of the
-        // half-angles, 2^96 of the four widths' 2^-128 (the other 2^32 sits in
-        // Fp32Consts::norm: the product of widths stays in the normal range)
+        // half-angles, 2^92 of the four widths' 2^-128 (the other 2^36 sits in
+        // Fp32Consts::norm).  2e29 at 2 bins, 4e37 at the most, 255: a factor of
+        // 2^96 would leave the FP32 range at 218.
         const double bb = (double)a.bins;
-        vol = (T)((bb * bb) * (bb * bb) * (4.0 * kLn2 * kLn2) * 0x1p96);
+        vol = (T)((bb * bb) * (bb * bb) * (4.0 * kLn2 * kLn2) * 0x1p92);
     } else {
         for (int d = 0; d < 4; ++d) vol = vol * wd[d];
     }
@@ -1264,7 +1265,7 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
         c32.pi = vector_reg(3.14159274f);
         c32.log2_r = (float)(log_rp * kLog2e);
         c32.cut = (float)(1e10 * ((rp * rp) * (rp * rp)));
-        c32.norm = vector_reg((float)(a.c.nc * a.c.nc * a.c.norm * (a.c.symmetrize ? 0.5 : 1.0) * 0x1p32));
+        c32.norm = vector_reg((float)(a.c.nc * a.c.nc * a.c.norm * (a.c.symmetrize ? 0.5 : 1.0) * 0x1p36));
         c32.mirror = vector_reg(a.c.symmetrize ? 1.0f : 0.0f);
         c32.nf_over_nc = vector_reg((float)(a.c.nf / a.c.nc));
         c32.mu = vector_reg((float)a.c.log_mu0 * kLog2ef);
