@@ -722,7 +722,7 @@ struct TMoments {
 // argument's reciprocal, and there are no divisions.  (FP32: the argument's
 // square root is the hardware one; the argument is a product of squared
 // scales, far from the denormal range.)
-template <typename T, bool G11 = true, bool G2 = true>
+template <typename T>
 __device__ __forceinline__ GValues<T> g_values(T num, T den, T iden, T om, T iy, T siy) {
     const T sq = num * den * iy;
     T arg, iarg;
@@ -733,48 +733,40 @@ __device__ __forceinline__ GValues<T> g_values(T num, T den, T iden, T om, T iy,
         iarg = dis_rsqrt(sq);
         arg = sq * iarg;
     }
-    const K01<T> k = bessel_k01<T, G11 || G2, true>(arg);
+    const K01<T> k = bessel_k01(arg);
+    const T k2 = k.k0 + T(2) * k.k1 * iarg;
+    const T nd = num * iden;
     const T ratio = num * siy * iarg;
-    GValues<T> g{T(0), T(0), T(0), T(0)};
-    if constexpr (G11) g.g11 = T(2) * k.k0 * iy;  // y^-1 2 K0
+    GValues<T> g;
+    g.g11 = T(2) * k.k0 * iy;                    // y^-1 2 K0
     g.g12 = T(4) * om * siy * iy * ratio * k.k1;  // y^-3/2 4 omega (num/den)^1/2 K1
-    if constexpr (G2) {
-        const T k2 = k.k0 + T(2) * k.k1 * iarg;
-        const T nd = num * iden;
-        g.g21 = T(4) * siy * ratio * k.k1;  // y^-1/2 4 (num/den)^1/2 K1
-        g.g22 = T(8) * om * iy * nd * k2;   // y^-1 8 omega (num/den) K2
-    }
+    g.g21 = T(4) * siy * ratio * k.k1;           // y^-1/2 4 (num/den)^1/2 K1
+    g.g22 = T(8) * om * iy * nd * k2;            // y^-1 8 omega (num/den) K2
     return g;
 }
 
-// G11: the G11 moments are read (not by the longitudinal I2); G2: so are G21
-// and G22bar (not by the longitudinal terms).
-template <typename T, bool G11 = true, bool G2 = true>
+template <typename T>
 __device__ __forceinline__ TMoments<T> t_moments(const Tripole<T>& v, T m2, T y) {
     const T iy = dis_rcp(y), siy = dis_rsqrt(y);
     const T dj = y * v.x3j2 + v.om_j * v.x2j2, dk = y * v.x3k2 + v.om_k * v.x2k2;
     const T idj = dis_rcp(dj), idk = dis_rcp(dk);
-    const GValues<T> j = g_values<T, G11, G2>(y * v.lam_j * m2 + v.qj2, dj, idj, v.om_j, iy, siy);
-    const GValues<T> j0 = g_values<T, false, G2>(v.qj2, dj, idj, v.om_j, iy, siy);
-    const GValues<T> k = g_values<T, G11, G2>(y * v.lam_k * m2 + v.qk2, dk, idk, v.om_k, iy, siy);
-    const GValues<T> k0 = g_values<T, false, G2>(v.qk2, dk, idk, v.om_k, iy, siy);
+    const GValues<T> j = g_values(y * v.lam_j * m2 + v.qj2, dj, idj, v.om_j, iy, siy);
+    const GValues<T> j0 = g_values(v.qj2, dj, idj, v.om_j, iy, siy);
+    const GValues<T> k = g_values(y * v.lam_k * m2 + v.qk2, dk, idk, v.om_k, iy, siy);
+    const GValues<T> k0 = g_values(v.qk2, dk, idk, v.om_k, iy, siy);
     return {j.g22 - j0.g22, k.g22 - k0.g22, j.g12 - j0.g12, k.g12 - k0.g12, j.g21, k.g21, j.g11, k.g11};
 }
 
-template <typename T, bool G11, bool G2>
+template <typename T>
 __device__ __forceinline__ void t_moments_axpy(TMoments<T>& acc, T w, const TMoments<T>& m) {
+    acc.b22j += w * m.b22j;
+    acc.b22k += w * m.b22k;
     acc.b12j += w * m.b12j;
     acc.b12k += w * m.b12k;
-    if constexpr (G2) {
-        acc.b22j += w * m.b22j;
-        acc.b22k += w * m.b22k;
-        acc.g21j += w * m.g21j;
-        acc.g21k += w * m.g21k;
-    }
-    if constexpr (G11) {
-        acc.g11j += w * m.g11j;
-        acc.g11k += w * m.g11k;
-    }
+    acc.g21j += w * m.g21j;
+    acc.g21k += w * m.g21k;
+    acc.g11j += w * m.g11j;
+    acc.g11k += w * m.g11k;
 }
 
 // Quantities of the transverse tripole that do not depend on the inner y.

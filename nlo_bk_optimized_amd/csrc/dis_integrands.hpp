@@ -154,23 +154,12 @@ __device__ __forceinline__ T qg_finish(const QgPoint<T>& p, T res) {
     return (p.Y >= T(0) && isfinite(res)) ? res : T(0);
 }
 
-// The G-value moments integrated over y_t on the nested inner rule.  The
-// longitudinal terms read a quarter of them (I2: G12bar) or half (I3: G12bar
-// and G11), the same for a whole block, so each has its own loop (F2 of 2 10^6
-// evaluations 15.8 -> 15.2 ms, four points in FP32 19.8 -> 19.4 ms).
-template <typename T, bool G11, bool G2>
-__device__ __forceinline__ TMoments<T> nested_moments_of(const Tripole<T>& v, T m2, const RuleView& rule) {
+// The G-value moments integrated over y_t on the nested inner rule.
+template <typename T>
+__device__ __forceinline__ TMoments<T> nested_moments(const Tripole<T>& v, T m2, const RuleView& rule) {
     TMoments<T> acc{T(0), T(0), T(0), T(0), T(0), T(0), T(0), T(0)};
-    for (int i = 0; i < rule.n; ++i)
-        t_moments_axpy<T, G11, G2>(acc, (T)rule.w[i], t_moments<T, G11, G2>(v, m2, (T)rule.y[i]));
+    for (int i = 0; i < rule.n; ++i) t_moments_axpy(acc, (T)rule.w[i], t_moments<T>(v, m2, (T)rule.y[i]));
     return acc;
-}
-
-// I3: the caller forms I3 (else I2 alone).
-template <typename T, bool I3>
-__device__ __forceinline__ TMoments<T> nested_moments(const DisArgs& a, const Tripole<T>& v, T m2,
-                                                      const RuleView& rule) {
-    return a.transverse ? nested_moments_of<T, true, true>(v, m2, rule) : nested_moments_of<T, I3, false>(v, m2, rule);
 }
 
 template <typename T, int K>
@@ -231,7 +220,7 @@ __device__ __forceinline__ T dis_value(const DisArgs& a, const double* u, const 
             // y_t integrals on the mapped inner rule: I2 is linear and I3
             // bilinear in the G values (K/dis/i2_i3/kernel.cu:768-912)
             const TFixed<T> f = t_fixed<T>(v, m2, z1, z2);
-            const TMoments<T> acc = nested_moments<T, K == NLO_DIS_QG_I3_NESTED>(a, v, m2, rule);
+            const TMoments<T> acc = nested_moments<T>(v, m2, rule);
             if constexpr (K == NLO_DIS_QG_I2_NESTED)
                 res = p.N012 * (a.transverse ? it_qg_i2<T>(v, f, m2, z1, z2, acc) : il_qg_i2<T>(v, f, Q2, z1, z2, acc));
             else
@@ -257,7 +246,7 @@ __device__ __forceinline__ void qg_nested_pair(const DisArgs& a, const double* u
     const Tripole<T> v = tripole_vars<T>(Q2, p.mf, p.z1, p.z2, p.x01sq, p.x02sq, p.x21sq);
     const T m2 = p.m2, z1 = p.z1, z2 = p.z2;
     const TFixed<T> f = t_fixed<T>(v, m2, z1, z2);
-    const TMoments<T> acc = nested_moments<T, true>(a, v, m2, rule);
+    const TMoments<T> acc = nested_moments<T>(v, m2, rule);
     if (a.transverse) {
         i2 = p.N012 * it_qg_i2<T>(v, f, m2, z1, z2, acc);
         i3 = p.N012 * it_qg_i3<T>(v, f, m2, z1, z2, acc, acc);

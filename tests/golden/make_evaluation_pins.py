@@ -17,9 +17,13 @@ import numpy as np
 import torch
 
 from nlo_bk_optimized_amd import device as dev
+from nlo_bk_optimized_amd._lib import DIS_DIMENSIONS
 from nlo_bk_optimized_amd.bk import MV, BKConfig
 from nlo_bk_optimized_amd.bk.config import RunningCouplingNLO
 from nlo_bk_optimized_amd.bk.evolution import uniform_edges
+from nlo_bk_optimized_amd.dipole import GBW
+from nlo_bk_optimized_amd.dis import DISConfig, Polarization, Quark, QuarkType
+from nlo_bk_optimized_amd.dis.fixed_sobol import gbw_qg_fixed_sobol_batch
 
 NODES = 24
 SOBOL_SEEDS = (109, 110, 215, 339)  # each with a sample next to a2 = b2 in some parent
@@ -51,7 +55,38 @@ def bk_sums() -> dict[str, np.ndarray]:
     return out
 
 
-SECTIONS = {"bk_fp64_sums": bk_sums}
+QUARK = Quark(QuarkType.C, 1.4)
+DIPOLE = GBW(Qs0sqr=0.4, lambda_=0.25, gamma=1.0, x0=1.0)
+
+
+def integrand_points(kinds, precision: str) -> dict[str, np.ndarray]:
+    """Integrands at points that crowd towards the lower faces of the cube,
+    where gluons are soft and the terms cancel."""
+
+    out = {}
+    for kind in kinds:
+        gen = torch.Generator().manual_seed(DIS_DIMENSIONS[kind])
+        u = torch.rand((512, DIS_DIMENSIONS[kind]), generator=gen, dtype=torch.float64)
+        u = (u ** (1 + 3 * torch.rand(u.shape, generator=gen, dtype=torch.float64))).cuda()
+        for transverse in (False, True):
+            desc = dev.dis_desc(10.0, 1e-3, transverse, (QUARK,), DIPOLE, DISConfig(quarks=(QUARK,), maxr=5.0))
+            out[f"{kind}_{'T' if transverse else 'L'}"] = dev.dis_integrand(desc, kind, u, precision=precision).cpu().numpy()
+    return out
+
+
+def nested_fp32() -> dict[str, np.ndarray]:
+    """The nested terms in FP32, and the fixed-Sobol estimator that sums them."""
+
+    out = integrand_points(("I2_nested", "I3_nested"), "fp32")
+    q2, x = torch.tensor(10.0, dtype=torch.float32), torch.tensor(1e-3, dtype=torch.float32)
+    entries = [(q2, x, pol, QUARK, 5) for pol in (Polarization.L, Polarization.T)]
+    results = gbw_qg_fixed_sobol_batch(entries, DIPOLE, DISConfig(quarks=(QUARK,), maxr=5.0))
+    rows = [r for f in results for r in (*f.contributions, f.total)]
+    out["estimator"] = torch.stack([torch.stack([r.value, r.error]).double() for r in rows]).cpu().numpy()
+    return out
+
+
+SECTIONS = {"bk_fp64_sums": bk_sums, "nested_fp32": nested_fp32}
 
 if __name__ == "__main__":
     for section, values in SECTIONS.items():
