@@ -7,8 +7,6 @@
 
 #include <hip/hip_runtime.h>
 
-#include <type_traits>
-
 #include "common.hpp"
 #include "fp64_math.hpp"
 #include "nlo_gfx950.h"
@@ -20,70 +18,6 @@ namespace dis {
 
 constexpr double kPiD = 3.14159265358979323846;
 constexpr double kEulerGamma = 0.57721566490153286061;
-
-// ------------------------------------------------------------- arithmetic
-
-// The FP64 path's number: a double whose quotients, logarithms, exponentials
-// and roots are those of fp64_math.hpp.  Same precision, other instructions:
-// the integrands hold up to 100 quotients each.  log(0) is -inf and the log of
-// a negative number NaN, as for double; a quotient by 0 is NaN (each integrand
-// counts a value that is not finite as 0).
-struct Real64 {
-    double v;
-    Real64() = default;
-    template <typename U, std::enable_if_t<std::is_arithmetic<U>::value, int> = 0>
-    __device__ constexpr explicit Real64(U x) : v((double)x) {}
-    __device__ explicit operator double() const { return v; }
-    __device__ friend Real64 operator+(Real64 a, Real64 b) { return Real64(a.v + b.v); }
-    __device__ friend Real64 operator-(Real64 a, Real64 b) { return Real64(a.v - b.v); }
-    __device__ friend Real64 operator-(Real64 a) { return Real64(-a.v); }
-    __device__ friend Real64 operator*(Real64 a, Real64 b) { return Real64(a.v * b.v); }
-    __device__ friend Real64 operator/(Real64 a, Real64 b) {
-        return Real64(__builtin_constant_p(b.v) ? a.v / b.v : div64(a.v, b.v));
-    }
-    __device__ Real64& operator+=(Real64 b) {
-        v += b.v;
-        return *this;
-    }
-    __device__ friend bool operator<(Real64 a, Real64 b) { return a.v < b.v; }
-    __device__ friend bool operator>(Real64 a, Real64 b) { return a.v > b.v; }
-    __device__ friend bool operator<=(Real64 a, Real64 b) { return a.v <= b.v; }
-    __device__ friend bool operator>=(Real64 a, Real64 b) { return a.v >= b.v; }
-    __device__ friend bool operator==(Real64 a, Real64 b) { return a.v == b.v; }
-    __device__ friend bool isfinite(Real64 a) { return ::isfinite(a.v); }
-    __device__ friend Real64 fabs(Real64 a) { return Real64(::fabs(a.v)); }
-    __device__ friend Real64 fmax(Real64 a, Real64 b) { return Real64(::fmax(a.v, b.v)); }
-    __device__ friend Real64 fmin(Real64 a, Real64 b) { return Real64(::fmin(a.v, b.v)); }
-    __device__ friend Real64 exp(Real64 a) { return Real64(exp64(a.v)); }
-    __device__ friend Real64 expm1(Real64 a) { return Real64(::expm1(a.v)); }
-    __device__ friend Real64 pow(Real64 a, Real64 b) { return Real64(::pow(a.v, b.v)); }
-    __device__ friend Real64 log(Real64 a) {
-        const double l = log64(a.v);
-        return Real64(a.v > 0.0 ? l : (a.v == 0.0 ? -INFINITY : NAN));
-    }
-    __device__ friend Real64 log1p(Real64 a) { return Real64(::log1p(a.v)); }
-};
-
-// The arithmetic that an FP64 or FP32 kernel evaluates its integrand in.
-template <typename T>
-using math_t = std::conditional_t<std::is_same<T, double>::value, Real64, T>;
-
-// Reciprocal, square root and its reciprocal: in FP64 those of fp64_math.hpp,
-// in FP32 the hardware approximations (about 1 ulp), where no FP32 result is a
-// small difference of them.  (The correctly rounded FP32 root scales denormal
-// arguments; every FP32 argument here is a product of squared physical scales,
-// zero or far above 1e-38.)
-__device__ __forceinline__ float dis_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ float dis_rsqrt(float x) { return __builtin_amdgcn_rsqf(x); }
-__device__ __forceinline__ float dis_sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
-__device__ __forceinline__ Real64 dis_rcp(Real64 x) { return Real64(rcp64(x.v)); }
-__device__ __forceinline__ Real64 dis_rsqrt(Real64 x) { return Real64(rsqrt64(x.v)); }
-__device__ __forceinline__ Real64 dis_sqrt(Real64 x) { return Real64(sqrt64(x.v)); }
-
-// cos(phi) for phi in [0, 2 pi]: in FP64 1 - 2 sin^2(phi / 2), which needs no
-// range reduction.
-__device__ __forceinline__ float dis_cos(float phi) { return cos(phi); }
-__device__ __forceinline__ Real64 dis_cos(Real64 phi) { return Real64(fma(-2.0, sin2_64(0.5 * phi.v), 1.0)); }
 
 // ------------------------------------------------------------ special functions
 
@@ -98,10 +32,40 @@ struct K01 {
 //   K1 = 1/x + (x/2)(ln(x/2) + gamma) sum t^k/(k!(k+1)!) - (x/4) sum (H_k + H_{k+1}) t^k/(k!(k+1)!),
 // the four sums as polynomials in t (15 terms FP64, 8 FP32) by Horner's rule;
 // x > 2: K = e^-x / sqrt(x) * sum c_m T_m(4/x - 1) (Chebyshev fit of the
-// scaled function, coefficients from gen_bessel_tables.py, in the power basis
-// by Horner's rule: in FP64 the error of Clenshaw's, 1.0 eps, in half the
-// operations).  FP32 takes 1/x, 1/sqrt(x) and ln from the hardware
-// approximations.  NU0, NU1: the orders that the caller reads.
+// scaled function, coefficients from gen_bessel_tables.py; Clenshaw in FP64,
+// the power-basis form by Horner in FP32).  FP32 takes 1/x, 1/sqrt(x) and ln
+// from the hardware approximations.  FP64 keeps the library's functions and IEEE
+// operations: the ab, T1 and qqbar-g terms are small differences of these
+// values, by up to ten digits in some samples, and another rounding of any of
+// them moves an integral by up to 4e-9.  NU0, NU1: the orders the caller reads.
+// Reciprocal, reciprocal square root and natural log: IEEE operations in
+// FP64; in FP32 the hardware approximations (about 1 ulp; the log with an
+// absolute error ~1e-7), where no FP32 result is a small difference of them.
+template <typename T>
+__device__ __forceinline__ T dis_rcp(T x) {
+    if constexpr (sizeof(T) == 4)
+        return __builtin_amdgcn_rcpf(x);
+    else
+        return T(1) / x;
+}
+template <typename T>
+__device__ __forceinline__ T dis_rsqrt(T x) {
+    if constexpr (sizeof(T) == 4)
+        return __builtin_amdgcn_rsqf(x);
+    else
+        return T(1) / sqrt(x);
+}
+// Square root: IEEE in FP64; in FP32 the hardware one (about 1 ulp, without
+// the correctly rounded expansion's denormal scaling: every FP32 argument here
+// is a product of squared physical scales, zero or far above 1e-38).
+template <typename T>
+__device__ __forceinline__ T dis_sqrt(T x) {
+    if constexpr (sizeof(T) == 4)
+        return __builtin_amdgcn_sqrtf(x);
+    else
+        return sqrt(x);
+}
+
 template <typename T, bool NU0 = true, bool NU1 = true>
 __device__ __forceinline__ K01<T> bessel_k01(T x) {
     constexpr bool f64 = sizeof(T) == 8;
@@ -111,37 +75,34 @@ __device__ __forceinline__ K01<T> bessel_k01(T x) {
     }
     if (x <= T(2)) {
         const T t = T(0.25) * x * x;
+        T i0, s0, i1, s1;
         if constexpr (f64) {
             // the four series as polynomials in t by Horner's rule, their 60
-            // coefficients in scalar registers as they are used
+            // coefficients in scalar registers as they are used (a rolled loop
+            // waits for them: single passes of 2^20 samples 852 -> 702 us)
             constexpr int n = kBesselSeriesTerms64;
-            const double td = t.v;
-            double p0 = 0.0, q0 = 0.0, p1 = 0.0, q1 = 0.0;
-            p0 = coef64(kBesselSeriesI0_64[n - 1]), p1 = coef64(kBesselSeriesI1_64[n - 1]);
-            if constexpr (NU0) q0 = coef64(kBesselSeriesS0_64[n - 1]);
-            if constexpr (NU1) q1 = coef64(kBesselSeriesS1_64[n - 1]);
+            i0 = s0 = i1 = s1 = T(0);
+            if constexpr (NU0) i0 = coef64(kBesselSeriesI0_64[n - 1]), s0 = coef64(kBesselSeriesS0_64[n - 1]);
+            if constexpr (NU1) i1 = coef64(kBesselSeriesI1_64[n - 1]), s1 = coef64(kBesselSeriesS1_64[n - 1]);
 #pragma unroll
             for (int k = n - 2; k >= 0; --k) {
                 if constexpr (NU0) {
-                    p0 = fma(p0, td, coef64(kBesselSeriesI0_64[k]));
-                    q0 = fma(q0, td, coef64(kBesselSeriesS0_64[k]));
+                    i0 = fma(i0, t, coef64(kBesselSeriesI0_64[k]));
+                    s0 = fma(s0, t, coef64(kBesselSeriesS0_64[k]));
                 }
                 if constexpr (NU1) {
-                    p1 = fma(p1, td, coef64(kBesselSeriesI1_64[k]));
-                    q1 = fma(q1, td, coef64(kBesselSeriesS1_64[k]));
+                    i1 = fma(i1, t, coef64(kBesselSeriesI1_64[k]));
+                    s1 = fma(s1, t, coef64(kBesselSeriesS1_64[k]));
                 }
             }
-            const double lg = log64(0.5 * x.v) + kEulerGamma;
-            K01<T> out{T(0), T(0)};
-            if constexpr (NU0) out.k0 = T(q0 - lg * p0);
-            if constexpr (NU1) out.k1 = T(1.0 / x.v + 0.5 * x.v * lg * p1 - 0.25 * x.v * q1);
-            return out;
+            const T lg = log(T(0.5) * x) + T(kEulerGamma);
+            return {NU0 ? s0 - lg * i0 : T(0), NU1 ? T(1) / x + T(0.5) * x * lg * i1 - T(0.25) * x * s1 : T(0)};
         } else {
             // the four series as polynomials in t (Horner, exact rational
             // coefficients rounded once; every term is positive)
             constexpr int n = kBesselSeriesTerms32;
-            float i0 = kBesselSeriesI0_32[n - 1], s0 = kBesselSeriesS0_32[n - 1];
-            float i1 = kBesselSeriesI1_32[n - 1], s1 = kBesselSeriesS1_32[n - 1];
+            i0 = kBesselSeriesI0_32[n - 1], s0 = kBesselSeriesS0_32[n - 1];
+            i1 = kBesselSeriesI1_32[n - 1], s1 = kBesselSeriesS1_32[n - 1];
 #pragma unroll
             for (int k = n - 2; k >= 0; --k) {
                 i0 = fmaf(i0, t, kBesselSeriesI0_32[k]);
@@ -153,26 +114,30 @@ __device__ __forceinline__ K01<T> bessel_k01(T x) {
             return {s0 - lg * i0, dis_rcp(x) + T(0.5) * x * lg * i1 - T(0.25) * x * s1};
         }
     }
+    const T s = (f64 ? T(4) / x : T(4) * dis_rcp(x)) - T(1);
     if constexpr (f64) {
-        const double xs = ::fmin(x.v, 1e4);  // e^-1e4 is 0
-        const double s = fma(4.0, rcp64(xs), -1.0);
-        K01<T> out{T(0), T(0)};
-        const double sc = exp64(-xs) * rsqrt64(xs);
-        if constexpr (NU0) {
-            double g = coef64(kBesselK0Mono64[kBesselK0Deg64]);
+        const T s2 = s + s;
+        T b0k0 = T(0), b1k0 = T(0), b0k1 = T(0), b1k1 = T(0);
 #pragma unroll
-            for (int m = kBesselK0Deg64 - 1; m >= 0; --m) g = fma(g, s, coef64(kBesselK0Mono64[m]));
-            out.k0 = T(g * sc);
+        for (int m = kBesselK0Deg64; m >= 1; --m) {
+            if constexpr (NU0) {
+                const T t0 = s2 * b0k0 - b1k0 + coef64(kBesselK0Cheb64[m]);
+                b1k0 = b0k0;
+                b0k0 = t0;
+            }
+            if constexpr (NU1) {
+                const T t1 = s2 * b0k1 - b1k1 + coef64(kBesselK1Cheb64[m]);
+                b1k1 = b0k1;
+                b0k1 = t1;
+            }
         }
-        if constexpr (NU1) {
-            double g = coef64(kBesselK1Mono64[kBesselK1Deg64]);
-#pragma unroll
-            for (int m = kBesselK1Deg64 - 1; m >= 0; --m) g = fma(g, s, coef64(kBesselK1Mono64[m]));
-            out.k1 = T(g * sc);
-        }
-        return out;
+        T g0 = T(0), g1 = T(0);
+        if constexpr (NU0) g0 = s * b0k0 - b1k0 + coef64(kBesselK0Cheb64[0]);
+        if constexpr (NU1) g1 = s * b0k1 - b1k1 + coef64(kBesselK1Cheb64[0]);
+        const T sc = exp(-x) / dis_sqrt(x);
+        return {g0 * sc, g1 * sc};
     } else {
-        const T s = T(4) * dis_rcp(x) - T(1);
+        // the degree-8 interpolant in the power basis of s (Horner)
         T g0 = kBesselK0Mono32[kBesselK0Deg32], g1 = kBesselK1Mono32[kBesselK1Deg32];
 #pragma unroll
         for (int m = kBesselK0Deg32 - 1; m >= 0; --m) {
@@ -243,14 +208,7 @@ __device__ __forceinline__ T dis_alpha(T r, const DisCoupling& c) {
         const T mu0 = T(2.0 / 0.2 * 0.91629073187415506518);  // 10 ln 2.5
         const T ls = log(arg) / T(0.2);
         const T hi = fmax(mu0, ls);
-        if constexpr (sizeof(T) == 8) {
-            // e^(mu0 - ls) = (2.5^2 / arg)^5; beyond 1e18 the term rounds away
-            const double v = 6.25 * rcp64(arg.v), v2 = v * v, u = v2 * v2 * v;
-            const double term = u > 1e-18 && u < 1e18 ? log1p_fold64(u) : 0.0;
-            return dis_rcp(T(c.b0) * T(0.2) * (hi + T(term)));
-        } else {
-            return T(1) / (T(c.b0) * T(0.2) * (hi + log1p(exp(-fabs(mu0 - ls)))));
-        }
+        return T(1) / (T(c.b0) * T(0.2) * (hi + log1p(exp(-fabs(mu0 - ls)))));
     }
     const T a = T(1) / (T(c.b0) * log(arg));
     return (a > T(c.max_alpha) || arg < T(1)) ? T(c.max_alpha) : a;
@@ -710,6 +668,23 @@ struct GValues {
     T g11, g12, g21, g22;
 };
 
+template <typename T>
+__device__ __forceinline__ GValues<T> g_values(T q2, T m2, T x22, T x32, T om, T lam, T y) {
+    const T num = y * lam * m2 + q2;
+    const T den = y * x32 + om * x22;
+    const T arg = dis_sqrt(num * den / y);
+    const K01<T> k = bessel_k01(arg);
+    const T k2 = k.k0 + T(2) * k.k1 / arg;
+    const T ratio = dis_sqrt(num / den);
+    const T iy = T(1) / y;
+    GValues<T> g;
+    g.g11 = T(2) * k.k0 * iy;                      // y^-1 2 K0
+    g.g12 = T(4) * om * dis_sqrt(iy) * iy * ratio * k.k1;  // y^-3/2 4 omega (num/den)^1/2 K1
+    g.g21 = T(4) * dis_sqrt(iy) * ratio * k.k1;         // y^-1/2 4 (num/den)^1/2 K1
+    g.g22 = T(8) * om * iy * (num / den) * k2;       // y^-1 8 omega (num/den) K2
+    return g;
+}
+
 // The eight transverse (four longitudinal) G moments at one inner y:
 // G22bar, G12bar (lam minus lam = 0), G21, G11, for the j and k legs.
 template <typename T>
@@ -717,44 +692,45 @@ struct TMoments {
     T b22j, b22k, b12j, b12k, g21j, g21k, g11j, g11k;
 };
 
-// 1/y, 1/sqrt(y) and 1/den are shared by the lam and lam = 0 evaluations of a
-// leg (den does not depend on lam), (num/den)^1/2 = num y^-1/2 / arg reuses the
-// argument's reciprocal, and there are no divisions.  (FP32: the argument's
-// square root is the hardware one; the argument is a product of squared
-// scales, far from the denormal range.)
-template <typename T>
-__device__ __forceinline__ GValues<T> g_values(T num, T den, T iden, T om, T iy, T siy) {
-    const T sq = num * den * iy;
-    T arg, iarg;
-    if constexpr (sizeof(T) == 4) {
-        arg = dis_sqrt(sq);
-        iarg = dis_rcp(arg);
-    } else {
-        iarg = dis_rsqrt(sq);
-        arg = sq * iarg;
-    }
-    const K01<T> k = bessel_k01(arg);
-    const T k2 = k.k0 + T(2) * k.k1 * iarg;
-    const T nd = num * iden;
-    const T ratio = num * siy * iarg;
-    GValues<T> g;
-    g.g11 = T(2) * k.k0 * iy;                    // y^-1 2 K0
-    g.g12 = T(4) * om * siy * iy * ratio * k.k1;  // y^-3/2 4 omega (num/den)^1/2 K1
-    g.g21 = T(4) * siy * ratio * k.k1;           // y^-1/2 4 (num/den)^1/2 K1
-    g.g22 = T(8) * om * iy * nd * k2;            // y^-1 8 omega (num/den) K2
+// FP32: g_values with 1/y, 1/sqrt(y) and 1/den shared by the lam and lam = 0
+// evaluations of a leg and no divisions (den does not depend on lam).
+// The argument's square root is the hardware one (about 1 ulp; the argument is
+// a product of squared scales, far from the denormal range) and
+// (num/den)^1/2 = num y^-1/2 / arg reuses its reciprocal.
+__device__ __forceinline__ GValues<float> g_values_f32(float num, float den, float iden, float om, float iy,
+                                                       float siy) {
+    const float arg = __builtin_amdgcn_sqrtf(num * den * iy);
+    const K01<float> k = bessel_k01(arg);
+    const float iarg = dis_rcp(arg);
+    const float k2 = k.k0 + 2.0f * k.k1 * iarg;
+    const float nd = num * iden;
+    const float ratio = num * siy * iarg;
+    GValues<float> g;
+    g.g11 = 2.0f * k.k0 * iy;
+    g.g12 = 4.0f * om * siy * iy * ratio * k.k1;
+    g.g21 = 4.0f * siy * ratio * k.k1;
+    g.g22 = 8.0f * om * iy * nd * k2;
     return g;
 }
 
 template <typename T>
 __device__ __forceinline__ TMoments<T> t_moments(const Tripole<T>& v, T m2, T y) {
-    const T iy = dis_rcp(y), siy = dis_rsqrt(y);
-    const T dj = y * v.x3j2 + v.om_j * v.x2j2, dk = y * v.x3k2 + v.om_k * v.x2k2;
-    const T idj = dis_rcp(dj), idk = dis_rcp(dk);
-    const GValues<T> j = g_values(y * v.lam_j * m2 + v.qj2, dj, idj, v.om_j, iy, siy);
-    const GValues<T> j0 = g_values(v.qj2, dj, idj, v.om_j, iy, siy);
-    const GValues<T> k = g_values(y * v.lam_k * m2 + v.qk2, dk, idk, v.om_k, iy, siy);
-    const GValues<T> k0 = g_values(v.qk2, dk, idk, v.om_k, iy, siy);
-    return {j.g22 - j0.g22, k.g22 - k0.g22, j.g12 - j0.g12, k.g12 - k0.g12, j.g21, k.g21, j.g11, k.g11};
+    if constexpr (sizeof(T) == 4) {
+        const float iy = dis_rcp(y), siy = dis_rsqrt(y);
+        const float dj = y * v.x3j2 + v.om_j * v.x2j2, dk = y * v.x3k2 + v.om_k * v.x2k2;
+        const float idj = dis_rcp(dj), idk = dis_rcp(dk);
+        const GValues<float> j = g_values_f32(y * v.lam_j * m2 + v.qj2, dj, idj, v.om_j, iy, siy);
+        const GValues<float> j0 = g_values_f32(v.qj2, dj, idj, v.om_j, iy, siy);
+        const GValues<float> k = g_values_f32(y * v.lam_k * m2 + v.qk2, dk, idk, v.om_k, iy, siy);
+        const GValues<float> k0 = g_values_f32(v.qk2, dk, idk, v.om_k, iy, siy);
+        return {j.g22 - j0.g22, k.g22 - k0.g22, j.g12 - j0.g12, k.g12 - k0.g12, j.g21, k.g21, j.g11, k.g11};
+    } else {
+        const GValues<T> j = g_values(v.qj2, m2, v.x2j2, v.x3j2, v.om_j, v.lam_j, y);
+        const GValues<T> j0 = g_values(v.qj2, m2, v.x2j2, v.x3j2, v.om_j, T(0), y);
+        const GValues<T> k = g_values(v.qk2, m2, v.x2k2, v.x3k2, v.om_k, v.lam_k, y);
+        const GValues<T> k0 = g_values(v.qk2, m2, v.x2k2, v.x3k2, v.om_k, T(0), y);
+        return {j.g22 - j0.g22, k.g22 - k0.g22, j.g12 - j0.g12, k.g12 - k0.g12, j.g21, k.g21, j.g11, k.g11};
+    }
 }
 
 template <typename T>

@@ -250,10 +250,10 @@ __device__ __forceinline__ void fs_pass(const FsDev& f, int item, int k, int blk
         double x[NK];
         if (valid) {
             if constexpr (PART == kFsI1) {
-                x[0] = (double)dis_value<Real64, NLO_DIS_QG_I1>(a, ud, rule) * w;
+                x[0] = (double)dis_value<double, NLO_DIS_QG_I1>(a, ud, rule) * w;
             } else {
-                math_t<T> i2, i3;
-                qg_nested_pair<math_t<T>>(a, ud, rule, i2, i3);
+                T i2, i3;
+                qg_nested_pair<T>(a, ud, rule, i2, i3);
                 x[0] = (double)i2 * w;
                 x[1] = (double)i3 * w;
             }

@@ -133,7 +133,7 @@ __device__ __forceinline__ QgPoint<T> qg_point(const DisArgs& a, const double* u
     const T phi = (T)(2.0 * kPiD * u[4]);
     p.x01sq = p.x01 * p.x01;
     p.x02sq = p.x02 * p.x02;
-    p.x21sq = fmax(p.x01sq + p.x02sq - T(2) * p.x01 * p.x02 * dis_cos(phi), T(0));
+    p.x21sq = fmax(p.x01sq + p.x02sq - T(2) * p.x01 * p.x02 * cos(phi), T(0));
     const T x21 = dis_sqrt(p.x21sq);
     const T maxr = (T)a.maxr;
     p.jac = (T(1) - z2min) * (T(1) - p.z1 - z2min) * p.x01 * p.x02 * maxr * maxr * T(2.0 * kPiD);

@@ -29,13 +29,12 @@ __global__ void __launch_bounds__(256) special_kernel(int fn, int64_t n, const d
                                                       double* __restrict__ out) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    using M = math_t<T>;
-    const M v = (M)x[i];
-    M r;
-    if (fn == NLO_FN_K0) r = bessel_k0<M>(v);
-    else if (fn == NLO_FN_K1) r = bessel_k1<M>(v);
-    else if (fn == NLO_FN_K2) r = bessel_k2<M>(v);
-    else r = dilog<M>(v);
+    const T v = (T)x[i];
+    T r;
+    if (fn == NLO_FN_K0) r = bessel_k0<T>(v);
+    else if (fn == NLO_FN_K1) r = bessel_k1<T>(v);
+    else if (fn == NLO_FN_K2) r = bessel_k2<T>(v);
+    else r = dilog<T>(v);
     out[i] = (double)r;
 }
 
@@ -43,7 +42,7 @@ __global__ void __launch_bounds__(256) dipole_kernel(DisDipole d, int64_t n, con
                                                      const double* __restrict__ Y, double* __restrict__ out) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    out[i] = (double)dipole_amplitude<Real64>(Real64(r[i]), Real64(Y[i]), d);
+    out[i] = dipole_amplitude<double>(r[i], Y[i], d);
 }
 
 // One block (64 lanes): N at the (moved) table nodes through the local-spline
@@ -143,7 +142,7 @@ __global__ void __launch_bounds__(256) integrand_kernel(DisArgs a, int64_t n, co
     double u[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) u[d] = x[i * D + d];
-    out[i] = (double)dis_value<math_t<T>, K>(a, u, rule);
+    out[i] = (double)dis_value<T, K>(a, u, rule);
 }
 
 // The nested I2 and I3 at each point from one pass over the inner rule.
@@ -157,8 +156,8 @@ __global__ void __launch_bounds__(256) i23_kernel(DisArgs a, int64_t n, const do
     double u[5];
 #pragma unroll
     for (int d = 0; d < 5; ++d) u[d] = x[i * 5 + d];
-    math_t<T> v2, v3;
-    qg_nested_pair<math_t<T>>(a, u, rule, v2, v3);
+    T v2, v3;
+    qg_nested_pair<T>(a, u, rule, v2, v3);
     i2[i] = (double)v2;
     i3[i] = (double)v3;
 }
@@ -324,7 +323,7 @@ __device__ __forceinline__ void vegas_pass(const DisArgs& a, const VegasView& v,
         }
         double wv = 0.0;
         if (valid) {
-            wv = (double)dis_value<math_t<T>, K>(a, u, rule) * jac;
+            wv = (double)dis_value<T, K>(a, u, rule) * jac;
             comp_add(s1, c1, wv);
             comp_add(s2, c2, wv * wv);
         }
@@ -446,7 +445,7 @@ __device__ __forceinline__ void gl_pass(const DisArgs& a, int points, int blk, d
     for (int idx = threadIdx.x; idx < n * n; idx += blockDim.x) {
         const int i = idx / n, j = idx - i * n;
         const double u[2] = {gx[i], gx[j]};
-        comp_add(s[0], e[0], gw[i] * gw[j] * (double)dis_value<math_t<T>, K>(a, u, none));
+        comp_add(s[0], e[0], gw[i] * gw[j] * (double)dis_value<T, K>(a, u, none));
     }
     block_comp_sums<1>(s, e, red, out + blk);
 }

@@ -107,13 +107,13 @@ def main() -> None:
     mp.mp.dps = 40
     lines = [
         "// Generated by gen_bessel_tables.py: g_nu(s) = e^x sqrt(x) K_nu(x), s = 4/x - 1,",
-        "// for x > 2, interpolated at Chebyshev nodes, in the power basis of s (Horner).",
+        "// for x > 2 (FP64: Chebyshev coefficients, sum c_m T_m(s); FP32: power basis).",
     ]
     for nu in (0, 1):
-        mono = monomial(chebyshev(nu, DEG64))
-        body = ",\n    ".join(mp.nstr(v, 21, min_fixed=-1, max_fixed=-1) for v in mono)
+        c = chebyshev(nu, DEG64)
+        body = ",\n    ".join(mp.nstr(v, 21, min_fixed=-1, max_fixed=-1) for v in c)
         lines.append(f"constexpr int kBesselK{nu}Deg64 = {DEG64};")
-        lines.append(f"__device__ constexpr double kBesselK{nu}Mono64[{DEG64 + 1}] = {{\n    {body}}};")
+        lines.append(f"__device__ constexpr double kBesselK{nu}Cheb64[{DEG64 + 1}] = {{\n    {body}}};")
     # FP32, x > 2: the degree-7 interpolant in the monomial basis of s
     # (Horner: one fma per degree; float32 evaluation error 1.0e-7)
     for nu in (0, 1):

@@ -86,7 +86,11 @@ def nested_fp32() -> dict[str, np.ndarray]:
     return out
 
 
-SECTIONS = {"bk_fp64_sums": bk_sums, "nested_fp32": nested_fp32}
+def dis_fp64() -> dict[str, np.ndarray]:
+    return integrand_points(DIS_DIMENSIONS, "fp64")
+
+
+SECTIONS = {"bk_fp64_sums": bk_sums, "nested_fp32": nested_fp32, "dis_fp64": dis_fp64}
 
 if __name__ == "__main__":
     for section, values in SECTIONS.items():

@@ -39,3 +39,10 @@ def test_nested_terms_in_fp32():
     # replicates; another rounding of the FP32 samples gives 4e-7 here and up to 1e-4 elsewhere
     error = np.abs(got["estimator"] / want["estimator"] - 1)
     assert error.max() < 1e-9, error
+
+
+def test_dis_integrands_in_fp64():
+    want, got = recorded("dis_fp64"), pins.dis_fp64()
+    assert want.keys() == got.keys()
+    for name in want:
+        assert np.array_equal(got[name], want[name]), name
