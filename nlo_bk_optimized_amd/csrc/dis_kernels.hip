@@ -213,6 +213,8 @@ struct VegasView {
     double* part_hist;    // blocks x D x bins
     double* part_cnt;
     const double* rule;   // the nested rule (2 x kMaxNested), or null: made here
+    double* stage_w;      // |w| and packed bins per sample, for a histogram by another
+    uint64_t* stage_b;    // kernel; null: the block forms it
 };
 
 struct ArgsSobol {  // a single pass: the table in the kernel arguments
@@ -229,6 +231,41 @@ struct TableSobol {  // a batch item: one of the batch's tables in device memory
     __device__ uint32_t first(int d) const { return t->first[d]; }
 };
 
+// The histogram of one block of samples, `per` per thread, sample j of a thread
+// from load(j, w, pk) (false: none), into hist and cnt (D x bins each).  The
+// block's largest |w| sets a fixed-point scale; the integer LDS sums are exact
+// and independent of the order of the atomics.  hh and hc: zeroed LDS cells.
+template <int D, typename Load>
+__device__ __forceinline__ void block_histogram(int bins, int per, const Load& load, unsigned long long* hh,
+                                                unsigned int* hc, double* hist, double* cnt) {
+    __shared__ double wmax[4];
+    double mx = 0.0, w = 0.0;
+    uint64_t pk = 0;
+    for (int j = 0; j < per; ++j)
+        if (load(j, w, pk)) mx = fmax(mx, w);
+    mx = wave_max(mx);
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    mx = fmax(fmax(wmax[0], wmax[1]), fmax(wmax[2], wmax[3]));
+    const int e = mx > 0.0 ? ilogb(mx) : 0;
+    const int sc = 50 - e;  // each term < 2^51; <= 2^12 terms per bin stay below 2^63
+    for (int j = 0; j < per; ++j) {
+        if (!load(j, w, pk)) continue;
+        const unsigned long long q = (unsigned long long)rint(ldexp(w, sc));
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            const int b = (int)((pk >> (8 * d)) & 0xff);
+            atomicAdd(&hh[d * bins + b], q);
+            atomicAdd(&hc[d * bins + b], 1u);
+        }
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < D * bins; k += blockDim.x) {
+        hist[k] = ldexp((double)hh[k], -sc);
+        cnt[k] = (double)hc[k];
+    }
+}
+
 // One block of a VEGAS pass.  Sobol point index = first + s with
 // s = ((blk * 4 + wave) * spt + j) * 64 + lane: each wave walks spt
 // consecutive 64-point groups; the high part of the gray code (direction
@@ -238,12 +275,12 @@ __device__ __forceinline__ void vegas_pass(const DisArgs& a, const VegasView& v,
     constexpr int D = kDims[K];
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ double red[4][2][2];  // [wave][sum][value, error]
-    __shared__ double wmax[4];
     __shared__ double ry[kMaxNested], rw[kMaxNested];
     RuleView rule{0, ry, rw};
     if constexpr (K == NLO_DIS_QG_I2_NESTED || K == NLO_DIS_QG_I3_NESTED)
         rule = v.rule ? load_nested_rule(a.nested_points, v.rule, ry, rw) : stage_nested_rule(a.nested_points, ry, rw);
-    const VegasLayout lay = vegas_layout(D, v.bins, v.spt, HIST);
+    const bool staged = HIST && v.stage_w;
+    const VegasLayout lay = vegas_layout(D, v.bins, v.spt, HIST && !staged);
     double* E = reinterpret_cast<double*>(smem + lay.edges);
     uint32_t* dir = reinterpret_cast<uint32_t*>(smem + lay.dir);
     for (int i = threadIdx.x; i < D * (v.bins + 1); i += blockDim.x) E[i] = v.edges[i];
@@ -252,7 +289,7 @@ __device__ __forceinline__ void vegas_pass(const DisArgs& a, const VegasView& v,
     unsigned int* hc = nullptr;
     double* st_w = nullptr;
     uint64_t* st_b = nullptr;
-    if (HIST) {
+    if (HIST && !staged) {
         hh = reinterpret_cast<unsigned long long*>(smem + lay.hist);
         hc = reinterpret_cast<unsigned int*>(smem + lay.cnt);
         st_w = reinterpret_cast<double*>(smem + lay.absw);
@@ -327,7 +364,12 @@ __device__ __forceinline__ void vegas_pass(const DisArgs& a, const VegasView& v,
             comp_add(s1, c1, wv);
             comp_add(s2, c2, wv * wv);
         }
-        if (HIST) {
+        if (staged) {
+            if (valid) {
+                v.stage_w[sample] = fabs(wv);
+                v.stage_b[sample] = packed;
+            }
+        } else if (HIST) {
             st_w[threadIdx.x + j * 256] = valid ? fabs(wv) : 0.0;
             st_b[threadIdx.x + j * 256] = valid ? packed : ~0ull;
         }
@@ -336,40 +378,22 @@ __device__ __forceinline__ void vegas_pass(const DisArgs& a, const VegasView& v,
         double t[2] = {s1, s2}, e[2] = {c1, c2};
         block_comp_sums<2>(t, e, red, v.part + (size_t)blk * 2);
     }
-    if (HIST) {
-        // block max of |w| sets a fixed-point scale; the integer LDS sums are
-        // exact and independent of the order of the atomics
-        double mx = 0.0;
-        for (int j = 0; j < v.spt; ++j) mx = fmax(mx, st_w[threadIdx.x + j * 256]);
-        mx = wave_max(mx);
-        if (lane == 0) wmax[wave] = mx;
-        __syncthreads();
-        mx = fmax(fmax(wmax[0], wmax[1]), fmax(wmax[2], wmax[3]));
-        const int e = mx > 0.0 ? ilogb(mx) : 0;
-        const int sc = 50 - e;  // each term < 2^51; <= 2^12 terms per bin stay below 2^63
-        for (int j = 0; j < v.spt; ++j) {
-            const uint64_t pk = st_b[threadIdx.x + j * 256];
-            if (pk == ~0ull) continue;
-            const unsigned long long q = (unsigned long long)rint(ldexp(st_w[threadIdx.x + j * 256], sc));
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                const int b = (int)((pk >> (8 * d)) & 0xff);
-                atomicAdd(&hh[d * v.bins + b], q);
-                atomicAdd(&hc[d * v.bins + b], 1u);
-            }
-        }
-        __syncthreads();
-        for (int k = threadIdx.x; k < D * v.bins; k += blockDim.x) {
-            v.part_hist[(size_t)blk * D * v.bins + k] = ldexp((double)hh[k], -sc);
-            v.part_cnt[(size_t)blk * D * v.bins + k] = (double)hc[k];
-        }
+    if (HIST && !staged) {
+        const auto load = [&](int j, double& w, uint64_t& pk) {
+            w = st_w[threadIdx.x + j * 256];
+            pk = st_b[threadIdx.x + j * 256];
+            return pk != ~0ull;
+        };
+        block_histogram<D>(v.bins, v.spt, load, hh, hc, v.part_hist + (size_t)blk * D * v.bins,
+                           v.part_cnt + (size_t)blk * D * v.bins);
     }
 }
 
 // One VEGAS pass (see nlo_dis_vegas).
 template <typename T, int K, bool HIST>
 __global__ void __launch_bounds__(256) vegas_kernel(DisArgs a, VegasArgs v) {
-    const VegasView view{v.bins, v.spt, v.n, v.first, v.edges, v.part, v.part_hist, v.part_cnt, nullptr};
+    const VegasView view{v.bins, v.spt, v.n, v.first, v.edges, v.part, v.part_hist, v.part_cnt, nullptr,
+                         nullptr, nullptr};
     vegas_pass<T, K, HIST>(a, view, ArgsSobol{v}, blockIdx.x);
 }
 
@@ -471,12 +495,18 @@ constexpr int kBatchMaxIterations = 16;
 // whose blocks would not reach kBatchBlocks: an iteration of a point budget of
 // 2^18 evaluations is 2^15 samples or fewer, 16 blocks of 8 groups on 256
 // CUs.  By the integral's own samples alone, so that its result does not
-// depend on what shares its batch.  One point on a table in FP64 / four points
-// in FP32 / F2 of 2 10^6 evaluations: always 8 groups 11.1 / 23.0 / 18.4 ms;
-// 256 blocks 7.8 / 21.8 / 16.9, 512 6.6 / 20.3 / 16.3, 1024 6.8 / 20.6 / 16.2,
-// 2048 7.1 / 22.2 / 16.4 (a block's fixed work, mostly its grid and histogram).
+// depend on what shares its batch.  A histogram always covers a tile of 2048
+// samples, a block of 8 groups: its fixed-point scale is the tile's largest
+// sample, and another partition would round the refined edges otherwise, which
+// the cancelling samples carry into the integral (up to 2e-9).  Smaller blocks
+// therefore stage their samples and vegas_batch_tiles_kernel forms the tiles.
+// One point on a table in FP64 / four points in FP32 / F2 of 2 10^6
+// evaluations: always 8 groups 11.5 / 22.8 / 17.4 ms, this rule 6.7 / 21.1 /
+// 16.5.  (512: the best of 256 to 2048, by 3 to 18 % for the one point, when each
+// block still formed its histogram.)
 constexpr int kBatchMaxSpt = 8;
 constexpr int kBatchBlocks = 512;
+constexpr int kTile = 256 * kBatchMaxSpt;
 
 int batch_spt(int64_t n) {
     const int64_t g64 = (n + 63) / 64;
@@ -488,12 +518,14 @@ int batch_spt(int64_t n) {
 // One VEGAS integral of a batch: its item, plan and where its data live.
 struct VItem {
     int item, K, D, table;
-    int spt, blocks, groups, per_group;
+    int spt, blocks, tiles, groups, per_group;
     int max_it, min_it;
     int64_t n, stride, first;
     int64_t part;   // doubles into the partial buffer: blocks x 2 sums, then the
-                    // per-block histogram and counts (2 x blocks x cells), then
+                    // per-tile histogram and counts (2 x tiles x cells), then
                     // the group histogram and counts (2 x groups x cells)
+    int64_t stage;  // doubles into the partial buffer: |w| and packed bins per
+                    // sample (2 x tiles x kTile), or -1 (a block is a tile)
     int64_t grid;   // doubles into the grid buffer: edges (2 buffers of
                     // D x (bins + 1)), histogram, counts (cells each), sums (2)
     int64_t rule;   // doubles into the grid buffer: the nested rule, or -1
@@ -510,8 +542,8 @@ __host__ __device__ inline int64_t vgrid_doubles(int D, int bins) {
     return 2 * (int64_t)D * (bins + 1) + 2 * (int64_t)D * bins + 2;
 }
 
-__host__ __device__ inline int64_t vpart_doubles(int blocks, int groups, int cells) {
-    return 2 * (int64_t)blocks + 2 * (int64_t)blocks * cells + 2 * (int64_t)groups * cells;
+__host__ __device__ inline int64_t vpart_doubles(int blocks, int tiles, int groups, int cells) {
+    return 2 * (int64_t)blocks + 2 * (int64_t)tiles * cells + 2 * (int64_t)groups * cells;
 }
 
 struct BatchDev {
@@ -547,14 +579,52 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kDisWa
     const double* edges = b.grid + it.grid + (int64_t)(st.iters & 1) * it.D * (b.bins + 1);
     double* part = b.part + it.part;
     double* ph = part + 2 * (int64_t)it.blocks;
+    double* stage = it.stage < 0 ? nullptr : b.part + it.stage;
     const VegasView view{b.bins, it.spt, it.n, it.first + (int64_t)st.iters * it.stride, edges, part, ph,
-                         ph + (int64_t)it.blocks * cells, it.rule < 0 ? nullptr : b.grid + it.rule};
+                         ph + (int64_t)it.tiles * cells, it.rule < 0 ? nullptr : b.grid + it.rule, stage,
+                         stage ? reinterpret_cast<uint64_t*>(stage + (int64_t)it.tiles * kTile) : nullptr};
     vegas_pass<T, K, true>(b.args[it.item], view, TableSobol{b.tables + it.table}, w.y);
+}
+
+// The tiles of the integrals whose blocks staged their samples: work entry
+// (integral, tile).
+__global__ void __launch_bounds__(256) vegas_batch_tiles_kernel(BatchDev b, const int2* __restrict__ work) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int2 w = work[blockIdx.x];
+    const VItem& it = b.vi[w.x];
+    if (!vitem_active(it, b.st[w.x])) return;
+    const int cells = it.D * b.bins;
+    unsigned long long* hh = reinterpret_cast<unsigned long long*>(smem);
+    unsigned int* hc = reinterpret_cast<unsigned int*>(hh + cells);
+    for (int k = threadIdx.x; k < cells; k += blockDim.x) {
+        hh[k] = 0ull;
+        hc[k] = 0u;
+    }
+    __syncthreads();
+    const double* sw = b.part + it.stage;
+    const uint64_t* sb = reinterpret_cast<const uint64_t*>(sw + (int64_t)it.tiles * kTile);
+    const auto load = [&](int j, double& v, uint64_t& pk) {
+        const int64_t s = (int64_t)w.y * kTile + j * 256 + threadIdx.x;
+        if (s >= it.n) return false;
+        v = sw[s];
+        pk = sb[s];
+        return true;
+    };
+    double* ph = b.part + it.part + 2 * (int64_t)it.blocks + (int64_t)w.y * cells;
+    double* pc = ph + (int64_t)it.tiles * cells;
+    switch (it.D) {
+#define DIS_TILE(D)                                                          \
+    case D:                                                                  \
+        block_histogram<D>(b.bins, kBatchMaxSpt, load, hh, hc, ph, pc);      \
+        break;
+        DIS_TILE(2) DIS_TILE(3) DIS_TILE(4) DIS_TILE(5) DIS_TILE(6) DIS_TILE(7)
+#undef DIS_TILE
+    }
 }
 
 // Histogram partials, first level, for every active integral: block
 // (v, g, c) sums cells [64 c, 64 c + 64) of integral v over its g-th range of
-// blocks, in block order (vegas_hist_groups_kernel per integral).
+// tiles, in tile order (vegas_hist_groups_kernel per integral).
 __global__ void __launch_bounds__(64) vegas_batch_groups_kernel(BatchDev b, int cblocks) {
     const int v = blockIdx.x / (kHistGroups * cblocks);
     const int rem = blockIdx.x - v * kHistGroups * cblocks;
@@ -565,10 +635,10 @@ __global__ void __launch_bounds__(64) vegas_batch_groups_kernel(BatchDev b, int 
     const int k = c * 64 + threadIdx.x;
     if (g >= it.groups || k >= cells) return;
     const double* ph = b.part + it.part + 2 * (int64_t)it.blocks;
-    const double* pc = ph + (int64_t)it.blocks * cells;
-    double* gh = b.part + it.part + 2 * (int64_t)it.blocks + 2 * (int64_t)it.blocks * cells;
+    const double* pc = ph + (int64_t)it.tiles * cells;
+    double* gh = b.part + it.part + 2 * (int64_t)it.blocks + 2 * (int64_t)it.tiles * cells;
     double* gc = gh + (int64_t)it.groups * cells;
-    const int b0 = g * it.per_group, b1 = min(b0 + it.per_group, it.blocks);
+    const int b0 = g * it.per_group, b1 = min(b0 + it.per_group, it.tiles);
     double h = 0.0, cn = 0.0;
     for (int bb = b0; bb < b1; ++bb) {
         h += ph[(size_t)bb * cells + k];
@@ -602,7 +672,7 @@ __global__ void __launch_bounds__(256) vegas_batch_reduce_kernel(BatchDev b, int
     }
     const int k = (r - 1) * blockDim.x + threadIdx.x;
     if (k >= cells) return;
-    const double* gh = part + 2 * (int64_t)it.blocks + 2 * (int64_t)it.blocks * cells;
+    const double* gh = part + 2 * (int64_t)it.blocks + 2 * (int64_t)it.tiles * cells;
     const double* gc = gh + (int64_t)it.groups * cells;
     double h = 0.0, cn = 0.0;
     for (int gg = 0; gg < it.groups; ++gg) {
@@ -904,13 +974,14 @@ struct BatchPlan {
     std::vector<VItem> vi;
     std::vector<int2> work;  // grouped by launch
     std::vector<Launch> launches;
+    std::vector<int2> tiles;  // of the integrals that stage their samples
     std::vector<int2> rows;
     std::vector<int4> gl_work;  // grouped by launch
     std::vector<Launch> gl_launches;
     std::vector<int4> map;
     int max_cells = 0, max_iterations = 0;
     int64_t part_doubles = 0, grid_doubles = 0;
-    size_t o_args = 0, o_vi = 0, o_st = 0, o_tables = 0, o_work = 0, o_rows = 0, o_gl_work = 0, o_gl_out = 0,
+    size_t o_args = 0, o_vi = 0, o_st = 0, o_tables = 0, o_work = 0, o_tiles = 0, o_rows = 0, o_gl_work = 0, o_gl_out = 0,
            o_map = 0, o_part = 0, o_grid = 0, total = 0;
 };
 
@@ -928,6 +999,7 @@ int batch_plan(const nlo_dis_batch_desc* d, BatchPlan& P, bool build_args) {
     // work entries and Gauss-Legendre items per launch (kind, arithmetic)
     std::vector<std::vector<int2>> work(NLO_DIS_KINDS * 2);
     std::vector<std::vector<int4>> glw(NLO_DIS_KINDS * 2);
+    std::vector<bool> fused(NLO_DIS_KINDS * 2, false);  // blocks that form their histogram
     std::vector<std::pair<const double*, std::array<double, 2>>> ends;
     P.map.resize(d->n_items);
     int n_gl = 0;
@@ -995,11 +1067,19 @@ int batch_plan(const nlo_dis_batch_desc* d, BatchPlan& P, bool build_args) {
         const int64_t blocks = (g64 + 4 * v.spt - 1) / (4 * v.spt);
         NLO_REQUIRE(blocks <= (1 << 24), "nlo_dis_batch: item %d: too many samples", i);
         v.blocks = (int)blocks;
-        v.per_group = (v.blocks + kHistGroups - 1) / kHistGroups;
-        v.groups = (v.blocks + v.per_group - 1) / v.per_group;
+        v.tiles = (int)((g64 + kTile / 64 - 1) / (kTile / 64));
+        v.per_group = (v.tiles + kHistGroups - 1) / kHistGroups;
+        v.groups = (v.tiles + v.per_group - 1) / v.per_group;
         const int cells = D * bins;
         v.part = P.part_doubles;
-        P.part_doubles += vpart_doubles(v.blocks, v.groups, cells);
+        P.part_doubles += vpart_doubles(v.blocks, v.tiles, v.groups, cells);
+        v.stage = -1;
+        if (v.spt < kBatchMaxSpt) {
+            v.stage = P.part_doubles;
+            P.part_doubles += 2 * (int64_t)v.tiles * kTile;
+        } else {
+            fused[slot] = true;
+        }
         v.grid = P.grid_doubles;
         P.grid_doubles += vgrid_doubles(D, bins);
         v.rule = -1;
@@ -1009,6 +1089,7 @@ int batch_plan(const nlo_dis_batch_desc* d, BatchPlan& P, bool build_args) {
         }
         const int vi = (int)P.vi.size();
         for (int b = 0; b < v.blocks; ++b) work[slot].push_back(make_int2(vi, b));
+        for (int t = 0; v.stage >= 0 && t < v.tiles; ++t) P.tiles.push_back(make_int2(vi, t));
         for (int dd = 0; dd < D; ++dd) P.rows.push_back(make_int2(vi, dd));
         P.map[i] = make_int4(0, vi, 0, 0);
         P.max_cells = std::max(P.max_cells, cells);
@@ -1020,7 +1101,8 @@ int batch_plan(const nlo_dis_batch_desc* d, BatchPlan& P, bool build_args) {
         if (!work[slot].empty()) {
             const size_t lds = vegas_layout(kDims[K], bins, kBatchMaxSpt, true).total;
             NLO_REQUIRE(lds <= 64 * 1024, "nlo_dis_batch: LDS %zu bytes exceeds 64 KiB (fewer bins)", lds);
-            P.launches.push_back({K, prec, (int)P.work.size(), (int)work[slot].size(), lds});
+            P.launches.push_back({K, prec, (int)P.work.size(), (int)work[slot].size(),
+                                  fused[slot] ? lds : vegas_layout(kDims[K], bins, kBatchMaxSpt, false).total});
             P.work.insert(P.work.end(), work[slot].begin(), work[slot].end());
         }
         if (!glw[slot].empty()) {
@@ -1039,6 +1121,7 @@ int batch_plan(const nlo_dis_batch_desc* d, BatchPlan& P, bool build_args) {
     P.o_st = section(sizeof(VState) * P.vi.size());
     P.o_tables = section(sizeof(nlo_sobol_table) * (size_t)d->n_tables);
     P.o_work = section(sizeof(int2) * P.work.size());
+    P.o_tiles = section(sizeof(int2) * P.tiles.size());
     P.o_rows = section(sizeof(int2) * P.rows.size());
     P.o_gl_work = section(sizeof(int4) * P.gl_work.size());
     P.o_gl_out = section(sizeof(double) * 2 * (size_t)n_gl);
@@ -1061,8 +1144,8 @@ void launch_gl_batch(const BatchPlan::Launch& L, const DisArgs* args, const int4
 }
 
 // One iteration of every active VEGAS integral of the batch on stream s.
-int enqueue_batch_iteration(const BatchPlan& P, const BatchDev& bd, const int2* work, const int2* rows, double eps,
-                            double tiny, double epsrel, double epsabs, hipStream_t s) {
+int enqueue_batch_iteration(const BatchPlan& P, const BatchDev& bd, const int2* work, const int2* tiles,
+                            const int2* rows, double eps, double tiny, double epsrel, double epsabs, hipStream_t s) {
     for (const auto& L : P.launches) {
         const int contribution = L.K;
 #define DIS_VB(K)                                                             \
@@ -1072,6 +1155,11 @@ int enqueue_batch_iteration(const BatchPlan& P, const BatchDev& bd, const int2* 
         break;
         DIS_DISPATCH(DIS_VB)
 #undef DIS_VB
+        NLO_LAUNCH_CHECK();
+    }
+    if (!P.tiles.empty()) {
+        const size_t lds = (size_t)P.max_cells * (sizeof(unsigned long long) + sizeof(unsigned int));
+        hipLaunchKernelGGL(vegas_batch_tiles_kernel, dim3((unsigned)P.tiles.size()), dim3(256), lds, s, bd, tiles);
         NLO_LAUNCH_CHECK();
     }
     const int nv = (int)P.vi.size();
@@ -1343,6 +1431,7 @@ int nlo_dis_batch_run(const nlo_dis_batch_desc* desc, double* d_results, void* d
     put(P.o_vi, P.vi.data(), sizeof(VItem) * P.vi.size());
     put(P.o_tables, desc->tables, sizeof(nlo_sobol_table) * (size_t)desc->n_tables);
     put(P.o_work, P.work.data(), sizeof(int2) * P.work.size());
+    put(P.o_tiles, P.tiles.data(), sizeof(int2) * P.tiles.size());
     put(P.o_rows, P.rows.data(), sizeof(int2) * P.rows.size());
     put(P.o_gl_work, P.gl_work.data(), sizeof(int4) * P.gl_work.size());
     put(P.o_map, P.map.data(), sizeof(int4) * P.map.size());
@@ -1378,6 +1467,7 @@ int nlo_dis_batch_run(const nlo_dis_batch_desc* desc, double* d_results, void* d
     const double eps = desc->precision == NLO_PREC_FP32 ? (double)FLT_EPSILON : DBL_EPSILON;
     const double tiny = desc->precision == NLO_PREC_FP32 ? (double)FLT_MIN : DBL_MIN;
     const int2* work = reinterpret_cast<const int2*>(w + P.o_work);
+    const int2* tiles = reinterpret_cast<const int2*>(w + P.o_tiles);
     const int2* rows = reinterpret_cast<const int2*>(w + P.o_rows);
     hipStream_t cs = nullptr;
     hipGraph_t graph = nullptr;
@@ -1388,7 +1478,7 @@ int nlo_dis_batch_run(const nlo_dis_batch_desc* desc, double* d_results, void* d
         NLO_HIP_CHECK(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
         hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
         if (e == hipSuccess) {
-            status = enqueue_batch_iteration(P, bd, work, rows, eps, tiny, desc->epsrel, desc->epsabs, cs);
+            status = enqueue_batch_iteration(P, bd, work, tiles, rows, eps, tiny, desc->epsrel, desc->epsabs, cs);
             const hipError_t e2 = hipStreamEndCapture(cs, &graph);
             if (status == NLO_OK && e2 != hipSuccess) e = e2;
         }

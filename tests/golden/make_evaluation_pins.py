@@ -21,8 +21,8 @@ from nlo_bk_optimized_amd._lib import DIS_DIMENSIONS
 from nlo_bk_optimized_amd.bk import MV, BKConfig
 from nlo_bk_optimized_amd.bk.config import RunningCouplingNLO
 from nlo_bk_optimized_amd.bk.evolution import uniform_edges
-from nlo_bk_optimized_amd.dipole import GBW
-from nlo_bk_optimized_amd.dis import DISConfig, Polarization, Quark, QuarkType
+from nlo_bk_optimized_amd.dipole import GBW, BKDipole, DipoleTable
+from nlo_bk_optimized_amd.dis import DISConfig, DISOrder, Polarization, Quark, QuarkType, structure_functions_batch
 from nlo_bk_optimized_amd.dis.fixed_sobol import gbw_qg_fixed_sobol_batch
 
 NODES = 24
@@ -90,7 +90,28 @@ def dis_fp64() -> dict[str, np.ndarray]:
     return integrand_points(DIS_DIMENSIONS, "fp64")
 
 
-SECTIONS = {"bk_fp64_sums": bk_sums, "nested_fp32": nested_fp32, "dis_fp64": dis_fp64}
+def dis_batch() -> dict[str, np.ndarray]:
+    """Structure functions of a table whose saturation scale grows with rapidity:
+    eight refinements of every grid, so that the last bit of a histogram tells."""
+
+    r = 1e-6 * torch.pow(torch.tensor(1e8 ** (1 / 127), dtype=torch.float64), torch.arange(128, dtype=torch.float64))
+    y = torch.arange(31, dtype=torch.float64) * 0.4
+    qs2 = 0.3 * torch.exp(0.22 * y)[:, None]
+    e = r * r * qs2 / 4 * torch.log(1 / (0.241 * r) + 8 * 2.7182818)
+    N = torch.where(e < 1e-5, e, -torch.expm1(-e))
+    dipole = BKDipole(DipoleTable(r=r.cuda(), y=y.cuda(), N=N.cuda(), x0=0.01))
+    out = {}
+    for dtype, maxeval in ((torch.float64, 80_000), (torch.float64, 290_000), (torch.float32, 290_000)):
+        config = DISConfig(order=DISOrder.NLO, maxeval=maxeval, epsrel=1e-12,
+                           quarks=(Quark(QuarkType.LIGHT, 0.14), Quark(QuarkType.C, 1.27)))
+        points = [(torch.tensor(q2, dtype=dtype), torch.tensor(x, dtype=dtype)) for q2, x in ((3.0, 5e-3), (40.0, 2e-4))]
+        pairs = structure_functions_batch(points, dipole, config, seed=44)
+        out[f"{'f64' if dtype is torch.float64 else 'f32'}_{maxeval}"] = torch.stack(
+            [torch.stack([f.value, f.error]).double() for p in pairs for f in p]).cpu().numpy()
+    return out
+
+
+SECTIONS = {"bk_fp64_sums": bk_sums, "nested_fp32": nested_fp32, "dis_fp64": dis_fp64, "dis_batch": dis_batch}
 
 if __name__ == "__main__":
     for section, values in SECTIONS.items():
