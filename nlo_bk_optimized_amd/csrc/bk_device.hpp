@@ -740,19 +740,32 @@ __device__ __forceinline__ float fmax2(float a, float b) {
 // select, which costs every wave).
 __device__ __forceinline__ void keep_branch(float& v) { asm volatile("" : "+v"(v)); }
 
-// 4 sin^2 y for |y| <= pi.  With w = |y| (pi - |y|), |sin y| = cos((pi^2/4 -
+// 4 sin^2 y from w = |y| (pi - |y|), 0 <= w <= pi^2/4: |sin y| = cos((pi^2/4 -
 // w)^1/2) is entire in w, and 2 |sin y| / w is its degree-4 interpolant at
-// Chebyshev nodes of [0, pi^2/4] (relative error 1e-9; all terms positive), so
-// that no fold into [0, pi/2] is needed.  pi - |y| is exact near pi, with the
-// low part of pi added.  pi: 3.14159274f in a vector register.
-__device__ __forceinline__ float f4sin2(float y, float pi) {
-    const float w = fabsf(y) * ((pi - fabsf(y)) + -8.74227766e-8f);
+// Chebyshev nodes of that range (relative error 1e-9; all terms positive), so
+// that no fold into [0, pi/2] is needed.
+__device__ __forceinline__ float f4sin2_from(float w) {
     float p = fmaf(w, 5.161262147e-07f, 4.312110734e-05f);
     p = fmaf(w, p, 2.320589108e-03f);
     p = fmaf(w, p, 6.450305465e-02f);
     p = fmaf(w, p, 6.366197731e-01f);
     const float s = w * p;
     return s * s;
+}
+
+// |y| <= pi.  pi - |y| is exact near pi, with the low part of pi added.  pi:
+// 3.14159274f in a vector register.
+__device__ __forceinline__ float f4sin2(float y, float pi) {
+    return f4sin2_from(fabsf(y) * ((pi - fabsf(y)) + -8.74227766e-8f));
+}
+
+// |y| <= 2 pi: the difference of two half-angles leaves [-pi, pi] where one of
+// them lies in a bin across pi/2 and the grids of the two differ.  With u = pi -
+// |y|, sin^2 y = sin^2 u and w = |u| (pi - |u|); outside [-pi, pi] the polynomial
+// is off by 4e-8 at 1.03 pi, 6e-5 at 1.3 pi and 1e-3 at 1.5 pi.
+__device__ __forceinline__ float f4sin2_wide(float y, float pi) {
+    const float u = (pi - fabsf(y)) + -8.74227766e-8f;
+    return f4sin2_from(fabsf(u) * fminf(fabsf(y), 6.28318548f - fabsf(y)));
 }
 
 // log2(1 + u) / 2 for |u| < 0.5: atanh(s) log2(e) with s = u / (2 + u),
@@ -866,6 +879,7 @@ struct Fp32Consts {
     float mu;          // ln mu0 log2 e
     float right0;      // 5 (ln 4 C2 / Lambda^2) log2 e - 10 log2 r
     float b0;          // b0 0.2 ln 2
+    bool wide;         // half-angle bins reach beyond 0.53 pi (the same for a whole block)
 };
 
 // The FP32 K2 + Kf integrand: the cancellation-free formula of
@@ -873,7 +887,7 @@ struct Fp32Consts {
 // on the fast primitives above, logs of distances (base 2) from the log1p
 // forms, N from the local-coordinate spline.  t1 = log2(z / r), t2 = log2(z' /
 // r), y1 = theta / 2, y2 = theta' / 2 (modulo pi, in [-pi/2, pi/2] but for the
-// bin across pi/2).
+// bin across pi/2, which reaches up to pi).
 //
 // Issue-bound: the cost of a sample is its instructions, an FP32 add, mul or fma
 // on vector registers or literals counting 2 cycles, min / max / compare /
@@ -893,7 +907,7 @@ __device__ __forceinline__ NloStable<float> nlo_integrand_fp32(const Fp32Consts&
                                                                const NloCoupling<float>& cpl) {
     NloStable<float> out{0.0f, 0.0f, 0.0f};
     const float z = fexp2(t1), z2 = fexp2(t2);
-    const float s1 = f4sin2(y1, c.pi), s2 = f4sin2(y2, c.pi), s3 = f4sin2(y1 - y2, c.pi);  // 4 sin^2
+    const float s1 = f4sin2(y1, c.pi), s2 = f4sin2(y2, c.pi), s3 = c.wide ? f4sin2_wide(y1 - y2, c.pi) : f4sin2(y1 - y2, c.pi);  // 4 sin^2
     const float zz2 = z * z2;
     float z1m = z - 1.0f, z2m = z2 - 1.0f;
     if (__any(fminf(fabsf(t1), fabsf(t2)) < 0.25f)) {  // 2^t - 1 near t = 0 without cancellation

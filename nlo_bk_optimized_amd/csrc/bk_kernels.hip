@@ -1135,6 +1135,7 @@ struct RunView {
 template <int MODE, bool HIST, bool FULL, bool ANYC>
 __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int p, int blk) {
     using T = typename std::conditional<MODE == NLO_PREC_FP32, float, double>::type;
+    __shared__ int wide;
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ double red[4][FULL ? 4 : 1][2];  // [wave][sum][value, error]
     __shared__ double wmax[4];
@@ -1204,17 +1205,22 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
         // takes these units back.  The four dimensions of a bin are adjacent,
         // so that the LDS address is the bin number shifted.  Wave 0 alone
         // builds the table, so that only one wave of the block evaluates the
-        // two FP64 logarithms of the bounds.
+        // two FP64 logarithms of the bounds.  wide: see f4sin2_wide (tested per
+        // sample it would cost 3 % of the launch).
         float2* E2 = reinterpret_cast<float2*>(smem + lay.edges);
         if (threadIdx.x < kWave) {
             const double log_rp = v.t64[2 + p];
+            bool across = false;
             for (int i = threadIdx.x; i < 4 * a.bins; i += kWave) {
                 const int b = i >> 2, d = i & 3;
                 const double left = ep[d * (a.bins + 1) + b], right = ep[d * (a.bins + 1) + b + 1];
                 const double x = d < 2 ? ((lo_r - log_rp) + w_r * left) * kLog2e : kPi * (left < 0.5 ? left : left - 1.0);
                 const double w = d < 2 ? w_r * kLog2e : kPi;
                 E2[i] = make_float2((float)x, (float)(w * (right - left)) * 0x1p-32f);
+                across |= d >= 2 && left < 0.5 && right > 0.53;
             }
+            across = __any(across);
+            if (threadIdx.x == 0) wide = across;
         }
     } else {
         for (int i = threadIdx.x; i < ne; i += blockDim.x) E[i] = ep[i];
@@ -1262,6 +1268,7 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
     }
     Fp32Consts c32{};
     if constexpr (MODE == NLO_PREC_FP32) {
+        c32.wide = uniform(wide) != 0;
         c32.pi = vector_reg(3.14159274f);
         c32.log2_r = (float)(log_rp * kLog2e);
         c32.cut = (float)(1e10 * ((rp * rp) * (rp * rp)));

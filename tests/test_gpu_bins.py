@@ -63,3 +63,23 @@ def test_fp32_steps(bins):
     batch.state.copy_(torch.cat([N, N]))
     batch.step()
     close(batch.state - torch.cat([N, N]), change["fp64_stable"].repeat(2), 1e-4)
+
+
+# An angular bin across theta = pi is not folded: its half-angles reach beyond
+# pi/2 and the difference of two of them beyond pi, the further the wider the
+# bin and the more the grids of the two angles differ.
+@pytest.mark.parametrize("first,second", [([0, 0.3, 1], [0, 0.55, 1]), ([0, 0.45, 0.98, 1], [0, 0.3, 0.52, 1])])
+def test_fp32_angles_in_wide_bins(first, second):
+    r, N = workload()
+    t64, t32 = dev.spline_build(r, N)
+    bins = len(first) - 1
+    config = BKConfig(RPOINTS=NODES - 1, MAXR=100.0, MC_BINS=bins)
+    edges, table = uniform_edges(NODES, bins, r.device), dev.sobol_table(4, 3)
+    for d, e in ((2, first), (3, second)):
+        edges[:, d] = torch.tensor(e, dtype=torch.float64, device=r.device)
+
+    def run(precision):
+        return dev.bk_nlo(r, N, t64, t32, edges, table, 1 << 16, config, precision=precision)[0][:, 0]
+
+    # FP32's own error of these sums is 5e-7, the unfolded difference gave 1e-5 to 2e-5
+    close(run("fp32"), run("fp64_stable"), 2e-6)
