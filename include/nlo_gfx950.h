@@ -316,8 +316,10 @@ int nlo_bk_evolver_create(const nlo_bk_evolver_desc* desc, const double* d_r,
                           const double* d_edges, void* d_workspace, size_t workspace_bytes,
                           hipStream_t stream, nlo_bk_evolver** out);
 double* nlo_bk_evolver_state(nlo_bk_evolver* ev);
-/* Device int32 flag, non-zero once any step produced a non-finite N
- * (S/bk/evolution.py:152-153 raises FloatingPointError). */
+/* Device int32 flag, 0 while every step is sound.  Bit 0: a step produced a
+ * non-finite N (S/bk/evolution.py:152-153 raises FloatingPointError).  Bit 1: the
+ * adaptive K1 rule gave up waiting for an inner integral, and K1 of some parents
+ * is missing from the step. */
 int32_t* nlo_bk_evolver_nonfinite_flag(nlo_bk_evolver* ev);
 /* Device uint64: number of (parent, right-hand side) evaluations with an
  * active parent since creation; times n_samples it is the exact count of

@@ -60,6 +60,15 @@ class BKSetup:
     n_samples: int
 
 
+def check_flag(flag: int) -> None:
+    """Raise for a step that is not sound (the bits of nlo_bk_evolver_nonfinite_flag)."""
+
+    if flag & 2:
+        raise RuntimeError("the adaptive K1 rule gave up waiting for an inner integral")
+    if flag:
+        raise FloatingPointError("non-finite BK amplitude during the rapidity evolution")
+
+
 def uniform_edges(R: int, bins: int, device: torch.device) -> torch.Tensor:
     e = torch.linspace(0, 1, bins + 1, dtype=torch.float64, device=device)
     return e.expand(R, 4, bins + 1).contiguous()
@@ -205,8 +214,7 @@ def solve_bk(
             ys.append(y)
             if y >= maxy - tolerance:
                 break
-        if int(evolver.flag.item()) != 0:
-            raise FloatingPointError("non-finite BK amplitude during the rapidity evolution")
+        check_flag(int(evolver.flag.item()))
     finally:
         evolver.close()
     N_out = torch.cat([history[: min(t, steps) + 1]] + rows[1:], dim=0)
@@ -301,8 +309,7 @@ def solve_bk_batch(
         for t in range(steps):
             ev.step()
             history[t + 1].copy_(ev.state)
-        if int(ev.flag.item()) != 0:
-            raise FloatingPointError("non-finite BK amplitude during the rapidity evolution")
+        check_flag(int(ev.flag.item()))
         if stats is not None:
             stats["spt"], stats["grid_blocks"], stats["ms_per_nlo_launch"] = ev.tuning()
             stats["active_evaluations"] = int(ev.active_evaluations.item())

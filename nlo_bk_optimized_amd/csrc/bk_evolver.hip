@@ -183,7 +183,7 @@ __global__ void clamp_flag_kernel(int R, double* __restrict__ N, int force_posit
     if (i >= R) return;
     double v = N[i];
     if (force_positive) v = fmin(fmax(v, 0.0), 1.0);
-    if (!isfinite(v)) flag[0] = 1;
+    if (!isfinite(v)) (void)atomicOr(flag, 1);
     N[i] = v;
 }
 

@@ -42,8 +42,8 @@ int launch_k1_adaptive(int R, const double* r, const double* N, const double* t6
                        int rint, int tint, double epsrel, double* k1, double* k1_err,
                        long long* k1_evals, hipStream_t stream, const K1History* hist = nullptr);
 // The same with the inner integrals of all parents in one queue:
-// `workspace` of k1_queue_workspace(R) bytes, 256-byte aligned; *flag is set to
-// 1 if a wait of the queue runs out of its limit.
+// `workspace` of k1_queue_workspace(R) bytes, 256-byte aligned; bit 1 of *flag
+// (value 2) is set if a wait of the queue runs out of its limit.
 size_t k1_queue_workspace(int R);
 int launch_k1_queue(int R, const double* r, const double* N, const double* t64, const BkConsts& c, int rint,
                     int tint, double epsrel, double* k1, void* workspace, int32_t* flag, hipStream_t stream,

@@ -816,7 +816,7 @@ struct K1Queue {
     double* state;      // R x kK1QueueState: outer list (4 x 128), 42 ln z nodes, 42 values
     int* pending;       // R: inner integrals that have not ended
     int* count;         // R: outer intervals
-    int* flag;          // set when a wait ran out of its limit
+    int* flag;          // kK1QueueGaveUp is set when a wait ran out of its limit
 };
 constexpr int kK1QueueCtl = 32;
 constexpr int kK1QueueState = 4 * 128 + 84;
@@ -825,9 +825,15 @@ constexpr unsigned kK1QueueEnd = (1u << 18) - 1u;
 static_assert(64 * kMaxR < (int)kK1QueueEnd, "a task fits below the lap");
 // laps: at most kMaxGkIntervals rings of tasks and one of end marks
 static_assert(kMaxGkIntervals + 2 < 1 << 14, "a lap fits above the task");
-// Bound of one wait in ticks of the 100 MHz clock (20 s).  A wait ends when a
-// running task does (at most kMaxGkIntervals bisections), so it is never met.
-constexpr long long kK1QueueTicks = 2000000000ll;
+// Bound of one wait in polls.  A wave waits only while its ring has fewer tasks
+// than waves, so every pending task runs, and the wait ends with the ring's
+// remaining work at the latest: at most kMaxGkIntervals outer steps of an inner
+// integral of at most kMaxGkIntervals bisections, 10^4 bisections in sequence of
+// 5 to 50 us.  2^25 polls, each a trip to memory of half a microsecond or more,
+// are at least 16 s.  Polls and not a clock: time in which the whole launch is
+// suspended does not count.
+constexpr unsigned kK1QueuePolls = 1u << 25;
+constexpr int kK1QueueGaveUp = 2;  // the bit of the flag
 
 template <typename T>
 __device__ __forceinline__ T q_load(const T* p) {
@@ -850,17 +856,20 @@ __device__ __forceinline__ unsigned* k1_queue_entry(const K1Queue& q, int ring, 
 // Orders what a wave shares: every access before it has reached the memory
 // that all XCDs see (stores at device scope are written through and
 // acknowledged there) before any after it is issued; loads at device scope
-// pass by the caches, so no cache is written back or dropped.
+// pass by the caches, so no cache is written back or dropped.  This is gfx950's
+// ordering and not the language's, which would ask for release and acquire; it
+// covers atomics at device scope only, so whatever waves share goes through
+// q_load, q_store and q_add.
 __device__ __forceinline__ void q_settle() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
 
 // Writes an entry of the ring when the reader of the lap before has emptied it.
 __device__ __forceinline__ void k1_queue_put(const K1Queue& q, int ring, unsigned ticket, unsigned task) {
     unsigned lap;
     unsigned* e = k1_queue_entry(q, ring, ticket, lap);
-    const long long t0 = wall_clock64();
+    unsigned polls = 0u;
     while (q_load(e) != lap) {
-        if (wall_clock64() - t0 > kK1QueueTicks) {
-            q_store(q.flag, 1);
+        if (++polls > kK1QueuePolls) {
+            (void)atomicOr(q.flag, kK1QueueGaveUp);
             return;
         }
         __builtin_amdgcn_s_sleep(1);
@@ -936,15 +945,15 @@ __global__ void __launch_bounds__(kK1aWaves<ANY> * 64)
         ticket = (unsigned)uniform((int)ticket);
         unsigned lap, task;
         unsigned* entry = k1_queue_entry(q, ring, ticket, lap);
-        const long long t0 = wall_clock64();
+        unsigned polls = 0u;
         for (;;) {
             task = (unsigned)uniform((int)q_load(entry)) - lap;
             if (task - 1u < kK1QueueEnd) break;
-            if (wall_clock64() - t0 > kK1QueueTicks) {
-                q_store(q.flag, 1);
+            if (++polls > kK1QueuePolls) {
+                if (lane == 0) (void)atomicOr(q.flag, kK1QueueGaveUp);
                 return;
             }
-            __builtin_amdgcn_s_sleep(4);
+            __builtin_amdgcn_s_sleep(16);  // half a microsecond: oftener, the polls slow the tasks by a few per cent
         }
         q_settle();
         if (lane == 0) q_store(entry, lap + (1u << 18));
@@ -1584,7 +1593,7 @@ __global__ void rk_final_kernel(int R, double* __restrict__ N, const double* __r
     if (K3) acc += b3 * K3[i];
     double v = N[i] + h * acc;
     if (force_positive) v = fmin(fmax(v, 0.0), 1.0);
-    if (!isfinite(v)) flag[0] = 1;
+    if (!isfinite(v)) (void)atomicOr(flag, 1);
     N[i] = v;
 }
 

@@ -180,3 +180,19 @@ def test_load_reference_nlobk_table():
     assert bool(((t.N >= 0) & (t.N <= 1)).all())
     # evolution increases N at fixed r
     assert bool((t.N[-1] >= t.N[0]).all())
+
+
+def test_step_flag_tells_its_causes_apart():
+    """Bit 0 is a non-finite amplitude, bit 1 a wait of the adaptive K1 rule that
+    ran out of its limit, whose cause the other message would hide."""
+
+    import pytest
+
+    from nlo_bk_optimized_amd.bk.evolution import check_flag
+
+    check_flag(0)
+    with pytest.raises(FloatingPointError, match="non-finite"):
+        check_flag(1)
+    for flag in (2, 3):
+        with pytest.raises(RuntimeError, match="gave up waiting"):
+            check_flag(flag)
