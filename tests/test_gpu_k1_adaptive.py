@@ -171,15 +171,19 @@ def test_evolver_adaptive_k1_step(dev):
     (30, None, {"RINTPOINTS": 100, "THETAINTPOINTS": 1, "INTACCURACY": 1e-30}, None),  # most laps of the ring
     (150, None, {}, None),  # more first tasks than waves, a longer ring
     (24, None, {"INTACCURACY": 1e-2}, "parent_dls"),
+    # no decision at a tolerance, outer and inner lists both split
+    (200, None, {"RINTPOINTS": 6, "THETAINTPOINTS": 3, "INTACCURACY": 1e-30}, None),
+    (24, None, {"RINTPOINTS": 100, "THETAINTPOINTS": 12, "INTACCURACY": 1e-30}, None),
 ])
 def test_evolver_queue_matches_the_block_kernel(dev, R, active, limits, variant):
     """The evolver takes the inner integrals of all parents from one queue,
-    nlo_bk_k1_adaptive one block per parent: the same sums in the same order,
-    so K1 agrees to rounding (1e-10 as in _compare; 1e-12 of the largest K1
-    where a parent's cancels), and within the error estimate where a decision
-    at the tolerance went the other way.  Each of several steps (replays of one
-    graph) is compared; the queue's own results are the same bits every time,
-    whichever wave took what."""
+    nlo_bk_k1_adaptive one block per parent: the same samples, decisions and
+    sums in the same order, so K1 agrees to rounding for every parent (the two
+    kernels may fuse other multiply-adds: 1e-12, and 1e-14 of the largest K1
+    where a parent's cancels; a lost, doubled or stale node or interval shows at
+    1e-7 and above).  Each of several steps (replays of one graph) is compared;
+    the queue's own results are the same bits every time, whichever wave took
+    what."""
 
     from nlo_bk_optimized_amd.bk.config import BKConfig
     from nlo_bk_optimized_amd.bk.evolution import prepare
@@ -199,15 +203,11 @@ def test_evolver_queue_matches_the_block_kernel(dev, R, active, limits, variant)
         for _ in range(3):
             state = ev.state.clone()
             t64, _ = dev.spline_build(setup.r, state)
-            stats = {}
-            want = dev.bk_k1(setup.r, state, t64, cfg, rule="adaptive", stats=stats)
+            want = dev.bk_k1(setup.r, state, t64, cfg, rule="adaptive")
             ev.step()
             got = ev.k1.clone()
-            diff, floor = (got - want).abs(), 1e-12 * want.abs().max()
-            near = diff <= 1e-10 * want.abs() + floor
-            print(f"near for {int(near.sum())} of {near.numel()} parents", flush=True)
-            assert near.double().mean() >= 0.9
-            assert torch.all(near | (diff <= 2.0 * stats["error"] + floor))
+            assert int(ev.flag.item()) == 0
+            assert torch.all((got - want).abs() <= 1e-12 * want.abs() + 1e-14 * want.abs().max())
             after = ev.state.clone()
             ev.state.copy_(state)
             ev.step()
