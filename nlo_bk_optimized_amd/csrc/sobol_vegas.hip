@@ -306,9 +306,12 @@ int launch_vegas_adapt(int rows, int dim, int bins, const double* edges, const d
                        const double* count, double eps, double* out, hipStream_t stream) {
     const int items = rows * dim;
     const size_t lds = kAdaptScratch(bins) * sizeof(double);
-    if (lds > 65536)  // more than 2730 bins: beyond the default limit of dynamic LDS
+    // more than 2730 bins: beyond the default limit of dynamic LDS.  Always the
+    // largest size: the limit is the kernel's and not the launch's, and another
+    // thread may launch between this call's setting and its launch.
+    if (lds > 65536)
         NLO_HIP_CHECK(hipFuncSetAttribute((const void*)vegas_adapt_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          (int)lds));
+                                          (int)(kAdaptScratch(kMaxAdaptBins) * sizeof(double))));
     hipLaunchKernelGGL(vegas_adapt_kernel, dim3(items), dim3(64), lds, stream, bins, edges, hist, count, eps, out);
     NLO_LAUNCH_CHECK();
     return NLO_OK;
@@ -486,7 +489,7 @@ int nlo_vegas_histogram(int32_t dim, int32_t bins, int64_t n, const uint8_t* d_b
 int nlo_vegas_adapt(int32_t rows, int32_t dim, int32_t bins, const double* d_edges,
                     const double* d_hist, const double* d_count, double eps, double* d_edges_out,
                     hipStream_t stream) {
-    NLO_REQUIRE(rows >= 1 && dim >= 1 && bins >= 2 && bins <= 4096,
+    NLO_REQUIRE(rows >= 1 && dim >= 1 && bins >= 2 && bins <= nlo::kMaxAdaptBins,
                 "nlo_vegas_adapt: rows=%d dim=%d bins=%d invalid", rows, dim, bins);
     NLO_REQUIRE(d_edges && d_hist && d_count && d_edges_out, "nlo_vegas_adapt: null pointer");
     NLO_REQUIRE(d_edges != d_edges_out, "nlo_vegas_adapt: in-place refinement is not supported");

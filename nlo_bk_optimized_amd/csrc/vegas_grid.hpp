@@ -43,6 +43,7 @@ __device__ __forceinline__ double vegas_smoothed(const double* h, const double* 
 // for a batch's grids and 124 us for 64 x 4 BK grids, a tenth of the runs that
 // refine between short passes.)
 __host__ __device__ constexpr int kAdaptScratch(int bins) { return 3 * bins + 2; }
+constexpr int kMaxAdaptBins = 4096;
 
 __device__ inline void vegas_adapt_block(const double* e, const double* hh, const double* cc, int bins, double eps,
                                          double* o, double* scratch) {

@@ -67,3 +67,36 @@ def test_refined_edges_equal_a_forward_sweep(bins):
     with np.errstate(invalid="ignore"):
         want = np.stack([_sweep(e, h, c, eps) for e, h, c in zip(edges, hist, count)])
     assert np.array_equal(got, want, equal_nan=True)
+
+
+def test_threads_refine_grids_of_different_sizes():
+    """Grids above the default LDS limit set the kernel's limit; threads with
+    other sizes launch in between."""
+
+    import threading
+
+    from nlo_bk_optimized_amd import device as dev
+
+    errors = []
+
+    def refine(bins):
+        try:
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                hist = torch.rand((1, 1, bins), generator=torch.Generator().manual_seed(bins), dtype=torch.float64).cuda()
+                count = torch.ones_like(hist)
+                edges = torch.linspace(0, 1, bins + 1, dtype=torch.float64).reshape(1, 1, -1).cuda()
+                first = dev.vegas_adapt(edges, hist, count, 1e-16)
+                for _ in range(300):
+                    out = dev.vegas_adapt(edges, hist, count, 1e-16)
+                stream.synchronize()
+                assert torch.equal(out, first)
+        except Exception as e:  # noqa: BLE001
+            errors.append((bins, e))
+
+    threads = [threading.Thread(target=refine, args=(bins,)) for bins in (2800, 3400, 4096, 4000)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
