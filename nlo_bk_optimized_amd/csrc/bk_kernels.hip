@@ -1937,12 +1937,15 @@ int launch_k1_adaptive(int R, const double* r, const double* N, const double* t6
 // and for the reads that lead to them once, which long runs amortise; runs are
 // as long as still leaves about 2 500 blocks (256 CUs hold 2 048 of the FP32
 // evolver's), at least 4 and, for the tail of the launch, at most 16 groups;
-// 64 in FP32 beyond 2^18 points (up to there a single run keeps the batch
-// kernel's 16 and both sum alike bit for bit; FP64 samples take ten times as
-// long and gain nothing).  A launch with runs of 4, 8 or 16 by 8 192 blocks
-// against this rule: 100 000 points of 100 parents 91 -> 80 us, 2^14 of 255
-// 80 -> 44 us, 2^20 of 255 1 222 -> 1 160 us.  A histogram pass stages its
-// samples in the LDS, at most 8 per lane.
+// 64 in FP32 beyond 2^18 points (FP64 samples take ten times as long and gain
+// nothing).  A launch with runs of 4, 8 or 16 by 8 192 blocks against this rule:
+// 100 000 points of 100 parents 91 -> 80 us, 2^14 of 255 80 -> 44 us, 2^20 of
+// 255 1 222 -> 1 160 us.  The line at 2^18, runs of at most 16 against 64: 2^17
+// points of 255 parents 179 / 185 us, 2^17 of 511 341 / 351, 2^18 of 255 333 /
+// 350, 2^16 of 1 023 343 / 353, 2^18 of 1 023 1 294 / 1 245 (the one found the
+// other way).  A block's partial is rounded once, so results depend on the rule
+// in the last bits, and single and batched runs agree to rounding.  A histogram
+// pass stages its samples in the LDS, at most 8 per lane.
 NloPlan nlo_plan(int R, int bins, int64_t n, bool hist, bool fp32) {
     NloPlan pl{};
     const int64_t parents = R - 1, groups = (n + kWave - 1) / kWave;
