@@ -2,12 +2,12 @@
 // known to be ordinary numbers.  The library's forms cover every input (zeros,
 // subnormal and infinite values, NaN) and carry the logarithm in
 // double-double: 98 instructions for log, 175 for log1p(exp(-x)), 12 for a
-// quotient, which made most of what the FP64 integrands issue.  Here: 33, 24
-// (log1p_fold64 from a power) and 6.  The fixed K1 rule on 1024 nodes went
+// quotient, which made most of what the BK integrands in FP64 issue.  Here: 39,
+// 24 (log1p_fold64 from a power) and 6.  The fixed K1 rule on 1024 nodes went
 // from 2.63 to 1.91 ms, on the default grid of 101 from 85 to 54 us with them,
-// one RHS of the adaptive rule on 256 nodes from 1.96 to 1.59 ms.  Largest
-// errors over 2^20 arguments of 2^-40 .. 2^20: rcp64 and div64 0.50 ulp, log64
-// 0.74 (the library's log 0.63), exp64 0.97 (0.86).
+// one RHS of the adaptive rule on 256 nodes from 1.96 to 1.59 ms.  Errors over
+// 2^22 arguments, largest / mean, in ulp: log64 0.65 / 0.250 (the library's log
+// 0.64 / 0.252), exp64 0.75 / 0.254 (0.87 / 0.256), rcp64 and div64 0.50.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -61,6 +61,9 @@ __device__ __forceinline__ double sqrt64(double x) {
 // sqrt 2); with s = f / (2 + f), ln(1 + f) = 2 atanh s = f - f^2/2 +
 // s (f^2/2 + R(s^2)), where R(z) = 2 (z/3 + z^2/5 + ..) (degree 7,
 // interpolated at Chebyshev nodes of z <= 0.0296, error 1.1e-17); f is exact.
+// The reduction, the grouping of the terms and the two parts of ln 2 are those of
+// FDLIBM's log (Sun Microsystems, 1993); the polynomial is its own.  What the
+// two large terms e ln 2 + f and f^2/2 lose is added with the small ones.
 __device__ __forceinline__ double log64(double x) {
     double m = __builtin_amdgcn_frexp_mant(x);  // [1/2, 1)
     int e = __builtin_amdgcn_frexp_exp(x);
@@ -76,15 +79,18 @@ __device__ __forceinline__ double log64(double x) {
     R = fma(R, z, coef64(0.28571428627528794));
     R = fma(R, z, coef64(0.3999999999989607));
     R = fma(R, z, coef64(0.666666666666667));
-    const double h = 0.5 * f * f, de = (double)e;
+    const double hf = 0.5 * f, h = hf * f, de = (double)e;
     // ln 2 = 0x1.62e42fee00000p-1 (33 bits: e times it is exact) + the rest
     const double low_part = fma(s, fma(R, z, h), de * 1.90821492927058770002e-10);
-    return fma(de, 6.93147180369123816490e-01, f - (h - low_part));
+    const double b = fma(de, 6.93147180369123816490e-01, f);
+    const double b_rest = fma(de, 6.93147180369123816490e-01, -b) + f;
+    const double g = fma(-hf, f, b), g_rest = fma(-hf, f, b - g);
+    return g + (low_part + (b_rest + g_rest));
 }
 
 // e^x for finite x (0 and infinity where it leaves the range, NaN for NaN):
 // x = n ln 2 + r, |r| <= ln 2 / 2, e^r = 1 + r + r^2 P(r), P of degree 10
-// interpolated at Chebyshev nodes (error 3e-19).
+// interpolated at Chebyshev nodes (error 3e-19); the reduction as in FDLIBM's exp.
 __device__ __forceinline__ double exp64(double x) {
     const double n = rint(x * 1.44269504088896340736);
     const double r = fma(-n, 1.90821492927058770002e-10, fma(-n, 6.93147180369123816490e-01, x));
@@ -99,7 +105,8 @@ __device__ __forceinline__ double exp64(double x) {
     p = fma(p, r, coef64(0.04166666666666667));
     p = fma(p, r, coef64(0.1666666666666667));
     p = fma(p, r, coef64(0.5));
-    return ldexp(1.0 + fma(r * r, p, r), (int)n);
+    const double v = 1.0 + r;
+    return ldexp(v + fma(r * r, p, (1.0 - v) + r), (int)n);
 }
 
 // ln(1 + min(u, 1/u)) for u in [1e-18, 1e18]: 2 atanh w with w = u / (2 + u)
