@@ -71,6 +71,36 @@ def test_batch_item_equals_host_driven_vegas(dev, kind, precision, quark_mass, t
     assert int(got[2]) == want.n_eval and bool(got[3]) == want.converged
 
 
+# Blocks of 256, 512 and 1024 samples stage them for tiles of 2048, blocks of
+# 2048 are a tile: below, at and above a block, a tile and each change of the
+# block size (512 blocks: 2^18, 2^19, 2^20), and a ragged last tile; all in one
+# batch, so that one launch of a kind holds both sorts of blocks.
+def test_batch_histogram_tiles(dev):
+    from nlo_bk_optimized_amd import _lib
+    from nlo_bk_optimized_amd.dis.config import DISConfig, Quark, QuarkType
+    from nlo_bk_optimized_amd.numerics.integration import vegas_device
+
+    cfg = DISConfig(quarks=(Quark(QuarkType.C, 1.4),), maxr=5.0)
+    desc = dev.dis_desc(9.0, 1e-3, True, cfg.quarks, _gbw(), cfg)
+    sizes = [2, 63, 256, 257, 2047, 2048, 2049, 4096 + 77, (1 << 18) - 5, (1 << 18) + 256, (1 << 19) + 3, (1 << 20) - 2048,
+             (1 << 20) + 1]
+    items = []
+    for n in sizes:
+        item = _lib.DisItem()
+        item.desc, item.contribution, item.method = desc, _lib.DIS_KINDS["LO"], _lib.NLO_DIS_METHOD_VEGAS
+        item.n, item.sobol_table, item.max_iterations, item.min_iterations, item.first_index = n, 0, 4, 4, 64
+        items.append(item)
+    got = dev.dis_batch(items, [dev.sobol_table(2, 5)], bins=cfg.bins, precision="fp64", epsrel=1e-12, device="cuda").cpu()
+    for n, row in zip(sizes, got):
+        print(f"samples {n}", flush=True)
+        want = vegas_device(desc, "LO", samples_per_iteration=n, max_iterations=4, min_iterations=4, bins=cfg.bins,
+                            epsrel=1e-12, seed=5, precision="fp64", first_index=64)
+        # the same samples; refined edges agree to the fixed-point step of 2^-50
+        assert float(row[0]) == pytest.approx(float(want.value), rel=1e-12, abs=0)
+        assert float(row[1]) == pytest.approx(float(want.error), rel=1e-10, abs=0)
+        assert int(row[2]) == want.n_eval
+
+
 def test_gauss_legendre_item_equals_single_rule(dev):
     from nlo_bk_optimized_amd import _lib
     from nlo_bk_optimized_amd.dis.config import DISConfig, Quark, QuarkType
