@@ -484,6 +484,28 @@ __device__ __forceinline__ NloKernels64 nlo_kernels64(double a2, double b2, doub
     return k;
 }
 
+// The same two kernels with every quotient and function of the library, one
+// order at a time, for the passes that refine the grids.
+__device__ __forceinline__ double kernel_nlo64(double r, double X, double Y, double X2, double Y2, double Z,
+                                               double z4) {
+    const double a2 = (X * Y2) * (X * Y2), b2 = (X2 * Y) * (X2 * Y);
+    const double diff = a2 - b2;
+    const double rz = r * Z;
+    const double k = -2.0 / z4 + ((a2 + b2 - 4.0 * rz * rz) / (z4 * diff) + (r * r) * (r * r) / (a2 * diff) +
+                                  r * r / ((X * Y2 * Z) * (X * Y2 * Z))) *
+                                     2.0 * log(X * Y2 / (X2 * Y));
+    return isfinite(k) ? k : 0.0;
+}
+
+__device__ __forceinline__ double kernel_nlo_fermion64(double r, double X, double Y, double X2, double Y2, double Z,
+                                                       double z4, double nf, double nc) {
+    const double a2 = (X * Y2) * (X * Y2), b2 = (X2 * Y) * (X2 * Y);
+    const double rz = r * Z;
+    double k = 2.0 / z4 - (a2 + b2 - rz * rz) / (z4 * (a2 - b2)) * 2.0 * log(X * Y2 / (X2 * Y));
+    k = k * nf / nc;
+    return isfinite(k) ? k : 0.0;
+}
+
 // |e^(lz) - r e^(i t)|^2, s = sin(t / 2).
 __device__ __forceinline__ double nlo_distance_sq64(double r, double z, double s) {
     const double d = r - z;
@@ -500,42 +522,68 @@ __device__ __forceinline__ double nlo_distance_sq64(double r, double z, double s
 // points on 256 nodes 6.31 -> 4.40 ms; the sums keep the values of the plain
 // evaluation to 1.2e-11 in 210 steps.  (Squared distances throughout, with one
 // logarithm for both orders of the kernels, took 3.45 ms, but left them by 6e-8.)
-template <bool ANYC>
+//
+// PLAIN (the passes with a histogram): every step by the library.  An edge that
+// moves by an ulp draws other roundings from the cancelling samples of all
+// passes behind it, so the grids have to come out to the last bit: with the
+// shared logarithms in those passes too, 5 of 150 FP64 evolutions were off by
+// more than 1e-10, up to 5e-8.
+template <bool ANYC, bool PLAIN>
 __device__ NloValue64 nlo_integrand64(double r, double log_r, double lz, double lz2, double tz, double tz2,
-                                      const LdsSpline<double>& sS, const BkConsts& c) {
+                                      const LdsSpline<double>& sS, double r_min, double r_max, const BkConsts& c) {
     NloValue64 out{0.0, 0.0, 0.0};
     const double z = exp(lz), z2 = exp(lz2);
     const double xsq = nlo_distance_sq64(r, z, sin(tz / 2.0));
     const double x2sq = nlo_distance_sq64(r, z2, sin(tz2 / 2.0));
     const double zsq = nlo_distance_sq64(z, z2, sin((tz - tz2) / 2.0));
     if (xsq < 1e-40 || z < 1e-20 || x2sq < 1e-40 || z2 < 1e-20 || zsq < 1e-40) return out;
-    const double X = sqrt64(xsq), X2 = sqrt64(x2sq);
-    const double lx = 0.5 * log64(xsq), lx2 = 0.5 * log64(x2sq), lZ = 0.5 * log64(zsq);
-    const double S_X = loglog_from_log(sS, lx, 1.0, 0.0);
-    const double S_Y = loglog_from_log(sS, lz, 1.0, 0.0);
-    const double S_X2 = loglog_from_log(sS, lx2, 1.0, 0.0);
-    const double S_Y2 = loglog_from_log(sS, lz2, 1.0, 0.0);
-    const double S_Z = loglog_from_log(sS, lZ, 1.0, 0.0);
-    const double rsq = r * r;
-    const double dminsq = fmin(fmin(fmin(rsq, xsq), z * z), fmin(fmin(x2sq, z2 * z2), zsq));
+    double S_X, S_Y, S_X2, S_Y2, S_Z, as, k, ks, kf, kfs, jac;
     // _nlo_alpha_s (S/bk/derivatives.py:615-632)
-    double as;
-    if constexpr (ANYC) {
-        as = (c.fixed || c.rc_nlo == NLO_RC_NLO_FIXED) ? c.fixed_as
-             : c.rc_nlo == NLO_RC_NLO_PARENT           ? alpha_any64(r, c)
-                                                       : alpha_any64(sqrt(dminsq), c);
+    const bool any_fixed = c.fixed || c.rc_nlo == NLO_RC_NLO_FIXED;
+    if constexpr (PLAIN) {
+        const double X = sqrt(xsq), X2 = sqrt(x2sq), Z = sqrt(zsq), z4 = Z * Z * Z * Z;
+        S_X = loglog64(sS, r_min, r_max, X, 1.0, 0.0);
+        S_Y = loglog64(sS, r_min, r_max, z, 1.0, 0.0);
+        S_X2 = loglog64(sS, r_min, r_max, X2, 1.0, 0.0);
+        S_Y2 = loglog64(sS, r_min, r_max, z2, 1.0, 0.0);
+        S_Z = loglog64(sS, r_min, r_max, Z, 1.0, 0.0);
+        const double dmin = fmin(fmin(fmin(r, X), z), fmin(fmin(X2, z2), Z));
+        if constexpr (ANYC)
+            as = any_fixed ? c.fixed_as : alpha_any64(c.rc_nlo == NLO_RC_NLO_PARENT ? r : dmin, c);
+        else
+            as = alpha_s64(dmin, c);
+        k = kernel_nlo64(r, X, z, X2, z2, Z, z4);
+        ks = kernel_nlo64(r, X2, z2, X, z, Z, z4);
+        kf = kernel_nlo_fermion64(r, X, z, X2, z2, Z, z4, c.nf, c.nc);
+        kfs = kernel_nlo_fermion64(r, X2, z2, X, z, Z, z4, c.nf, c.nc);
+        jac = exp(2.0 * lz + 2.0 * lz2);
     } else {
-        const double lmin = fmin(fmin(fmin(log_r, lx), lz), fmin(fmin(lx2, lz2), lZ));
-        as = rcp64(alpha_s64_den(dminsq, lmin, c));
+        const double X = sqrt64(xsq), X2 = sqrt64(x2sq);
+        const double lx = 0.5 * log64(xsq), lx2 = 0.5 * log64(x2sq), lZ = 0.5 * log64(zsq);
+        S_X = loglog_from_log(sS, lx, 1.0, 0.0);
+        S_Y = loglog_from_log(sS, lz, 1.0, 0.0);
+        S_X2 = loglog_from_log(sS, lx2, 1.0, 0.0);
+        S_Y2 = loglog_from_log(sS, lz2, 1.0, 0.0);
+        S_Z = loglog_from_log(sS, lZ, 1.0, 0.0);
+        const double rsq = r * r;
+        const double dminsq = fmin(fmin(fmin(rsq, xsq), z * z), fmin(fmin(x2sq, z2 * z2), zsq));
+        if constexpr (ANYC) {
+            as = any_fixed ? c.fixed_as : alpha_any64(c.rc_nlo == NLO_RC_NLO_PARENT ? r : sqrt(dminsq), c);
+        } else {
+            const double lmin = fmin(fmin(fmin(log_r, lx), lz), fmin(fmin(lx2, lz2), lZ));
+            as = rcp64(alpha_s64_den(dminsq, lmin, c));
+        }
+        const double iz = rcp64(zsq);
+        // p ~ q: the rounding of p, q, their squares and quotients is amplified by
+        // 1 / d, so that another order of these steps would move a sum by up to 6e-8
+        const double p = X * z2, q = X2 * z, a2 = p * p, b2 = q * q, d = fma(-q, q, a2);
+        const double nf_over_nc = c.nf / c.nc;
+        const NloKernels64 ka = nlo_kernels64(a2, b2, d, div64(p, q), rsq, zsq, iz, nf_over_nc);
+        const NloKernels64 kb = nlo_kernels64(b2, a2, -d, div64(q, p), rsq, zsq, iz, nf_over_nc);
+        k = ka.k2, ks = kb.k2, kf = ka.kf, kfs = kb.kf;
+        const double zz = z * z2;
+        jac = zz * zz;
     }
-    const double iz = rcp64(zsq);
-    // p ~ q: the rounding of p, q, their squares and quotients is amplified by
-    // 1 / d, so that another order of these steps would move a sum by up to 6e-8
-    const double p = X * z2, q = X2 * z, a2 = p * p, b2 = q * q, d = fma(-q, q, a2);
-    const double nf_over_nc = c.nf / c.nc;
-    const NloKernels64 ka = nlo_kernels64(a2, b2, d, div64(p, q), rsq, zsq, iz, nf_over_nc);
-    const NloKernels64 kb = nlo_kernels64(b2, a2, -d, div64(q, p), rsq, zsq, iz, nf_over_nc);
-    double k = ka.k2, ks = kb.k2;
     double dip = -(S_X * S_Z * S_Y2 - S_X * S_Y);
     double dips = -(S_X2 * S_Z * S_Y - S_X2 * S_Y2);
     if (fabs(k) > 1e10 && fabs(dip) < 1e-10) { k = 0.0; dip = 0.0; }
@@ -545,10 +593,9 @@ __device__ NloValue64 nlo_integrand64(double r, double log_r, double lz, double 
     if (c.nf > 0.0) {
         const double df = S_Y * (S_X2 - S_X);
         const double dfs = S_Y2 * (S_X - S_X2);
-        kfr = -(c.symmetrize ? (ka.kf * df + kb.kf * dfs) / 2.0 : ka.kf * df);
+        kfr = -(c.symmetrize ? (kf * df + kfs * dfs) / 2.0 : kf * df);
     }
-    const double zz = z * z2;
-    const double scale = (as * c.nc) * (as * c.nc) * c.norm * (zz * zz);
+    const double scale = (as * c.nc) * (as * c.nc) * c.norm * jac;
     k2r *= scale;
     kfr *= scale;
     out.k2 = isfinite(k2r) ? k2r : 0.0;

@@ -1301,8 +1301,10 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
     const bool ordered = wv < a.ordered_waves;
     const int waves = ordered ? a.ordered_waves : 4 * a.bpp - a.ordered_waves;
     const int total = ordered ? a.ordered : a.groups - a.ordered, w0 = ordered ? wv : wv - a.ordered_waves;
-    const int share = total / waves, extra = total - share * waves;
-    const int mine = share + (w0 < extra ? 1 : 0);
+    // (a histogram pass: spt groups each, the blocks' tiles; another partition
+    // would round the histogram and the refined edges otherwise)
+    const int share = HIST ? a.spt : total / waves, extra = HIST ? 0 : total - share * waves;
+    const int mine = HIST ? min(max(total - w0 * share, 0), share) : share + (w0 < extra ? 1 : 0);
     const int64_t hi0 = (a.first >> 6) + (ordered ? 0 : a.ordered) + (int64_t)w0 * share + min(w0, extra);
     // The state of group hi: a per-lane part (direction bits 0..5 of the lane's
     // gray code) and a wave-uniform part (bits 6..29 of gray(hi), and bit 5 for
@@ -1344,7 +1346,9 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
         const bool valid = lane < min(rest, kWave);
         const bool odd = (hi & 1) != 0;
         T x[4];
-        T jac = vol;
+        // FP32: the volume first, which keeps the product in range; FP64: last, as
+        // the sum is written (the grids' last bits come from it)
+        T jac = MODE == NLO_PREC_FP32 ? vol : T(1);
         uint32_t packed = 0u;
         for (int d = 0; d < 4; ++d) {
             // bin = min(floor(u B), B - 1), frac = u B - bin with u = q 2^-30:
@@ -1376,10 +1380,12 @@ __device__ __forceinline__ void nlo_body(const NloArgs& a, const RunView& v, int
             }
             if (HIST) packed |= b << (8 * d);
         }
+        if constexpr (MODE != NLO_PREC_FP32) jac = vol * jac;
         double wv = 0.0, k2 = 0.0, kf = 0.0;
         if (valid) {
             if constexpr (MODE == NLO_PREC_FP64) {
-                const NloValue64 f = nlo_integrand64<ANYC>(rp, log_rp, x[0], x[1], x[2], x[3], spl, a.c);
+                const NloValue64 f = nlo_integrand64<ANYC, HIST>(rp, log_rp, x[0], x[1], x[2], x[3], spl,
+                                                                         v.t64[0], v.t64[1], a.c);
                 wv = f.total * (double)jac;
                 k2 = f.k2 * (double)jac;
                 kf = f.kf * (double)jac;

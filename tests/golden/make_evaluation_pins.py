@@ -5,7 +5,7 @@
 The FP64 integrands have samples whose terms cancel by many digits, where
 another order of the same operations gives other digits.  The recorded numbers
 are those of the formulas written out with the math library's functions and
-IEEE operations (the library as built from commit de78377); later kernels keep
+IEEE operations (the library as built from commit ccae63a); later kernels keep
 them.  Each section is one .npz next to this file.
 """
 
@@ -52,6 +52,20 @@ def bk_sums() -> dict[str, np.ndarray]:
     ev.state.copy_(state)
     ev.step()
     out["batch_109"] = (ev.state - state).cpu().numpy()
+    return out
+
+
+def bk_grids() -> dict[str, np.ndarray]:
+    """Importance grids after five FP64 refinements, for the production coupling
+    and the coupling at the parent."""
+
+    from nlo_bk_optimized_amd.bk.evolution import prepare
+
+    out = {}
+    for name, kw in (("production", {"PRECISION": "fp64"}),
+                     ("parent", {"PRECISION": "fp64", "RC_NLO": RunningCouplingNLO.PARENT_NLO})):
+        config = BKConfig(RPOINTS=NODES - 1, MAXR=100.0, MCINTPOINTS=20_000, K1_RULE="fixed", **kw)
+        out[name] = prepare(MV(qs0sqr=0.2), config, device=torch.device("cuda"), seed=3).edges[1::4].cpu().numpy()
     return out
 
 
@@ -111,7 +125,8 @@ def dis_batch() -> dict[str, np.ndarray]:
     return out
 
 
-SECTIONS = {"bk_fp64_sums": bk_sums, "nested_fp32": nested_fp32, "dis_fp64": dis_fp64, "dis_batch": dis_batch}
+SECTIONS = {"bk_fp64_sums": bk_sums, "bk_fp64_grids": bk_grids, "nested_fp32": nested_fp32, "dis_fp64": dis_fp64,
+            "dis_batch": dis_batch}
 
 if __name__ == "__main__":
     for section, values in SECTIONS.items():
